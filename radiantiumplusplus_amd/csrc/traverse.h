@@ -541,10 +541,20 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
   if (lane == 0) *pool.ctr = 0u;
   wave_lds_fence();
   TraceRay r;
-  bool active = false, exhausted = false;
+  bool active = false, done = false, exhausted = false;  // done: a finished ray not yet written out
   uint32_t idx = 0, tag = 0, visits = 0;
   uint32_t cbase = 0, cleft = 0;  // the wave's chunk (wave-uniform)
   for (;;) {
+    // Finished closest-hit rays are written out here, together: a wave's 64
+    // rays end a few at a time, and recomputing and storing the hit in the
+    // step in which its ray ended ran that code with about four lanes active
+    // in nearly every step (1080p large-mesh frame 145.6 -> 138.0 ms).  An
+    // any-hit ray has one byte or nothing to write and does so when it ends.
+    if (!ANY && done) {
+      trace_finish(s, r);
+      job.finish(Job::kTagIsIndex ? tag : idx, tag, r);
+      done = false;
+    }
     if (!exhausted || cleft > 0) {
       unsigned long long need = __ballot(!active);
       if (need) {
@@ -595,14 +605,16 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
       }
     }
     if (__ballot(active) == 0ull) {
-      if (exhausted && cleft == 0) break;
+      if (exhausted && cleft == 0) break;  // every finished ray was written out above
       continue;
     }
     for (int k = 0; k < 256; k++) {
       if (active) {
         if (trace_step<ANY, true>(s, r, st, pool)) {
-          if (!ANY) trace_finish(s, r);
-          job.finish(Job::kTagIsIndex ? tag : idx, tag, r);
+          if (ANY)
+            job.finish(Job::kTagIsIndex ? tag : idx, tag, r);
+          else
+            done = true;
           active = false;
         } else if constexpr (Job::kSuspend) {
           if (++visits >= job.budget) {
