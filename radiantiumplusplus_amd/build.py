@@ -41,6 +41,7 @@ SOURCES = [
     "scene_host.cpp",
     "render_job.cpp",
     "capi.cpp",
+    "trace_kernels.hip",
     "path_kernels.hip",
     "volpath_kernels.hip",
     "texture_kernels.hip",

@@ -23,8 +23,10 @@ struct DeviceBvhStats {
 void BuildBvh4Device(const float* bounds, const float4* records, uint32_t n, int maxLeaf, hipStream_t st,
                      DeviceBuffer& nodesOut, DeviceBuffer& primsOut, DeviceBvhStats& stats);
 
-// The traversal's 64-byte copy of m nodes (device buffers); throws if a
-// child box cannot be bounded.
-void QuantizeBvh4(const DeviceBuffer& nodes, uint32_t m, hipStream_t st, DeviceBuffer& out);
+// The traversal's nodes from a tree of m BvhNode4 over n primitive records
+// (device buffers): writes them to `out` and returns their number, puts the
+// primitive records in the order of their leaves and renumbers the BvhNode4
+// leaves to match; throws if a child box cannot be bounded.
+uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, DeviceBuffer& prims, uint32_t n, hipStream_t st, DeviceBuffer& out);
 
 }  // namespace rad

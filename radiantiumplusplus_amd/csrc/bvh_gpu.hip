@@ -11,9 +11,11 @@
 //    kSmall primitives are built to the leaves by one wave each, with an
 //    exact SAH sweep over the centroid order of every axis.  Ranges of at
 //    most max_leaf primitives become leaves.
-// 3. The binary tree is collapsed into the 4-wide, one-cache-line nodes the
-//    traversal reads (repeatedly opening the inner child of largest area),
-//    again level by level.
+// 3. The binary tree is collapsed into 4-wide nodes (repeatedly opening the
+//    inner child of largest area), again level by level.
+// 4. The traversal's 8-wide quantised nodes are made from the 4-wide tree of
+//    either builder, level by level, with the primitives put in the order of
+//    its leaves.
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -701,97 +703,311 @@ __global__ void k_sah(const BvhNode4* nodes, uint32_t m, float rootA, double* co
   if (__lane_id() == 0 && c != 0.f) atomicAdd(cost, double(c));
 }
 
-// ---------------------------------------------------------------- quantised copy
-// Step 2^e per axis, e the smallest with 255 * 2^e >= the node's extent
-// (raised further if rounding keeps a bound out of reach); bounds rounded
-// outward and verified with the traversal's own dequantisation.
-__device__ bool quantize_axis(const float* clo, const float* chi, const bool* valid, float o, float ext, uint32_t& biased,
-                              uint32_t& qlo, uint32_t& qhi) {
+// ---------------------------------------------------------------- traversal nodes
+// A node of the 8-wide tree: a BvhNode4 (count 0) whose inner children are
+// opened while they fit, or a leaf that does not fit beside its siblings
+// (count > 0, primitives [begin, begin + count) of the new order, the box of
+// child `src` of BvhNode4 n4).
+struct WideJob {
+  uint32_t n4, src, begin, count;
+};
+
+struct WideSlot {  // child `s` of BvhNode4 `n`
+  uint32_t n, s;
+};
+
+__device__ __forceinline__ void slot_box(const BvhNode4* nodes, WideSlot w, float lo[3], float hi[3]) {
+  const BvhNode4& nd = nodes[w.n];
+  lo[0] = nd.lox[w.s], lo[1] = nd.loy[w.s], lo[2] = nd.loz[w.s];
+  hi[0] = nd.hix[w.s], hi[1] = nd.hiy[w.s], hi[2] = nd.hiz[w.s];
+}
+
+// The children of the 8-wide node made from BvhNode4 `root`: its own four,
+// then the inner one of largest area replaced by its children while at most
+// eight result and their leaves hold at most kWideNodePrims primitives.
+__device__ int wide_children(const BvhNode4* nodes, uint32_t root, WideSlot out[8]) {
+  int n = 0;
+  uint32_t prims = 0;
+  for (uint32_t s = 0; s < 4; s++)
+    if (nodes[root].child[s] >= 0) {
+      prims += nodes[root].count[s];
+      out[n++] = WideSlot{root, s};
+    }
+  for (;;) {
+    int best = -1;
+    float area = -1.f;
+    uint32_t bestPrims = 0;
+    for (int i = 0; i < n; i++) {
+      const BvhNode4& nd = nodes[out[i].n];
+      if (nd.count[out[i].s] > 0) continue;
+      const BvhNode4& c = nodes[nd.child[out[i].s]];
+      int k = 0;
+      uint32_t p = 0;
+      for (int s = 0; s < 4; s++)
+        if (c.child[s] >= 0) {
+          k++;
+          p += c.count[s];
+        }
+      if (n - 1 + k > 8 || prims + p > kWideNodePrims) continue;
+      float lo[3], hi[3];
+      slot_box(nodes, out[i], lo, hi);
+      const float a = half_area(lo, hi);
+      if (a > area) {
+        area = a;
+        best = i;
+        bestPrims = p;
+      }
+    }
+    if (best < 0) return n;
+    const uint32_t c = uint32_t(nodes[out[best].n].child[out[best].s]);
+    prims += bestPrims;
+    bool first = true;
+    for (uint32_t s = 0; s < 4; s++)
+      if (nodes[c].child[s] >= 0) {
+        out[first ? best : n++] = WideSlot{c, s};
+        first = false;
+      }
+  }
+}
+
+// slot[i]: the slot of child i, chosen greedily so that bit a of a slot says
+// on which side of the node's centre the child's centre lies along axis a.
+__device__ void wide_order(const BvhNode4* nodes, const WideSlot* w, int n, const float lo[3], const float hi[3], int slot[8]) {
+  float d[8][3];
+  for (int i = 0; i < n; i++) {
+    float l[3], h[3];
+    slot_box(nodes, w[i], l, h);
+    for (int a = 0; a < 3; a++) d[i][a] = (l[a] + h[a]) - (lo[a] + hi[a]);
+    slot[i] = -1;
+  }
+  uint32_t used = 0;
+  for (int k = 0; k < n; k++) {
+    float best = -kInf;
+    int bi = -1, bs = 0;
+    for (int i = 0; i < n; i++) {
+      if (slot[i] >= 0) continue;
+      for (int s = 0; s < 8; s++) {
+        if (used >> s & 1u) continue;
+        const float c = (s & 1 ? d[i][0] : -d[i][0]) + (s & 2 ? d[i][1] : -d[i][1]) + (s & 4 ? d[i][2] : -d[i][2]);
+        if (bi < 0 || c > best) best = c, bi = i, bs = s;
+      }
+    }
+    slot[bi] = bs;
+    used |= 1u << bs;
+  }
+}
+
+// Step 2^e per axis, e the smallest with kWidePlaneMax * 2^e >= the node's
+// extent (raised further if rounding keeps a bound out of reach); bounds
+// rounded outward and verified with the traversal's own dequantisation.
+__device__ bool quantize_axis(const float* clo, const float* chi, uint32_t valid, float o, float ext, uint32_t& biased,
+                              uint16_t* qlo, uint16_t* qhi) {
+  constexpr float top = float(kWidePlaneMax);
   int e = -126;
   if (ext > 0.f) {
-    frexpf(ext / 255.f, &e);  // ext / 255 = m 2^e, m in [0.5, 1)
+    frexpf(ext / top, &e);  // ext / top = m 2^e, m in [0.5, 1)
     e = max(e, -126);
   }
   for (; e <= 127; e++) {
     const uint32_t b = uint32_t(e + 127);
     const float step = quant_step(b);
     bool ok = true;
-    uint32_t lo = 0, hi = 0;
-    for (int i = 0; i < 4 && ok; i++) {
-      if (!valid[i]) continue;
-      float fl = fminf(fmaxf(floorf((clo[i] - o) / step), 0.f), 255.f);
-      float fh = fminf(fmaxf(ceilf((chi[i] - o) / step), 0.f), 255.f);
-      uint32_t a = uint32_t(fl), c = uint32_t(fh);
+    for (int i = 0; i < 8 && ok; i++) {
+      qlo[i] = plane_bits(kWidePlaneMax);  // an empty slot: an inverted box
+      qhi[i] = 0;
+      if (!(valid >> i & 1u)) continue;
+      uint32_t a = uint32_t(fminf(fmaxf(floorf((clo[i] - o) / step), 0.f), top));
+      uint32_t c = uint32_t(fminf(fmaxf(ceilf((chi[i] - o) / step), 0.f), top));
       while (a > 0 && dequant(a, step, o) > clo[i]) a--;
-      while (c < 255 && dequant(c, step, o) < chi[i]) c++;
-      if (dequant(a, step, o) > clo[i] || dequant(c, step, o) < chi[i]) ok = false;
-      lo |= a << (8 * i);
-      hi |= c << (8 * i);
+      while (c < kWidePlaneMax && dequant(c, step, o) < chi[i]) c++;
+      if (!(dequant(a, step, o) <= clo[i] && dequant(c, step, o) >= chi[i])) ok = false;
+      qlo[i] = plane_bits(a);
+      qhi[i] = plane_bits(c);
     }
     if (ok) {
       biased = b;
-      qlo = lo;
-      qhi = hi;
       return true;
     }
   }
   return false;
 }
 
-__global__ void k_quantize(const BvhNode4* in, uint32_t m, BvhNodeQ* out, uint32_t* error) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const BvhNode4 nd = in[i];
-  bool valid[4];
-  float o[3] = {kInf, kInf, kInf}, h[3] = {-kInf, -kInf, -kInf};
-  for (int c = 0; c < 4; c++) {
-    valid[c] = nd.child[c] >= 0;
-    if (!valid[c]) continue;
-    o[0] = fminf(o[0], nd.lox[c]), o[1] = fminf(o[1], nd.loy[c]), o[2] = fminf(o[2], nd.loz[c]);
-    h[0] = fmaxf(h[0], nd.hix[c]), h[1] = fmaxf(h[1], nd.hiy[c]), h[2] = fmaxf(h[2], nd.hiz[c]);
-  }
-  BvhNodeQ q;
-  uint32_t counts = 0;
-  for (int c = 0; c < 4; c++) {
-    q.child[c] = nd.child[c];
-    counts |= (valid[c] ? min(nd.count[c], 255u) : 0u) << (8 * c);
-  }
-  q.counts = counts;
-  q.pad = 0;
-  if (!(valid[0] || valid[1] || valid[2] || valid[3])) {
-    q.ox = q.oy = q.oz = 0.f;
-    q.exps = 127u | 127u << 8 | 127u << 16;
-    q.qlox = q.qhix = q.qloy = q.qhiy = q.qloz = q.qhiz = 0;
-    out[i] = q;
+// One thread per node of a level.  EMIT = false: sums[j] = its inner children
+// (low word) and the primitives it places (high word).  EMIT = true, after an
+// exclusive scan of the sums: writes the node, its inner children's jobs, the
+// new place of its primitives, and that place into the BvhNode4 leaves.
+struct WideLevel {
+  uint32_t nodes, next, prims;  // first node of this level, of the next level, first primitive this level places
+};
+template <bool EMIT>
+__global__ void k_wide(const WideJob* jobs, uint32_t nJobs, BvhNode4* nodes, unsigned long long* sums, WideLevel lv,
+                       BvhNode8* out, WideJob* next, uint32_t* perm, uint32_t* error) {
+  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= nJobs) {
+    if (!EMIT && j == nJobs) sums[j] = 0ull;  // the scan's last entry is the level's total
     return;
   }
+  const WideJob jb = jobs[j];
+  WideSlot w[8];
+  uint32_t cnt[8];   // leaf: primitives; 0: inner
+  uint32_t wrap = 0;  // children that are leaves with a node of their own
+  int n;
+  if (jb.count > 0) {  // a leaf on its own: one slot, or the next nodes hold kWideNodePrims each
+    n = int((jb.count + kWideNodePrims - 1) / kWideNodePrims);
+    for (int i = 0; i < n; i++) {
+      w[i] = WideSlot{jb.n4, jb.src};
+      cnt[i] = min(kWideNodePrims, jb.count - uint32_t(i) * kWideNodePrims);
+    }
+    if (n > 1) wrap = (1u << n) - 1u;
+  } else {
+    n = wide_children(nodes, jb.n4, w);
+    uint32_t acc = 0;
+    for (int i = 0; i < n; i++) {
+      cnt[i] = nodes[w[i].n].count[w[i].s];
+      if (acc + cnt[i] > kWideNodePrims)
+        wrap |= 1u << i;
+      else
+        acc += cnt[i];
+    }
+  }
+  uint32_t inner = 0, prims = 0;
+  for (int i = 0; i < n; i++) {
+    inner += cnt[i] == 0 || (wrap >> i & 1u) ? 1u : 0u;
+    prims += cnt[i];
+  }
+  if (jb.count > 0) prims = 0;  // placed by its parent
+  if (!EMIT) {
+    sums[j] = (static_cast<unsigned long long>(prims) << 32) | inner;
+    return;
+  }
+  const uint32_t child0 = lv.next + uint32_t(sums[j]), job0 = uint32_t(sums[j]);
+  const uint32_t prim0 = jb.count > 0 ? jb.begin : lv.prims + uint32_t(sums[j] >> 32);
+  float lo[3] = {kInf, kInf, kInf}, hi[3] = {-kInf, -kInf, -kInf};
+  for (int i = 0; i < n; i++) {
+    float l[3], h[3];
+    slot_box(nodes, w[i], l, h);
+    for (int a = 0; a < 3; a++) lo[a] = fminf(lo[a], l[a]), hi[a] = fmaxf(hi[a], h[a]);
+  }
+  int slot[8], at[8];
+  wide_order(nodes, w, n, lo, hi, slot);
+  for (int s = 0; s < 8; s++) at[s] = -1;
+  for (int i = 0; i < n; i++) at[slot[i]] = i;
+  BvhNode8 o;
+  float cl[3][8], ch[3][8];
+  uint32_t valid = 0, imask = 0, placed = 0, k = 0;
+  uint32_t ends[2] = {0, 0};
+  uint32_t later = 0;  // wrapped leaves are placed behind the node's own
+  for (int i = 0; i < n; i++) later += wrap >> i & 1u ? 0u : cnt[i];
+  for (int s = 0; s < 8; s++) {
+    const int i = at[s];
+    if (i >= 0) {
+      float l[3], h[3];
+      slot_box(nodes, w[i], l, h);
+      for (int a = 0; a < 3; a++) cl[a][s] = l[a], ch[a][s] = h[a];
+      valid |= 1u << s;
+      uint32_t begin = prim0;
+      if (cnt[i] > 0 && jb.count == 0) {  // a leaf of the BvhNode4 tree gets its new place
+        const bool wrapped = wrap >> i & 1u;
+        begin += wrapped ? later : placed;
+        (wrapped ? later : placed) += cnt[i];
+        const uint32_t from = uint32_t(nodes[w[i].n].child[w[i].s]);
+        for (uint32_t q = 0; q < cnt[i]; q++) perm[begin + q] = from + q;
+        nodes[w[i].n].child[w[i].s] = int32_t(begin);
+      } else if (cnt[i] > 0) {
+        begin += uint32_t(i) * kWideNodePrims;
+        if (!(wrap >> i & 1u)) placed += cnt[i];
+      }
+      if (cnt[i] == 0 || (wrap >> i & 1u)) {
+        imask |= 1u << s;
+        next[job0 + k] = cnt[i] == 0 ? WideJob{uint32_t(nodes[w[i].n].child[w[i].s]), 0, 0, 0}
+                                     : WideJob{w[i].n, w[i].s, begin, cnt[i]};
+        k++;
+      }
+    }
+    ends[s >> 2] |= placed << (8 * (s & 3));
+  }
   uint32_t bx = 127, by = 127, bz = 127;
-  bool ok = quantize_axis(nd.lox, nd.hix, valid, o[0], h[0] - o[0], bx, q.qlox, q.qhix) &&
-            quantize_axis(nd.loy, nd.hiy, valid, o[1], h[1] - o[1], by, q.qloy, q.qhiy) &&
-            quantize_axis(nd.loz, nd.hiz, valid, o[2], h[2] - o[2], bz, q.qloz, q.qhiz);
-  if (!ok || nd.count[0] > 255u || nd.count[1] > 255u || nd.count[2] > 255u || nd.count[3] > 255u) atomicOr(error, 1u);
-  q.ox = o[0];
-  q.oy = o[1];
-  q.oz = o[2];
-  q.exps = bx | by << 8 | bz << 16;
-  out[i] = q;
+  const bool ok = quantize_axis(cl[0], ch[0], valid, lo[0], hi[0] - lo[0], bx, o.lox, o.hix) &&
+                  quantize_axis(cl[1], ch[1], valid, lo[1], hi[1] - lo[1], by, o.loy, o.hiy) &&
+                  quantize_axis(cl[2], ch[2], valid, lo[2], hi[2] - lo[2], bz, o.loz, o.hiz);
+  if (!ok) atomicOr(error, 1u);
+  o.ox = lo[0];
+  o.oy = lo[1];
+  o.oz = lo[2];
+  o.exps = bx | by << 8 | bz << 16 | imask << 24;
+  o.child_base = child0;
+  o.prim_base = prim0;
+  o.ends[0] = ends[0];
+  o.ends[1] = ends[1];
+  out[lv.nodes + j] = o;
 }
 
 unsigned Grid(uint64_t n, unsigned t = 256) { return unsigned((n + t - 1) / t); }
 
 }  // namespace
 
-void QuantizeBvh4(const DeviceBuffer& nodes, uint32_t m, hipStream_t st, DeviceBuffer& out) {
-  out.alloc(size_t(std::max(m, 1u)) * sizeof(BvhNodeQ));
-  DeviceBuffer err;
-  err.alloc(16);
-  HipCheck(hipMemsetAsync(err.ptr, 0, 4, st), "quantize flag");
-  if (m) hipLaunchKernelGGL(k_quantize, dim3(Grid(m)), dim3(256), 0, st, nodes.as<BvhNode4>(), m, out.as<BvhNodeQ>(),
-                            err.as<uint32_t>());
+uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, DeviceBuffer& prims, uint32_t n, hipStream_t st, DeviceBuffer& out) {
+  DeviceBuffer wide, jobs0, jobs1, sums, perm, flag, tmp;
+  flag.alloc(16);
+  HipCheck(hipMemsetAsync(flag.ptr, 0, 4, st), "wide node flag");
+  perm.alloc(size_t(std::max(n, 1u)) * 4);
+  const auto grow = [&](DeviceBuffer& b, size_t bytes, size_t keep) {  // at least `bytes`, the first `keep` kept
+    if (b.bytes >= bytes) return;
+    DeviceBuffer old;
+    std::swap(old.ptr, b.ptr);
+    std::swap(old.bytes, b.bytes);
+    b.alloc(std::max(bytes, 2 * keep));
+    if (keep) HipCheck(hipMemcpyAsync(b.ptr, old.ptr, keep, hipMemcpyDeviceToDevice, st), "wide nodes");
+    HipCheck(hipStreamSynchronize(st), "wide nodes");
+  };
+  grow(jobs0, 4096 * sizeof(WideJob), 0);
+  const WideJob root{0, 0, 0, 0};
+  HipCheck(hipMemcpyAsync(jobs0.ptr, &root, sizeof(root), hipMemcpyHostToDevice, st), "wide root");
+  DeviceBuffer *cur = &jobs0, *nxt = &jobs1;
+  uint32_t nJobs = 1;
+  WideLevel lv{0, 1, 0};
+  while (nJobs > 0) {
+    grow(wide, size_t(lv.nodes + nJobs) * sizeof(BvhNode8), size_t(lv.nodes) * sizeof(BvhNode8));
+    grow(sums, size_t(nJobs + 1) * 8, 0);
+    hipLaunchKernelGGL(k_wide<false>, dim3(Grid(nJobs + 1, 64)), dim3(64), 0, st, cur->as<WideJob>(), nJobs,
+                       nodes.as<BvhNode4>(), sums.as<unsigned long long>(), lv, nullptr, nullptr, nullptr, nullptr);
+    size_t bytes = 0;
+    HipCheck(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, sums.as<unsigned long long>(), sums.as<unsigned long long>(),
+                                              int(nJobs + 1), st),
+             "wide scan size");
+    grow(tmp, std::max<size_t>(bytes, 16), 0);
+    HipCheck(hipcub::DeviceScan::ExclusiveSum(tmp.ptr, bytes, sums.as<unsigned long long>(), sums.as<unsigned long long>(),
+                                              int(nJobs + 1), st),
+             "wide scan");
+    unsigned long long total = 0;
+    HipCheck(hipMemcpyAsync(&total, sums.as<unsigned long long>() + nJobs, 8, hipMemcpyDeviceToHost, st), "wide level");
+    HipCheck(hipStreamSynchronize(st), "wide level");
+    const uint32_t inner = uint32_t(total), placed = uint32_t(total >> 32);
+    if (placed > n - lv.prims) throw std::runtime_error("traversal nodes place more primitives than there are");
+    lv.next = lv.nodes + nJobs;
+    grow(*nxt, size_t(std::max(inner, 1u)) * sizeof(WideJob), 0);
+    hipLaunchKernelGGL(k_wide<true>, dim3(Grid(nJobs, 64)), dim3(64), 0, st, cur->as<WideJob>(), nJobs, nodes.as<BvhNode4>(),
+                       sums.as<unsigned long long>(), lv, wide.as<BvhNode8>(), nxt->as<WideJob>(), perm.as<uint32_t>(),
+                       flag.as<uint32_t>());
+    lv.nodes = lv.next;
+    lv.prims += placed;
+    nJobs = inner;
+    std::swap(cur, nxt);
+  }
+  if (lv.prims != n) throw std::runtime_error("traversal nodes do not reference every primitive");
+  out.alloc(size_t(lv.nodes) * sizeof(BvhNode8));
+  HipCheck(hipMemcpyAsync(out.ptr, wide.ptr, size_t(lv.nodes) * sizeof(BvhNode8), hipMemcpyDeviceToDevice, st), "wide nodes");
+  DeviceBuffer ordered;
+  ordered.alloc(size_t(std::max(n, 1u)) * 48);
+  if (n) hipLaunchKernelGGL(k_gather_prims, dim3(Grid(n)), dim3(256), 0, st, prims.as<float4>(), perm.as<uint32_t>(), n,
+                            ordered.as<float4>());
+  std::swap(prims.ptr, ordered.ptr);
+  std::swap(prims.bytes, ordered.bytes);
   uint32_t e = 0;
-  HipCheck(hipMemcpyAsync(&e, err.ptr, 4, hipMemcpyDeviceToHost, st), "quantize flag");
-  HipCheck(hipStreamSynchronize(st), "quantize");
+  HipCheck(hipMemcpyAsync(&e, flag.ptr, 4, hipMemcpyDeviceToHost, st), "wide node flag");
+  HipCheck(hipStreamSynchronize(st), "wide nodes");
   if (e) throw std::runtime_error("BVH node bounds cannot be quantised (non-finite boxes?)");
+  return lv.nodes;
 }
 
 void BuildBvh4Device(const float* bounds, const float4* records, uint32_t n, int maxLeaf, hipStream_t st,

@@ -2,6 +2,7 @@
 // BVH build, ray-batch intersection, asynchronous render jobs and the
 // per-function probes.  No exception crosses this boundary.
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <cstdlib>
@@ -269,11 +270,14 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
                                                  " traversal stack entries; the traversal holds " +
                                                  std::to_string(kTraceStackEntries));
     }
-    QuantizeBvh4(scene->d_nodes, nodeCount, scene->ctx->stream, scene->d_qnodes);
+    scene->wide_count = BuildWideNodes(scene->d_nodes, nodeCount, scene->d_prims, n, scene->ctx->stream, scene->d_wnodes);
     scene->builder = builder;
     scene->bvh_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     scene->dev.nodes = scene->d_nodes.as<BvhNode4>();
-    scene->dev.qnodes = scene->d_qnodes.as<BvhNodeQ>();
+    scene->dev.wnodes = scene->d_wnodes.as<BvhNode8>();
+    // RAD_TRACE_FAR=1 forces the 64-bit node addresses of trees of 4 GiB or
+    // more, so that tests can drive them; results do not depend on it.
+    scene->dev.wide_far = scene->wide_count >= (1u << 25) || std::getenv("RAD_TRACE_FAR") ? 1u : 0u;
     scene->dev.prims = scene->d_prims.as<float4>();
     scene->dev.prim_count = n;
     scene->dev.node_count = nodeCount;
@@ -349,6 +353,66 @@ rad_status rad_hip_autotune(rad_scene* scene, const rad_render_desc* probe, rad_
   });
 }
 
+// Errors of the traversal's nodes: primitives not referenced exactly once,
+// node references out of range or repeated, and child boxes that do not
+// contain the triangles and spheres below them.
+static uint32_t CheckWideNodes(const std::vector<BvhNode8>& wide, const std::vector<float4>& prims, uint32_t n) {
+  uint32_t errors = 0;
+  std::vector<uint8_t> seen(n, 0), parents(wide.size(), 0);
+  std::vector<std::array<float, 6>> bounds(wide.size());
+  for (size_t x = wide.size(); x-- > 0;) {  // children come after their parents
+    const BvhNode8& w = wide[x];
+    std::array<float, 6>& nb = bounds[x];
+    nb = {kInf, kInf, kInf, -kInf, -kInf, -kInf};
+    const float step[3] = {quant_step(w.exps), quant_step(w.exps >> 8), quant_step(w.exps >> 16)};
+    const float org[3] = {w.ox, w.oy, w.oz};
+    uint32_t inner = 0, begin = 0;
+    for (int s = 0; s < 8; s++) {
+      const uint32_t end = (w.ends[s >> 2] >> (8 * (s & 3))) & 0xffu;
+      std::array<float, 6> b = {kInf, kInf, kInf, -kInf, -kInf, -kInf};
+      if (w.exps >> 24 >> s & 1u) {
+        const uint32_t c = w.child_base + inner++;
+        if (c <= x || c >= wide.size()) {
+          errors++;
+          continue;
+        }
+        parents[c]++;
+        b = bounds[c];
+      } else {
+        for (uint32_t k = begin; k < end; k++) {
+          const uint64_t p = uint64_t(w.prim_base) + k;
+          if (p >= n || k >= kWideNodePrims) {
+            errors++;
+            continue;
+          }
+          if (seen[p]++) errors++;
+          const float4 r[3] = {prims[3 * p], prims[3 * p + 1], prims[3 * p + 2]};
+          uint32_t kind;
+          std::memcpy(&kind, &r[2].w, 4);
+          if (kind == PRIM_RECT) continue;  // bounded through their shape transform
+          for (int v = 0; v < (kind == PRIM_TRI ? 3 : 1); v++) {
+            const float q[3] = {r[v].x, r[v].y, r[v].z}, rad = kind == PRIM_TRI ? 0.f : r[0].w;
+            for (int a = 0; a < 3; a++) b[a] = std::min(b[a], q[a] - rad), b[3 + a] = std::max(b[3 + a], q[a] + rad);
+          }
+        }
+      }
+      begin = end;
+      const uint16_t* lo[3] = {w.lox, w.loy, w.loz};
+      const uint16_t* hi[3] = {w.hix, w.hiy, w.hiz};
+      for (int a = 0; a < 3; a++) {
+        if (b[a] <= b[3 + a] && !(dequant(plane_value(lo[a][s]), step[a], org[a]) <= b[a] &&
+                                  dequant(plane_value(hi[a][s]), step[a], org[a]) >= b[3 + a]))
+          errors++;
+        nb[a] = std::min(nb[a], b[a]);
+        nb[3 + a] = std::max(nb[3 + a], b[3 + a]);
+      }
+    }
+  }
+  for (uint32_t p = 0; p < n; p++) errors += seen[p] != 1;
+  for (size_t x = 0; x < wide.size(); x++) errors += parents[x] != (x ? 1 : 0);
+  return errors;
+}
+
 rad_status rad_hip_bvh_check(rad_scene* scene, rad_bvh_report* rep) {
   if (!scene || !rep) return Fail(RAD_ERR_INVALID_ARG, "NULL argument");
   return Guard([&] {
@@ -357,11 +421,11 @@ rad_status rad_hip_bvh_check(rad_scene* scene, rad_bvh_report* rep) {
     HipCheck(hipSetDevice(scene->ctx->device), "hipSetDevice");
     const uint32_t m = scene->dev.node_count, n = scene->dev.prim_count;
     std::vector<BvhNode4> nodes(m);
-    std::vector<BvhNodeQ> qnodes(m);
+    std::vector<BvhNode8> wide(scene->wide_count);
     std::vector<float4> prims(3 * size_t(n));
     HipCheck(hipMemcpy(nodes.data(), scene->d_nodes.ptr, size_t(m) * sizeof(BvhNode4), hipMemcpyDeviceToHost), "nodes");
-    HipCheck(hipMemcpy(qnodes.data(), scene->d_qnodes.ptr, size_t(m) * sizeof(BvhNodeQ), hipMemcpyDeviceToHost),
-             "quantised nodes");
+    HipCheck(hipMemcpy(wide.data(), scene->d_wnodes.ptr, wide.size() * sizeof(BvhNode8), hipMemcpyDeviceToHost),
+             "traversal nodes");
     HipCheck(hipMemcpy(prims.data(), scene->d_prims.ptr, prims.size() * sizeof(float4), hipMemcpyDeviceToHost), "prims");
     std::memset(rep, 0, sizeof(*rep));
     std::vector<uint8_t> seen(n, 0), visited(m, 0);
@@ -378,23 +442,6 @@ rad_status rad_hip_bvh_check(rad_scene* scene, rad_bvh_report* rep) {
       visited[x] = 1;
       rep->depth = std::max(rep->depth, d);
       const BvhNode4& nd = nodes[x];
-      {  // the traversal copy: same children and counts, dequantised boxes around the exact ones
-        const BvhNodeQ& qn = qnodes[x];
-        const float sx = quant_step(qn.exps), sy = quant_step(qn.exps >> 8), sz = quant_step(qn.exps >> 16);
-        for (int s = 0; s < 4; s++) {
-          if (qn.child[s] != nd.child[s]) {
-            rep->quantized_box_violations++;
-            continue;
-          }
-          if (nd.child[s] < 0) continue;
-          const int sh = 8 * s;
-          if (((qn.counts >> sh) & 0xffu) != nd.count[s] ||
-              !(dequant((qn.qlox >> sh) & 0xffu, sx, qn.ox) <= nd.lox[s] && dequant((qn.qhix >> sh) & 0xffu, sx, qn.ox) >= nd.hix[s] &&
-                dequant((qn.qloy >> sh) & 0xffu, sy, qn.oy) <= nd.loy[s] && dequant((qn.qhiy >> sh) & 0xffu, sy, qn.oy) >= nd.hiy[s] &&
-                dequant((qn.qloz >> sh) & 0xffu, sz, qn.oz) <= nd.loz[s] && dequant((qn.qhiz >> sh) & 0xffu, sz, qn.oz) >= nd.hiz[s]))
-            rep->quantized_box_violations++;
-        }
-      }
       for (int s = 0; s < 4; s++) {
         if (nd.child[s] < 0) continue;
         if (nd.count[s] > 0) {
@@ -445,6 +492,7 @@ rad_status rad_hip_bvh_check(rad_scene* scene, rad_bvh_report* rep) {
       if (seen[p] != 1) rep->unreferenced_or_repeated++;
     for (uint32_t x = 0; x < m; x++)
       if (!visited[x]) rep->structure_errors++;
+    rep->quantized_box_violations = CheckWideNodes(wide, prims, n);
     rep->node_count = m;
     rep->primitive_count = n;
     rep->sah_cost = BvhSahCost(nodes);

@@ -1,5 +1,5 @@
-// Wavefront kernels of the `path` integrator (renderer/path.cpp:131-227) and
-// the ray-batch intersection kernels (accel/embree.cpp:79-111).
+// Wavefront kernels of the `path` integrator (renderer/path.cpp:131-227); its
+// traversal kernels are in trace_kernels.hip.
 #include <algorithm>
 
 #include "guide_dev.h"
@@ -166,61 +166,6 @@ __global__ void k_reset(uint32_t* cnt, uint32_t* gcnt, int out) {
     cnt[CNT_SUSP + out] = 0;  // resume pool `out` was drained by the previous extend
     if (gcnt) gcnt[G_QUEUE] = 0;
   }
-}
-
-// The tag of an extend ray is its queue position; its state index is base + tag.
-struct ExtendJob {
-  static constexpr bool kSuspend = true;
-  static constexpr bool kTagIsIndex = true;
-  uint32_t base;
-  const float4* ray;
-  float4* hit;
-  uint32_t* hit_geom;
-  uint32_t* susp;                 // null: traversals run to the end
-  const ResumeState* rin;         // pool this launch resumes from
-  ResumeState* rout;              // pool this launch suspends into
-  uint32_t* rcount;               // entries of rout
-  uint32_t cap, budget;
-  __device__ __forceinline__ void resume(uint32_t i, TraceRay& r, TraceStack& st) {
-    if (!susp) return;
-    const uint32_t s = base + i;
-    const uint32_t j = susp[s];
-    if (j == kNoSusp) return;
-    restore_trace(rin[j], r, st);
-    susp[s] = kNoSusp;
-  }
-  __device__ __forceinline__ bool suspend(uint32_t i, const TraceRay& r, const TraceStack& st) {
-    const uint32_t j = atomicAdd(rcount, 1u);
-    if (j >= cap) return false;  // pool full: the ray finishes in this launch
-    save_trace(rout[j], r, st);
-    susp[base + i] = j;
-    return true;
-  }
-  __device__ __forceinline__ bool load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax, uint32_t& tag) {
-    float4 a = ray[2 * size_t(i)], b = ray[2 * size_t(i) + 1];
-    o = mk(a.x, a.y, a.z);
-    d = mk(b.x, b.y, b.z);
-    tmin = a.w;
-    tmax = b.w;
-    tag = i;
-    return true;
-  }
-  // hits are stored by extend-queue position: consecutive rays of the
-  // queue write consecutive entries, and classify reads them in order
-  __device__ __forceinline__ void finish(uint32_t i, uint32_t, const TraceRay& r) {
-    hit[i] = make_float4(r.h.t, r.h.u, r.h.v, __uint_as_float(r.hit ? r.h.prim : 0u));
-    hit_geom[i] = r.hit ? r.h.geom : 0xffffffffu;
-  }
-};
-
-// Capped at 80 VGPRs (6 waves per SIMD; four registers spill): traversal
-// waits on node and primitive loads, and resident waves hide that wait, but
-// the pooled primitive tests need registers; per 1080p large-mesh frame
-// 78.2 ms at 6 waves, 84.8 ms at 5.
-__global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6))) k_extend(Wavefront w, DevScene scene, int in) {
-  ExtendJob job{state_index(w.Q, in, 0), w.ray[in], w.hit, w.hit_geom, w.susp, w.resume[in], w.resume[1 - in],
-                &w.cnt[CNT_SUSP + 1 - in], w.resume_cap, w.susp ? w.visit_budget : 0xffffffffu};
-  trace_stream<false>(scene, w.cnt[in], &w.cnt[CNT_FETCH_EXT], job);
 }
 
 // A vertex is guided when it is a surface hit at depth <= max_depth, on a
@@ -758,35 +703,6 @@ __global__ void k_queue_verify(Wavefront w, uint32_t* tally) {
   if (bad) atomicAdd(&w.stats[ST_QERR], (unsigned long long)bad);
 }
 
-struct ShadowJob {
-  static constexpr bool kSuspend = false;
-  static constexpr bool kTagIsIndex = false;
-  const float4 *sh_o, *sh_d, *sh_c;
-  SlotField<float4> lsum;
-  __device__ __forceinline__ bool load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax, uint32_t& tag) {
-    float4 a = sh_o[i], b = sh_d[i];
-    o = mk(a.x, a.y, a.z);
-    d = mk(b.x, b.y, b.z);
-    tmin = 0.f;
-    tmax = a.w;
-    tag = __float_as_uint(b.w);
-    return true;
-  }
-  __device__ __forceinline__ void finish(uint32_t i, uint32_t s, const TraceRay& r) {
-    if (r.hit) return;  // occluded
-    float4 c = sh_c[i];
-    float4 l = lsum[s];
-    lsum[s] = make_float4(l.x + c.x, l.y + c.y, l.z + c.z, l.w);
-  }
-};
-
-// Capped at 72 VGPRs (7 waves per SIMD; five registers spill): per 1080p
-// large-mesh frame 32.1 ms at 7 waves, 33.6 ms at 6.
-__global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(7))) k_shadow(Wavefront w, DevScene scene) {
-  ShadowJob job{w.sh_o, w.sh_d, w.sh_c, w.lsum};
-  trace_stream<true>(scene, w.cnt[CNT_SHADOW], &w.cnt[CNT_FETCH_SH], job);
-}
-
 // Add the pass's samples of each pixel in sample order, dropping the ones
 // the reference drops (sample_renderer.cpp:100-105: NaN anywhere; infinite
 // or negative values, which the reference's HasInfinity / HasNegative look
@@ -828,57 +744,6 @@ __global__ void k_final(Wavefront w, float* fb, float* sq) {
     sq[3 * p + 1] = a2.y;
     sq[3 * p + 2] = a2.z;
   }
-}
-
-struct ClosestJob {
-  static constexpr bool kSuspend = false;
-  static constexpr bool kTagIsIndex = false;
-  const float4* rays;
-  float* hits;
-  __device__ __forceinline__ bool load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax, uint32_t& tag) {
-    float4 a = rays[2 * i], b = rays[2 * i + 1];
-    o = mk(a.x, a.y, a.z);
-    d = mk(b.x, b.y, b.z);
-    tmin = a.w;
-    tmax = b.w;
-    tag = __float_as_uint(b.w);
-    return true;
-  }
-  __device__ __forceinline__ void finish(uint32_t i, uint32_t tmax_bits, const TraceRay& r) {
-    float* o = hits + 5 * size_t(i);
-    o[0] = r.hit ? r.h.t : __uint_as_float(tmax_bits);
-    o[1] = r.hit ? r.h.u : 0.f;
-    o[2] = r.hit ? r.h.v : 0.f;
-    o[3] = __uint_as_float(r.hit ? r.h.prim : 0xffffffffu);
-    o[4] = __uint_as_float(r.hit ? r.h.geom : 0xffffffffu);
-  }
-};
-
-struct AnyJob {
-  static constexpr bool kSuspend = false;
-  static constexpr bool kTagIsIndex = false;
-  const float4* rays;
-  uint8_t* occ;
-  __device__ __forceinline__ bool load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax, uint32_t& tag) {
-    float4 a = rays[2 * i], b = rays[2 * i + 1];
-    o = mk(a.x, a.y, a.z);
-    d = mk(b.x, b.y, b.z);
-    tmin = a.w;
-    tmax = b.w;
-    tag = 0;
-    return true;
-  }
-  __device__ __forceinline__ void finish(uint32_t i, uint32_t, const TraceRay& r) { occ[i] = r.hit ? 1 : 0; }
-};
-
-__global__ void __launch_bounds__(kTraceBlock) k_closest(DevScene scene, const float4* rays, uint32_t n, float* hits) {
-  ClosestJob job{rays, hits};
-  trace_stream<false>(scene, n, nullptr, job);
-}
-
-__global__ void __launch_bounds__(kTraceBlock) k_any(DevScene scene, const float4* rays, uint32_t n, uint8_t* occ) {
-  AnyJob job{rays, occ};
-  trace_stream<true>(scene, n, nullptr, job);
 }
 
 __global__ void k_bsdf_eval(BsdfRec b, bool quirks, const float* in, uint32_t n, float* out) {
@@ -924,9 +789,6 @@ void LaunchRegen(const Wavefront& w, const DevScene& scene, int in, bool fresh, 
 }
 void LaunchReset(const Wavefront& w, int out, hipStream_t s) {
   hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, w.cnt, w.gcnt, out);
-}
-void LaunchExtend(const Wavefront& w, const DevScene& scene, int in, const LaunchCfg& c, hipStream_t s) {
-  hipLaunchKernelGGL(k_extend, dim3(c.trace_blocks), dim3(kTraceBlock), 0, s, w, scene, in);
 }
 // TX: texture code compiled in.  The four specialised material kernels need
 // it only for textured emitters (textured BSDFs are queued as "others"); the
@@ -992,23 +854,11 @@ void LaunchGuideInfer(const Wavefront& w, const DevScene& scene, int in, int blo
   else
     hipLaunchKernelGGL(k_guide_infer_hits<false>, dim3(blocks), dim3(kInferBlock), 0, s, w, scene, in);
 }
-void LaunchShadow(const Wavefront& w, const DevScene& scene, const LaunchCfg& c, hipStream_t s) {
-  hipLaunchKernelGGL(k_shadow, dim3(c.trace_blocks), dim3(kTraceBlock), 0, s, w, scene);
-}
 void LaunchAccum(const Wavefront& w, hipStream_t s) {
   hipLaunchKernelGGL(k_accum, dim3(Blocks(w.npix, 256)), dim3(256), 0, s, w);
 }
 void LaunchFinal(const Wavefront& w, float* fb, float* sq, hipStream_t s) {
   hipLaunchKernelGGL(k_final, dim3(Blocks(w.npix, 256)), dim3(256), 0, s, w, fb, sq);
-}
-void LaunchClosest(const DevScene& scene, const void* rays, uint32_t n, void* hits, hipStream_t s) {
-  if (n)
-    hipLaunchKernelGGL(k_closest, dim3(Blocks(n, kTraceBlock)), dim3(kTraceBlock), 0, s, scene, (const float4*)rays, n,
-                       (float*)hits);
-}
-void LaunchAny(const DevScene& scene, const void* rays, uint32_t n, uint8_t* occ, hipStream_t s) {
-  if (n)
-    hipLaunchKernelGGL(k_any, dim3(Blocks(n, kTraceBlock)), dim3(kTraceBlock), 0, s, scene, (const float4*)rays, n, occ);
 }
 void LaunchBsdfEval(const BsdfRec& b, bool quirks, const float* in, uint32_t n, float* out, hipStream_t s) {
   if (n) hipLaunchKernelGGL(k_bsdf_eval, dim3(Blocks(n, 128)), dim3(128), 0, s, b, quirks, in, n, out);

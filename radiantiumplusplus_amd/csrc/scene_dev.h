@@ -1,14 +1,14 @@
 // Device-resident scene layout.
 //
 // Geometry for traversal lives in two HBM arrays:
-//   nodes  - 4-wide BVH nodes, 128 B each (one cache line): six 4-float slab
-//            planes, four child links, four leaf counts;
+//   wnodes - 8-wide quantised BVH nodes, 128 B each (one cache line);
 //   prims  - primitives in leaf order, three float4 (48 B) each:
 //            triangle: (v0, geomID) (v1, primID) (v2, PRIM_TRI)
 //            sphere:   (center, radius) (-, geomID) (-, PRIM_SPHERE)
 //            rectangle:(-) (-, geomID) (-, PRIM_RECT); matrix in its ShapeRec.
 // Shading data (vertex attributes, per-shape records, BSDF / light / medium
-// records) is separate, so traversal touches only nodes + prims.
+// records) is separate, so traversal touches only wnodes + prims.  The 4-wide
+// full-precision tree the builders make is kept for checks and statistics.
 #pragma once
 
 #include "../../include/rad_hip.h"
@@ -33,25 +33,58 @@ static_assert(sizeof(BvhNode4) == 128, "BVH node must be one 128-byte line");
 // entries (0 for a node whose children are all leaves); the builders compute
 // need(root) and a tree that needs more than this is refused.
 constexpr uint32_t kTraceStackEntries = 64;
+// Entries of the traversal's own stack.  It holds groups of siblings still to
+// be visited, one per BvhNode8 on the way down that has more than one inner
+// child; such a node holds a BvhNode4 with more than one inner child on the
+// same way, so the need is at most the BvhNode4 tree's, plus two for leaves
+// that get nodes of their own (kWideNodePrims).
+constexpr uint32_t kGroupStackEntries = kTraceStackEntries + 2;
 // Entries of a wave's pooled primitive tests per node step (traverse.h); a
 // lane whose entries fall beyond the pool tests them itself.
 constexpr uint32_t kTracePool = 64;
 
-// The traversal's copy of a BvhNode4 in 64 bytes: the node box origin, a
-// power-of-two step per axis, and every child's bounds as 8-bit multiples of
-// the step, rounded outward, so each child box contains the exact one.  A
-// dequantised bound is fmaf(q, step, origin): one rounding, computed the same
-// way when the node is built, where the outward rounding is verified.
-struct alignas(64) BvhNodeQ {
+// The traversal's node: up to eight children, one 128-byte L2 line, built from
+// the BvhNode4 tree by opening inner children (bvh_gpu.hip).  Child planes are
+// integers 0..2047 held as binary16 (exact), in multiples of a power-of-two
+// step from the node's origin, rounded outward, so each child box contains the
+// exact one.  A dequantised bound is fmaf(q, step, origin): one rounding,
+// computed the same way when the node is built, where the outward rounding is
+// verified.  The eight 16-byte chunks are placed so that the near and far
+// planes of x, y, z are chosen by one address bit each (16, 32 and 64): a ray
+// loads its near plane at `near chunk | (direction negative ? bit : 0)` and its
+// far plane at that address ^ bit, and no plane is selected in registers.
+//
+// Slot i holds the child whose centre lies, as far as the slots allow, on the
+// positive side of axis a where bit a of i is set: a ray visits the slots in
+// the order of slot ^ (its negative axes).  Inner children are consecutive in
+// slot order from child_base; the primitives of the leaf children are
+// consecutive in slot order from prim_base (ends: byte i = where slot i's end).
+struct alignas(128) BvhNode8 {
+  uint16_t lox[8], hix[8];
   float ox, oy, oz;
-  uint32_t exps;                    // biased exponents of the x, y, z steps (bytes 0, 1, 2)
-  uint32_t qlox, qhix, qloy, qhiy;  // child i's bound in byte i
-  uint32_t qloz, qhiz;
-  uint32_t counts;                  // child i's leaf primitive count in byte i (0: inner)
-  uint32_t pad;
-  int32_t child[4];                 // as in BvhNode4
+  uint32_t exps;  // biased exponents of the x, y, z steps (bytes 0, 1, 2); byte 3: mask of the inner children
+  uint16_t loz[8];
+  uint16_t loy[8];
+  uint32_t child_base, prim_base;
+  uint32_t ends[2];
+  uint16_t hiy[8];
+  uint16_t hiz[8];
 };
-static_assert(sizeof(BvhNodeQ) == 64, "quantised BVH node must be 64 bytes");
+static_assert(sizeof(BvhNode8) == 128, "traversal node must be one 128-byte line");
+constexpr uint32_t kWidePlaneMax = 2047;  // largest plane value (every integer up to 2048 is exact in binary16)
+constexpr uint32_t kWideNodePrims = 32;   // most primitives in the leaf children of one node
+
+// binary16 bits of an integer 0..2047, and back.
+__host__ __device__ inline uint16_t plane_bits(uint32_t q) {
+  if (q == 0) return 0;
+  int e = 0;
+  while (q >> (e + 1)) e++;
+  return uint16_t(((e + 15) << 10) | ((q << (10 - e)) & 0x3ffu));
+}
+__host__ __device__ inline uint32_t plane_value(uint16_t h) {
+  const int e = int(h >> 10) - 15;
+  return h == 0 ? 0u : ((0x400u | (h & 0x3ffu)) >> (10 - e));
+}
 
 __host__ __device__ inline float quant_step(uint32_t biased) {
   union {
@@ -195,7 +228,7 @@ struct CameraRec {
 
 struct DevScene {
   const BvhNode4* nodes;   // full-precision nodes (checks, statistics)
-  const BvhNodeQ* qnodes;  // traversal copy
+  const BvhNode8* wnodes;  // traversal nodes
   const float4* prims;
   uint32_t prim_count, node_count;
   const ShapeRec* shapes;
@@ -227,6 +260,7 @@ struct DevScene {
   f3 world_center;
   float world_radius;
   uint32_t quirks;
+  uint32_t wide_far;  // 1: the traversal nodes take 4 GiB or more (32-bit byte offsets do not reach them)
   uint32_t pool_cap;  // pooled primitive tests per wave step, 1..kTracePool (smaller only to test the overflow path)
 };
 

@@ -87,12 +87,13 @@ struct rad_scene {
   rad_ctx* ctx = nullptr;
   rad::HostScene host;
   rad::DevScene dev{};
-  rad::DeviceBuffer d_nodes, d_qnodes, d_prims, d_shapes, d_pos, d_nrm, d_uv, d_idx, d_tris, d_bsdfs, d_lights, d_cdf, d_media, d_grid,
+  rad::DeviceBuffer d_nodes, d_wnodes, d_prims, d_shapes, d_pos, d_nrm, d_uv, d_idx, d_tris, d_bsdfs, d_lights, d_cdf, d_media, d_grid,
       d_tex, d_texels, d_ldist;
   rad::DeviceBuffer d_rays, d_hits, d_occ;  // staging for the host-pointer intersect entry points
   std::mutex mu;
   bool bvh_ready = false;
   double bvh_ms = 0;
+  uint32_t wide_count = 0;  // traversal nodes
   uint32_t bvh_depth = 0;
   uint32_t bvh_stack_need = 0;
   int32_t builder = -1;

@@ -1,5 +1,4 @@
-// Device ray traversal over the 4-wide BVH (its 64-byte quantised copy):
-// closest hit
+// Device ray traversal over the 8-wide quantised BVH: closest hit
 // (Embree::RayIntersectPreliminary, embree.cpp:87-111) and occlusion
 // (Embree::RayIntersect, embree.cpp:79-85).
 #pragma once
@@ -118,24 +117,26 @@ __device__ __forceinline__ bool isect_rect(const Affine& toObj, f3 ro, f3 rd, fl
 
 __device__ __forceinline__ f3 xyz(float4 a) { return mk(a.x, a.y, a.z); }
 
-// Test one primitive record; on a hit narrows `tfar` to its distance.
-__device__ __forceinline__ bool isect_prim(const DevScene& s, uint32_t p, f3 o, f3 d, float tnear, float& tfar) {
-  const float4* rec = s.prims + 3 * size_t(p);
-  const float4 c = rec[2];
+// Test one primitive record (its three float4, already loaded); on a hit
+// narrows `tfar` to its distance.
+__device__ __forceinline__ bool isect_rec(const DevScene& s, float4 a, float4 b, float4 c, f3 o, f3 d, float tnear,
+                                          float& tfar) {
   const uint32_t kind = __float_as_uint(c.w);
   float t;
   if (kind == PRIM_TRI) {
-    const float4 a = rec[0], b = rec[1];
     if (!isect_tri(xyz(a), xyz(b), xyz(c), o, d, tnear, tfar, t)) return false;
   } else if (kind == PRIM_SPHERE) {
-    const float4 a = rec[0];
     if (!isect_sphere(xyz(a), a.w, o, d, tnear, tfar, t)) return false;
   } else {
     float u, v;
-    if (!isect_rect(s.shapes[__float_as_uint(rec[1].w)].to_local, o, d, tnear, tfar, t, u, v)) return false;
+    if (!isect_rect(s.shapes[__float_as_uint(b.w)].to_local, o, d, tnear, tfar, t, u, v)) return false;
   }
   tfar = t;
   return true;
+}
+__device__ __forceinline__ bool isect_prim(const DevScene& s, uint32_t p, f3 o, f3 d, float tnear, float& tfar) {
+  const float4* rec = s.prims + 3 * size_t(p);
+  return isect_rec(s, rec[0], rec[1], rec[2], o, d, tnear, tfar);
 }
 
 // The hit record of primitive p at distance t (the closest hit the
@@ -165,75 +166,95 @@ __device__ __forceinline__ void prim_hit(const DevScene& s, uint32_t p, f3 o, f3
 }
 
 // ---------------------------------------------------------------- traversal
-// Each lane keeps its traversal stack as (node, entry distance) pairs: the
-// newest kLdsStack entries in LDS (a ring, lane-interleaved so a wave's
-// accesses hit distinct banks), older ones spilled to a private overflow
-// array that only deep traversals touch.
-constexpr int kStackDepth = int(kTraceStackEntries);
-constexpr int kLdsStack = 8;
+// A ray walks groups of siblings: the inner children of one node that it hits
+// are one group (first child's index, hit mask in visiting order, the node's
+// inner mask), the current group is in registers, and a node whose own group
+// replaces an unfinished one pushes that one: at most one push per node, and
+// none for the children themselves.  Each lane keeps the newest kLdsStack
+// entries in LDS (a ring, lane-interleaved so a wave's accesses are
+// conflict-free), older ones in a private overflow array that only deep
+// traversals touch.
+constexpr int kStackDepth = int(kGroupStackEntries);
+constexpr int kLdsStack = 4;
 constexpr int kTraceBlock = 256;  // threads per block of every traversal kernel
 
-// LDS pointers spelled with their address space, so stack accesses compile
-// to ds_read / ds_write rather than flat accesses.
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-typedef __attribute__((address_space(3))) float lds_f32;
+// LDS pointers spelled with their address space, so accesses compile to
+// ds_read / ds_write rather than flat accesses.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) u32x2 lds_u2;
+typedef __attribute__((address_space(3))) u32x4 lds_u4;
+typedef __attribute__((address_space(3))) unsigned long long lds_u64;
 
 // Per-lane private overflow of a traversal stack (entries below the LDS ring).
 struct TraceOverflow {
-  uint32_t node[kStackDepth - kLdsStack];
-  float dist[kStackDepth - kLdsStack];
+  uint2 e[kStackDepth - kLdsStack];
 };
 
 // The struct holds no arrays, so its fields stay in registers; only the
 // overflow array, indexed by the stack depth, lives in private memory.
 struct TraceStack {
-  lds_u32* node;  // LDS, entry k of this lane at node[k * kTraceBlock]
-  lds_f32* dist;
-  uint32_t* ov_node;  // TraceOverflow of this lane
-  float* ov_dist;
-  int sp, lo;  // entries [0, lo) live in the overflow array, [lo, sp) in LDS
+  lds_u64* ring;  // entry k of this lane at ring[k * kTraceBlock]
+  uint2* ov;      // TraceOverflow of this lane
+  int sp, lo;     // entries [0, lo) live in the overflow array, [lo, sp) in LDS
 
-  __device__ __forceinline__ void push(uint32_t n, float d) {
+  static __device__ __forceinline__ unsigned long long pack(uint32_t base, uint32_t mask) {
+    return (static_cast<unsigned long long>(mask) << 32) | base;
+  }
+  __device__ __forceinline__ void push(uint32_t base, uint32_t mask) {
     if (sp >= kStackDepth) return;  // unreachable: the builders refuse trees that need more entries
     if (sp - lo == kLdsStack) {
-      int k = (lo & (kLdsStack - 1)) * kTraceBlock;
-      ov_node[lo] = node[k];
-      ov_dist[lo] = dist[k];
+      const unsigned long long e = ring[(lo & (kLdsStack - 1)) * kTraceBlock];
+      ov[lo] = make_uint2(uint32_t(e), uint32_t(e >> 32));
       lo++;
     }
-    int k = (sp & (kLdsStack - 1)) * kTraceBlock;
-    node[k] = n;
-    dist[k] = d;
+    ring[(sp & (kLdsStack - 1)) * kTraceBlock] = pack(base, mask);
     sp++;
   }
-  __device__ __forceinline__ void pop(uint32_t& n, float& d) {
+  __device__ __forceinline__ void pop(uint32_t& base, uint32_t& mask) {
     sp--;
     if (sp < lo) {
       lo = sp;
-      n = ov_node[sp];
-      d = ov_dist[sp];
+      const uint2 e = ov[sp];
+      base = e.x;
+      mask = e.y;
     } else {
-      int k = (sp & (kLdsStack - 1)) * kTraceBlock;
-      n = node[k];
-      d = dist[k];
+      const unsigned long long e = ring[(sp & (kLdsStack - 1)) * kTraceBlock];
+      base = uint32_t(e);
+      mask = uint32_t(e >> 32);
     }
   }
 };
 
+// The closest hit is the minimum of (t, primitive) over the accepted
+// primitives, whatever order they are tested in: an unsigned key in that
+// order (t may be negative where tmin is).
+__device__ __forceinline__ unsigned long long hit_key(float t, uint32_t prim) {
+  const uint32_t u = __float_as_uint(t);
+  return (static_cast<unsigned long long>(u ^ (uint32_t(int32_t(u) >> 31) | 0x80000000u)) << 32) | prim;
+}
+__device__ __forceinline__ float key_t(unsigned long long key) {
+  const uint32_t u = uint32_t(key >> 32);
+  return __uint_as_float(u ^ (uint32_t(~int32_t(u) >> 31) | 0x80000000u));
+}
+
 struct TraceRay {
   f3 o, d;
-  f3 inv;           // 1 / d, components below 1e-18 in magnitude raised to it (sign kept)
-  bool nx, ny, nz;  // direction components negative: the near plane is the box's high bound
-  float tmin, tfar;  // tfar: the closest hit's distance once hit is set
+  f3 inv;          // 1 / d, components below 1e-18 in magnitude raised to it (sign kept)
+  uint32_t oct;    // negative axes: bit 4 x, bit 5 y, bit 6 z (the address bits of a node's plane chunks)
+  float tmin, tfar;  // tfar: the closest hit's distance once there is one
   uint32_t node;
-  uint32_t hitp;  // primitive record of the closest hit
-  bool hit;
-  Hit h;  // filled by trace_finish
+  uint32_t gbase, gmask;  // current group: first inner child; bits 0-7 children to visit, in visiting order; 8-15 inner mask
+  uint32_t hitp;   // primitive record of the closest hit, kNoHit: none
+  Hit h;           // filled by trace_finish
+  static constexpr uint32_t kNoHit = 0xffffffffu;
+  __device__ __forceinline__ bool hit() const { return hitp != kNoHit; }
+  __device__ __forceinline__ unsigned long long key() const { return hit_key(tfar, hitp); }
 };
 
 // Fills the hit record of a finished closest-hit traversal.
 __device__ __forceinline__ void trace_finish(const DevScene& s, TraceRay& r) {
-  if (r.hit) {
+  if (r.hit()) {
     prim_hit(s, r.hitp, r.o, r.d, r.tfar, r.h);
   } else {
     r.h.t = r.tfar;
@@ -244,30 +265,29 @@ __device__ __forceinline__ void trace_finish(const DevScene& s, TraceRay& r) {
 }
 
 // A closest-hit traversal interrupted at a launch's visit budget: the node
-// to visit next, the pending stack, the closest hit so far.  Resuming it
-// replays nothing, so the result is the one an uninterrupted traversal gives.
+// to visit next, the current group and the pending ones, the closest hit so
+// far.  Resuming it replays nothing, so the result is the one an
+// uninterrupted traversal gives.
 struct ResumeState {
-  uint32_t node, sp, hit, hitp;
+  uint32_t node, sp, gbase, gmask, hitp;
   float tfar;
-  uint32_t pad[7];
-  uint32_t stack_node[kStackDepth];
-  float stack_dist[kStackDepth];
+  uint32_t pad[2];
+  uint2 stack[kStackDepth];
 };
 
 __device__ inline void save_trace(ResumeState& rs, const TraceRay& r, const TraceStack& st) {
   rs.node = r.node;
   rs.sp = uint32_t(st.sp);
-  rs.hit = r.hit ? 1u : 0u;
+  rs.gbase = r.gbase;
+  rs.gmask = r.gmask;
   rs.hitp = r.hitp;
   rs.tfar = r.tfar;
   for (int k = 0; k < st.sp; k++) {
     if (k < st.lo) {
-      rs.stack_node[k] = st.ov_node[k];
-      rs.stack_dist[k] = st.ov_dist[k];
+      rs.stack[k] = st.ov[k];
     } else {
-      const int j = (k & (kLdsStack - 1)) * kTraceBlock;
-      rs.stack_node[k] = st.node[j];
-      rs.stack_dist[k] = st.dist[j];
+      const unsigned long long e = st.ring[(k & (kLdsStack - 1)) * kTraceBlock];
+      rs.stack[k] = make_uint2(uint32_t(e), uint32_t(e >> 32));
     }
   }
 }
@@ -275,11 +295,12 @@ __device__ inline void save_trace(ResumeState& rs, const TraceRay& r, const Trac
 // After trace_begin on the same ray.
 __device__ inline void restore_trace(const ResumeState& rs, TraceRay& r, TraceStack& st) {
   r.node = rs.node;
-  r.hit = rs.hit != 0;
+  r.gbase = rs.gbase;
+  r.gmask = rs.gmask;
   r.hitp = rs.hitp;
   r.tfar = rs.tfar;
   const int n = min(int(rs.sp), kStackDepth);
-  for (int k = 0; k < n; k++) st.push(rs.stack_node[k], rs.stack_dist[k]);
+  for (int k = 0; k < n; k++) st.push(rs.stack[k].x, rs.stack[k].y);
 }
 
 __device__ __forceinline__ void trace_begin(TraceRay& r, TraceStack& st, f3 o, f3 d, float tmin, float tmax) {
@@ -289,37 +310,15 @@ __device__ __forceinline__ void trace_begin(TraceRay& r, TraceStack& st, f3 o, f
   // inf - inf; a tiny one of the same sign keeps every slab finite.
   const auto safe = [](float x) { return fabsf(x) < 1e-18f ? copysignf(1e-18f, x) : x; };
   r.inv = mk(1.0f / safe(d.x), 1.0f / safe(d.y), 1.0f / safe(d.z));
-  r.nx = r.inv.x < 0.f;
-  r.ny = r.inv.y < 0.f;
-  r.nz = r.inv.z < 0.f;
+  r.oct = (r.inv.x < 0.f ? 16u : 0u) | (r.inv.y < 0.f ? 32u : 0u) | (r.inv.z < 0.f ? 64u : 0u);
   r.tmin = tmin;
   r.tfar = tmax;
   r.node = 0;
-  r.hit = false;
-  r.hitp = 0xffffffffu;
+  r.gbase = r.gmask = 0;
+  r.hitp = TraceRay::kNoHit;
   st.sp = 0;
   st.lo = 0;
 }
-
-__device__ __forceinline__ void cswap(float& da, uint32_t& na, float& db, uint32_t& nb) {
-  bool sw = db < da;
-  float td = sw ? db : da;
-  uint32_t tn = sw ? nb : na;
-  db = sw ? da : db;
-  nb = sw ? na : nb;
-  da = td;
-  na = tn;
-}
-
-// Per-wave LDS of the pooled primitive tests: a counter, kPoolSize
-// (primitive, owner lane) entries and one closest-hit key per lane.
-constexpr uint32_t kPoolSize = kTracePool;
-struct PrimPool {
-  lds_u32* ctr;    // entries posted in this node step
-  lds_u32* prim;   // [kPoolSize]
-  lds_u32* owner;  // [kPoolSize]
-  __attribute__((address_space(3))) unsigned long long* key;  // this wave's 64 lanes
-};
 
 // Orders the wave's LDS accesses around the pooled tests: LDS executes one
 // wave's instructions in order, so only the compiler needs holding back.
@@ -328,183 +327,123 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Visit one node: test its four child boxes, push its hit inner children
-// (far first) and descend into the nearest, and intersect the primitives of
-// its hit leaf children; the closest hit is the minimum of (t, primitive)
-// over the accepted primitives.  POOL: the lanes of a wave test their leaf
-// primitives as one pool: each lane posts its (primitive, lane) entries to
-// LDS, every lane taking part in this step tests entries of the pool against
-// the owner's ray, and a 64-bit LDS minimum returns each owner its closest
-// hit; every lane whose ray is in flight then calls it together (the pool
-// reads other lanes' registers).  Without POOL each lane tests its own
-// primitives.  Returns true when the ray is finished.
-template <bool ANY, bool POOL>
-__device__ __forceinline__ bool trace_step(const DevScene& s, TraceRay& r, TraceStack& st, const PrimPool& pool) {
-  // one 64-byte quantised node: origin + steps, 8-bit child bounds, counts, children
-  const uint4* q = reinterpret_cast<const uint4*>(s.qnodes) + 4 * size_t(r.node);
-  const uint4 hdr = q[0], bxy = q[1], bz = q[2];
-  const int4 ch = *reinterpret_cast<const int4*>(q + 3);
-  // A child plane at 8-bit offset q along x lies at origin + q * step; its ray
-  // parameter is q * (step / d) + (origin - o) / d.  step is a power of two,
-  // so the first factor is exact, and the near plane of each axis is chosen
-  // once per node by the direction's sign.
+// Leaf children of one node hit by a ray: their mask (slots) and where their
+// primitives are.
+struct LeafGroup {
+  uint32_t prim_base, ends0, ends1, hits;
+};
+
+// Bits [begin, end) of the node's primitives for every hit leaf slot.
+__device__ __forceinline__ uint32_t leaf_prims(const LeafGroup& g) {
+  const unsigned long long ends = (static_cast<unsigned long long>(g.ends1) << 32) | g.ends0;
+  const unsigned long long begins = ends << 8;
+  uint32_t pm = 0;
+  for (uint32_t h = g.hits; h; h &= h - 1u) {
+    const uint32_t sh = 8u * uint32_t(__ffs(int(h)) - 1);
+    const uint32_t b = uint32_t(begins >> sh) & 0xffu, c = (uint32_t(ends >> sh) & 0xffu) - b;
+    if (c) pm |= (0xffffffffu >> (32u - c)) << b;
+  }
+  return pm;
+}
+
+// Visit node r.node: test its eight child boxes, make the hit inner children
+// the current group and choose the node to visit next.  leaf: the hit leaf
+// children, for the caller to intersect.  Returns false when no node is left.
+//
+// Bound by instruction issue (the loads hide behind the other waves): a child
+// costs six v_fma_mix_f32 straight from the packed planes, two three-way and
+// two two-way min / max, one fused multiply-add of slack and one compare.
+//
+// FAR: byte offsets of nodes need 64 bits (a tree of 4 GiB or more).  Without
+// it a chunk's address is a scalar base and one 32-bit register.
+template <bool FAR>
+__device__ __forceinline__ bool trace_node(const DevScene& s, TraceRay& r, TraceStack& st, LeafGroup& leaf) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  const uint32_t sx = r.oct & 16u, sy = r.oct & 32u, sz = r.oct & 64u;
+  uint4 hdr, nx, fx, ny, fy, nz, fz, hb;
+  const auto load = [&](const char* nodes, auto off) {  // the chunks' bits are clear in off: | is +
+    const auto at = [&](auto k, int fixed) { return *reinterpret_cast<const uint4*>(nodes + k + fixed); };
+    hdr = at(off, 0x20);
+    nx = at(off | sx, 0), fx = at(off | (sx ^ 16u), 0);
+    ny = at(off | sy, 0x40), fy = at(off | (sy ^ 32u), 0x40);
+    nz = at(off | sz, 0x30), fz = at(off | (sz ^ 64u), 0x30);
+    hb = at(off, 0x50);
+  };
+  if constexpr (FAR)
+    load(reinterpret_cast<const char*>(s.wnodes), size_t(r.node) << 7);
+  else
+    load(reinterpret_cast<const char*>(s.wnodes), r.node << 7);
+  // A child plane at offset q along x lies at origin + q * step; its ray
+  // parameter is q * (step / d) + (origin - o) / d, the step a power of two,
+  // so the first factor is exact.
   const float ax = quant_step(hdr.w) * r.inv.x, ay = quant_step(hdr.w >> 8) * r.inv.y,
               az = quant_step(hdr.w >> 16) * r.inv.z;
   const float bx = (__uint_as_float(hdr.x) - r.o.x) * r.inv.x, by = (__uint_as_float(hdr.y) - r.o.y) * r.inv.y,
-              bz0 = (__uint_as_float(hdr.z) - r.o.z) * r.inv.z;
-  const uint32_t nearx = r.nx ? bxy.y : bxy.x, farx = r.nx ? bxy.x : bxy.y;
-  const uint32_t neary = r.ny ? bxy.w : bxy.z, fary = r.ny ? bxy.z : bxy.w;
-  const uint32_t nearz = r.nz ? bz.y : bz.x, farz = r.nz ? bz.x : bz.y;
-  const int cc[4] = {ch.x, ch.y, ch.z, ch.w};
-  uint32_t cnt[4];
-  float tn[4];
-  bool m[4];
+              bz = (__uint_as_float(hdr.z) - r.o.z) * r.inv.z;
+  uint32_t hits = 0;
+  const uint32_t wnx[4] = {nx.x, nx.y, nx.z, nx.w}, wny[4] = {ny.x, ny.y, ny.z, ny.w}, wnz[4] = {nz.x, nz.y, nz.z, nz.w};
+  const uint32_t wfx[4] = {fx.x, fx.y, fx.z, fx.w}, wfy[4] = {fy.x, fy.y, fy.z, fy.w}, wfz[4] = {fz.x, fz.y, fz.z, fz.w};
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int sh = 8 * i;
-    cnt[i] = (bz.z >> sh) & 0xffu;
-    const float tnx = fmaf(float((nearx >> sh) & 0xffu), ax, bx), tfx = fmaf(float((farx >> sh) & 0xffu), ax, bx);
-    const float tny = fmaf(float((neary >> sh) & 0xffu), ay, by), tfy = fmaf(float((fary >> sh) & 0xffu), ay, by);
-    const float tnz = fmaf(float((nearz >> sh) & 0xffu), az, bz0), tfz = fmaf(float((farz >> sh) & 0xffu), az, bz0);
-    float tnear = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, r.tmin));
-    float tfb = fminf(fminf(tfx, tfy), fminf(tfz, r.tfar));
-    // slack for the rounding of the slab arithmetic
-    tnear = fmaf(-fabsf(tnear), 4.8e-7f, tnear);
-    tfb = fmaf(fabsf(tfb), 4.8e-7f, tfb);
-    m[i] = cc[i] >= 0 && tnear <= tfb;
-    tn[i] = tnear;
-  }
-  // inner children in front of the current closest hit, sorted by a fixed
-  // network: the nearest is visited next, the others pushed far first.  A
-  // leaf hit below can only move tfar closer; entries then behind it are
-  // skipped when popped.  Any-hit rays end at their first hit, whatever its
-  // distance, so they take the children in node order (per 1080p
-  // large-mesh frame, shadow rays 33.2 -> 31.9 ms).
-  float d0 = kInf, d1 = kInf, d2 = kInf, d3 = kInf;
-  uint32_t n0 = 0, n1 = 0, n2 = 0, n3 = 0;
-  if (m[0] && cnt[0] == 0 && tn[0] <= r.tfar) { d0 = tn[0]; n0 = uint32_t(cc[0]); }
-  if (m[1] && cnt[1] == 0 && tn[1] <= r.tfar) { d1 = tn[1]; n1 = uint32_t(cc[1]); }
-  if (m[2] && cnt[2] == 0 && tn[2] <= r.tfar) { d2 = tn[2]; n2 = uint32_t(cc[2]); }
-  if (m[3] && cnt[3] == 0 && tn[3] <= r.tfar) { d3 = tn[3]; n3 = uint32_t(cc[3]); }
-  if constexpr (!ANY) {
-    cswap(d0, n0, d1, n1);
-    cswap(d2, n2, d3, n3);
-    cswap(d0, n0, d2, n2);
-    cswap(d1, n1, d3, n3);
-    cswap(d1, n1, d2, n2);
-  }
-  if (d3 != kInf) st.push(n3, d3);
-  if (d2 != kInf) st.push(n2, d2);
-  if (d1 != kInf) st.push(n1, d1);
-  // this lane's leaf primitives as one list (children in order)
-  const uint32_t l0 = (m[0] && cnt[0] > 0) ? cnt[0] : 0u, l1 = (m[1] && cnt[1] > 0) ? cnt[1] : 0u;
-  const uint32_t l2 = (m[2] && cnt[2] > 0) ? cnt[2] : 0u, l3 = (m[3] && cnt[3] > 0) ? cnt[3] : 0u;
-  const uint32_t e0 = l0, e1 = e0 + l1, e2 = e1 + l2, total = e2 + l3;
-  const uint32_t b0 = uint32_t(cc[0]), b1 = uint32_t(cc[1]) - e0, b2 = uint32_t(cc[2]) - e1, b3 = uint32_t(cc[3]) - e2;
-  bool leafHit = false;
-  if constexpr (!POOL) {
-    // one lane on its own: its primitives in order, the same (t, primitive) minimum
-    unsigned long long best = ~0ull;
-    for (uint32_t k = 0; k < total; k++) {
-      const uint32_t prim = k >= e2 ? b3 + k : k >= e1 ? b2 + k : k >= e0 ? b1 + k : b0 + k;
-      float tf = r.tfar;
-      if (isect_prim(s, prim, r.o, r.d, r.tmin, tf)) {
-        const unsigned long long key = (uint64_t(__float_as_uint(tf)) << 32) | prim;
-        if (key < best) best = key;
-        if (ANY) break;
-      }
-    }
-    if (best != ~0ull) {
-      r.tfar = __uint_as_float(uint32_t(best >> 32));
-      r.hitp = uint32_t(best);
-      r.hit = true;
-      leafHit = true;
-    }
-  } else {
-  const uint32_t lane = __lane_id();
-  const uint32_t pre =  // this lane's first pool index
-      total ? __hip_atomic_fetch_add(pool.ctr, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) : 0u;
-  wave_lds_fence();
-  const uint32_t sum = *pool.ctr;  // wave-uniform
-  if (sum > 0) {
-    // Post the entries that fit the pool; a lane whose entries run past it
-    // (the wave has more than kPoolSize, which is rare) tests those itself.
-    const uint32_t cap = s.pool_cap;
-    const uint32_t fit = pre < cap ? min(total, cap - pre) : 0u;
-    unsigned long long best = ~0ull;
-    for (uint32_t k = 0; k < total; k++) {
-      const uint32_t prim = k >= e2 ? b3 + k : k >= e1 ? b2 + k : k >= e0 ? b1 + k : b0 + k;
-      if (k < fit) {
-        pool.prim[pre + k] = prim;
-        pool.owner[pre + k] = lane;
-      } else {
-        float tf = r.tfar;
-        if (isect_prim(s, prim, r.o, r.d, r.tmin, tf)) {
-          const unsigned long long key = (uint64_t(__float_as_uint(tf)) << 32) | prim;
-          if (key < best) best = key;  // unsigned order: (t, primitive)
-        }
-      }
-    }
-    if (total) pool.key[lane] = best;
-    wave_lds_fence();
-    const unsigned long long act = __ballot(true);
-    const uint32_t nact = (uint32_t)__popcll(act);
-    const uint32_t rank = (uint32_t)__popcll(act & ((1ull << lane) - 1ull));
-    const uint32_t cnt_r = min(cap, sum);
-    for (uint32_t jb = 0; jb < cnt_r; jb += nact) {
-      const uint32_t j = jb + rank;
-      const bool valid = j < cnt_r;
-      const uint32_t own = valid ? pool.owner[j] : lane;
-      // the owner's ray, read from its registers (all lanes of the step take part)
-      const f3 o = mk(__shfl(r.o.x, own), __shfl(r.o.y, own), __shfl(r.o.z, own));
-      const f3 d = mk(__shfl(r.d.x, own), __shfl(r.d.y, own), __shfl(r.d.z, own));
-      const float tmin = __shfl(r.tmin, own);
-      float tfar = __shfl(r.tfar, own);
-      if (valid) {
-        const uint32_t prim = pool.prim[j];
-        if (isect_prim(s, prim, o, d, tmin, tfar))
-          __hip_atomic_fetch_min(&pool.key[own], (uint64_t(__float_as_uint(tfar)) << 32) | prim, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_WAVEFRONT);
-      }
-    }
-    wave_lds_fence();
-    if (total) {
-      const unsigned long long k = pool.key[lane];
-      if (k != ~0ull) {
-        r.tfar = __uint_as_float(uint32_t(k >> 32));
-        r.hitp = uint32_t(k);
-        r.hit = true;
-        leafHit = true;
-      }
-    }
-    if (rank == 0) *pool.ctr = 0u;  // ready for the next step
-    wave_lds_fence();
-  }
-  }
-  if (ANY && leafHit) return true;
-  if (d0 != kInf && d0 <= r.tfar) {
-    r.node = n0;
-    return false;
-  }
-  // pop, skipping subtrees entered beyond the closest hit found since the push
-  while (st.sp > 0) {
-    uint32_t n;
-    float d;
-    st.pop(n, d);
-    if (d <= r.tfar) {
-      r.node = n;
-      return false;
+  for (int w = 0; w < 4; w++) {
+    const h2 hnx = __builtin_bit_cast(h2, wnx[w]), hny = __builtin_bit_cast(h2, wny[w]), hnz = __builtin_bit_cast(h2, wnz[w]);
+    const h2 hfx = __builtin_bit_cast(h2, wfx[w]), hfy = __builtin_bit_cast(h2, wfy[w]), hfz = __builtin_bit_cast(h2, wfz[w]);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const float tnx = fmaf(float(hnx[c]), ax, bx), tfx = fmaf(float(hfx[c]), ax, bx);
+      const float tny = fmaf(float(hny[c]), ay, by), tfy = fmaf(float(hfy[c]), ay, by);
+      const float tnz = fmaf(float(hnz[c]), az, bz), tfz = fmaf(float(hfz[c]), az, bz);
+      const float tn = fmaxf(fmaxf(fmaxf(tnx, tny), tnz), r.tmin);
+      float tf = fminf(fminf(fminf(tfx, tfy), tfz), r.tfar);
+      tf = fmaf(fabsf(tf), 9.6e-7f, tf);  // slack for the rounding of the slab arithmetic on both sides
+      hits |= tn <= tf ? 1u << (2 * w + c) : 0u;
     }
   }
+  const uint32_t imask = hdr.w >> 24;
+  leaf.hits = hits & ~imask;
+  leaf.prim_base = hb.y;
+  leaf.ends0 = hb.z;
+  leaf.ends1 = hb.w;
+  const uint32_t o = r.oct >> 4;
+  uint32_t g = hits & imask;
+  if (g) {
+    if (r.gmask & 0xffu) st.push(r.gbase, r.gmask);
+    // bit slot -> bit slot ^ o, so the lowest set bit is the child to visit first
+    g = ((g & 0xaau) >> (o & 1u)) | ((g & 0x55u) << (o & 1u));
+    g = ((g & 0xccu) >> (o & 2u)) | ((g & 0x33u) << (o & 2u));
+    g = ((g & 0xf0u) >> (o & 4u)) | ((g & 0x0fu) << (o & 4u));
+    r.gbase = hb.x;
+    r.gmask = g | imask << 8;
+  } else if (!(r.gmask & 0xffu)) {
+    if (st.sp == 0) return false;
+    st.pop(r.gbase, r.gmask);
+  }
+  const uint32_t slot = uint32_t(__ffs(int(r.gmask)) - 1) ^ o;
+  r.gmask &= r.gmask - 1u;
+  r.node = r.gbase + uint32_t(__popc(r.gmask & (((1u << slot) - 1u) << 8)));
   return true;
 }
 
-// Stream traversal for kernels that own a batch of rays.  A lane whose ray
-// finishes is refilled from the batch while the other lanes of its wave keep
-// traversing.  Each wave takes rays from a private chunk of kChunk
-// consecutive items and grabs the next chunk with one atomic on `fetch`, so
-// the shared counter sees one atomic per kChunk rays (with fetch == nullptr
-// each wave takes the 64 items at its own position once).
+// Sum of v over the lanes below this one (all 64 lanes active).
+__device__ __forceinline__ uint32_t wave_exclusive_sum(uint32_t v) {
+  int x = int(v);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return uint32_t(x) - v;
+}
+
+// Stream traversal for kernels that own a batch of rays.  Rays end at
+// different steps, so a lane that has none takes the next of the batch while
+// the others continue; and about one lane-step in nine reaches leaves, so a
+// wave queues the leaf groups its lanes find and intersects their primitives
+// together, 64 at a time, once enough have gathered (flush_leaves).
+//
+// Rays: with fetch, each wave takes chunks of consecutive items, the first by
+// its position and later ones with one atomic each; with fetch == nullptr,
+// wave w of the grid owns the items [w * per_wave, (w + 1) * per_wave).
 // Job: bool load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax, uint32_t& tag)
 //      void finish(uint32_t i, uint32_t tag, const TraceRay& r)
 //      static constexpr bool kTagIsIndex; with it the tag is the item index
@@ -518,80 +457,105 @@ __device__ __forceinline__ bool trace_step(const DevScene& s, TraceRay& r, Trace
 //      void resume(uint32_t tag, TraceRay& r, TraceStack& st)   (after trace_begin)
 //      bool suspend(uint32_t tag, const TraceRay& r, const TraceStack& st)
 // Launch with kTraceBlock threads per block; every lane must call this.
-template <bool ANY, class Job>
-__device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint32_t* fetch, Job& job) {
-  __shared__ uint32_t lds_node[kLdsStack * kTraceBlock];
-  __shared__ float lds_dist[kLdsStack * kTraceBlock];
-  __shared__ uint32_t pool_ctr[kTraceBlock / 64], pool_prim[kTraceBlock / 64][kPoolSize],
-      pool_owner[kTraceBlock / 64][kPoolSize];
-  __shared__ unsigned long long pool_key[kTraceBlock];
-  constexpr int kRefillBelow = 48;  // refill once fewer lanes than this are busy
-  constexpr uint32_t kChunk = 128;
+constexpr uint32_t kGroupFlush = 24;                // queued leaf groups at which a wave tests them
+constexpr uint32_t kGroupQueue = kGroupFlush + 64;  // a step adds at most one group per lane
+constexpr uint32_t kPoolSize = kTracePool;
+// Waves that a launch's rays are spread over before a wave fills all its lanes
+// (two per SIMD: 1024 to 4096 measured alike, without it a 64x48 render's
+// traversal took 8 % longer), fewest lanes of a wave, and the largest chunk.
+constexpr uint32_t kSpreadWaves = 2048, kMinLanes = 8, kMaxChunk = 256;
+
+template <bool ANY, bool FAR, class Job>
+__device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint32_t* fetch, uint32_t per_wave, Job& job) {
+  __shared__ unsigned long long lds_ring[kLdsStack * kTraceBlock];
+  __shared__ u32x4 lds_group[kTraceBlock / 64][kGroupQueue];
+  __shared__ u32x2 lds_pool[kTraceBlock / 64][kPoolSize];
+  __shared__ unsigned long long lds_key[kTraceBlock];
   const uint32_t lane = __lane_id();
   const unsigned long long below = (1ull << lane) - 1ull;
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  lds_u4* const group = (lds_u4*)lds_group[wv];
+  lds_u2* const pool = (lds_u2*)lds_pool[wv];
+  lds_u64* const key = (lds_u64*)&lds_key[wv * 64];
   TraceOverflow ov;
   TraceStack st;
-  st.node = (lds_u32*)(lds_node + threadIdx.x);
-  st.dist = (lds_f32*)(lds_dist + threadIdx.x);
-  st.ov_node = ov.node;
-  st.ov_dist = ov.dist;
-  const uint32_t wv = threadIdx.x >> 6;
-  const PrimPool pool{(lds_u32*)&pool_ctr[wv], (lds_u32*)pool_prim[wv], (lds_u32*)pool_owner[wv],
-                      (__attribute__((address_space(3))) unsigned long long*)&pool_key[wv * 64]};
-  if (lane == 0) *pool.ctr = 0u;
-  wave_lds_fence();
+  st.ring = (lds_u64*)(lds_ring + threadIdx.x);
+  st.ov = ov.e;
   TraceRay r;
-  bool active = false, done = false, exhausted = false;  // done: a finished ray not yet written out
+  // A lane's ray is being traversed (active), waits for queued leaf groups of
+  // its own with no node left (pend only), or has ended (have only).
+  bool have = false, active = false, pend = false;
   uint32_t idx = 0, tag = 0, visits = 0;
+  uint32_t queued = 0;            // leaf groups queued by the wave (wave-uniform)
   uint32_t cbase = 0, cleft = 0;  // the wave's chunk (wave-uniform)
+  bool exhausted = false;
+  // With few rays a wave fills only some of its lanes, so that they spread over
+  // the chip: a wave's step takes the longer the more lanes it has (more of
+  // them reach leaves), and a launch cannot end before its slowest wave.
+  // With fetch, a wave's first chunk is its own by position and only later
+  // ones cost an atomic: the counter takes about 11 ns per atomic, and one per
+  // wave made an empty launch of 8192 waves last 95 us.
+  const uint32_t wave = blockIdx.x * (kTraceBlock / 64) + wv, waves = gridDim.x * (kTraceBlock / 64);
+  uint32_t lanes, chunk;
+  if (!fetch) {
+    chunk = per_wave;
+    lanes = min(64u, per_wave);
+  } else {
+    lanes = min(64u, max(kMinLanes, (n + kSpreadWaves - 1) / kSpreadWaves));
+    chunk = lanes < 64 ? lanes : min(max(n / waves / 4u, 64u), kMaxChunk);
+  }
+  {
+    const unsigned long long b = static_cast<unsigned long long>(wave) * chunk;
+    cbase = uint32_t(b);
+    cleft = b < n ? min(chunk, uint32_t(n - b)) : 0u;
+    exhausted = !fetch || static_cast<unsigned long long>(waves) * chunk >= n;
+  }
+  const unsigned long long usable = ~0ull >> (64 - lanes);
+  const uint32_t refill = lanes * 3 / 4;                    // refill once fewer lanes than this have a ray in flight
+  const uint32_t flush = min(kGroupFlush, lanes * 3 / 8);  // queued leaf groups at which the wave tests them
   for (;;) {
     // Finished closest-hit rays are written out here, together: a wave's 64
     // rays end a few at a time, and recomputing and storing the hit in the
     // step in which its ray ended ran that code with about four lanes active
     // in nearly every step (1080p large-mesh frame 145.6 -> 138.0 ms).  An
     // any-hit ray has one byte or nothing to write and does so when it ends.
-    if (!ANY && done) {
+    if (!ANY && have && !active && !pend) {
       trace_finish(s, r);
       job.finish(Job::kTagIsIndex ? tag : idx, tag, r);
-      done = false;
+      have = false;
     }
     if (!exhausted || cleft > 0) {
-      unsigned long long need = __ballot(!active);
+      const unsigned long long need = __ballot(!have) & usable;
       if (need) {
         const uint32_t want = (uint32_t)__popcll(need);
         const uint32_t rank = (uint32_t)__popcll(need & below);
         uint32_t i = 0xffffffffu;
-        if (fetch) {
-          uint32_t nbase = 0, nleft = 0;
-          if (cleft < want && !exhausted) {
-            uint32_t b = 0;
-            if (lane == 0) b = atomicAdd(fetch, kChunk);
-            b = __shfl(b, 0);
-            if (b >= n) {
-              exhausted = true;
-            } else {
-              nbase = b;
-              nleft = min(kChunk, n - b);
-              if (b + kChunk >= n) exhausted = true;
-            }
+        uint32_t nbase = 0, nleft = 0;
+        if (cleft < want && !exhausted) {
+          uint32_t b = 0;
+          if (lane == 0) b = atomicAdd(fetch, chunk);
+          b = __builtin_amdgcn_readfirstlane(b) + waves * chunk;  // scalar, as are the loop's exits
+          if (b >= n) {
+            exhausted = true;
+          } else {
+            nbase = b;
+            nleft = min(chunk, n - b);
+            if (n - b <= chunk) exhausted = true;
           }
-          if (rank < cleft)
-            i = cbase + rank;
-          else if (rank - cleft < nleft)
-            i = nbase + (rank - cleft);
-          const uint32_t fromOld = min(want, cleft);
-          cbase += fromOld;
-          cleft -= fromOld;
-          if (nleft) {
-            const uint32_t fromNew = min(want - fromOld, nleft);
-            cbase = nbase + fromNew;
-            cleft = nleft - fromNew;
-          }
-        } else {
-          i = blockIdx.x * kTraceBlock + (threadIdx.x & ~63u) + lane;
-          exhausted = true;
         }
-        if (!active && i < n) {
+        if (rank < cleft)
+          i = cbase + rank;
+        else if (rank - cleft < nleft)
+          i = nbase + (rank - cleft);
+        const uint32_t fromOld = min(want, cleft);
+        cbase += fromOld;
+        cleft -= fromOld;
+        if (nleft) {
+          const uint32_t fromNew = min(want - fromOld, nleft);
+          cbase = nbase + fromNew;
+          cleft = nleft - fromNew;
+        }
+        if ((need >> lane & 1ull) && i < n) {
           f3 o, d;
           float tmin, tmax;
           if (job.load(i, o, d, tmin, tmax, tag)) {
@@ -599,33 +563,99 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
             trace_begin(r, st, o, d, tmin, tmax);
             if constexpr (Job::kSuspend) job.resume(tag, r, st);
             visits = 0;
-            active = true;
+            have = active = true;
           }
         }
       }
     }
-    if (__ballot(active) == 0ull) {
+    if (__ballot(have) == 0ull) {
       if (exhausted && cleft == 0) break;  // every finished ray was written out above
       continue;
     }
-    for (int k = 0; k < 256; k++) {
-      if (active) {
-        if (trace_step<ANY, true>(s, r, st, pool)) {
-          if (ANY)
-            job.finish(Job::kTagIsIndex ? tag : idx, tag, r);
-          else
-            done = true;
-          active = false;
-        } else if constexpr (Job::kSuspend) {
-          if (++visits >= job.budget) {
-            if (job.suspend(tag, r, st)) active = false;
-            visits = 0;
-          }
+    for (;;) {
+      LeafGroup leaf;
+      leaf.hits = 0;
+      if (active) active = trace_node<FAR>(s, r, st, leaf);
+      const unsigned long long found = __ballot(leaf.hits != 0);
+      if (found) {
+        if (leaf.hits) {
+          const uint32_t k = queued + (uint32_t)__popcll(found & below);
+          group[k] = u32x4{leaf.prim_base, leaf.ends0, leaf.ends1, leaf.hits | lane << 8};
+          pend = true;
+        }
+        queued += (uint32_t)__popcll(found);
+      }
+      if constexpr (Job::kSuspend) {
+        if (active && ++visits >= job.budget && !pend) {
+          if (job.suspend(tag, r, st)) have = active = false;
+          visits = 0;
         }
       }
-      unsigned long long busy = __ballot(active);
-      if (busy == 0ull) break;
-      if ((!exhausted || cleft > 0) && __popcll(busy) < kRefillBelow) break;
+      uint32_t busy = (uint32_t)__popcll(__ballot(active));
+      const uint32_t waiting = (uint32_t)__popcll(__ballot(pend && !active));
+      // Test the queued primitives when a wave's worth has gathered, or when
+      // the lanes that can do nothing else outnumber a third of the others.
+      if (queued >= flush || 3 * waiting > busy) {
+        key[lane] = ~0ull;
+        wave_lds_fence();
+        for (uint32_t g0 = 0; g0 < queued; g0 += 64) {
+          uint32_t pm = 0, base = 0, owner = 0;
+          if (g0 + lane < queued) {
+            const u32x4 e = group[g0 + lane];
+            const LeafGroup lg{e.x, e.y, e.z, e.w & 0xffu};
+            pm = leaf_prims(lg);
+            base = e.x;
+            owner = e.w >> 8;
+          }
+          while (__ballot(pm != 0)) {
+            const uint32_t t = (uint32_t)__popc(pm);
+            const uint32_t pre = wave_exclusive_sum(t);
+            const uint32_t total = __builtin_amdgcn_readlane(pre + t, 63);
+            const uint32_t cap = s.pool_cap;
+            const uint32_t fit = min(t, cap - min(pre, cap));  // entries beyond the pool wait for the next round
+            for (uint32_t k = 0; k < fit; k++) {
+              pool[pre + k] = u32x2{base + uint32_t(__ffs(int(pm)) - 1), owner};
+              pm &= pm - 1u;
+            }
+            wave_lds_fence();
+            const bool valid = lane < min(total, cap);
+            u32x2 e = {0u, lane};
+            if (valid) e = pool[lane];
+            // the owner's ray, read from its registers
+            const f3 o = mk(__shfl(r.o.x, e.y), __shfl(r.o.y, e.y), __shfl(r.o.z, e.y));
+            const f3 d = mk(__shfl(r.d.x, e.y), __shfl(r.d.y, e.y), __shfl(r.d.z, e.y));
+            const float tmin = __shfl(r.tmin, e.y);
+            float tfar = __shfl(r.tfar, e.y);
+            if (valid && isect_prim(s, e.x, o, d, tmin, tfar)) {
+              if (ANY)
+                key[e.y] = 0;
+              else
+                __hip_atomic_fetch_min(&key[e.y], hit_key(tfar, e.x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            }
+            wave_lds_fence();
+          }
+        }
+        queued = 0;
+        pend = false;
+        const unsigned long long k = key[lane];
+        if (ANY) {
+          if (have && k == 0) {
+            r.hitp = 0;
+            active = false;
+          }
+        } else if (have && k < r.key()) {
+          r.tfar = key_t(k);
+          r.hitp = uint32_t(k);
+        }
+        wave_lds_fence();
+        busy = (uint32_t)__popcll(__ballot(active));
+      }
+      if (ANY && have && !active && !pend) {
+        job.finish(Job::kTagIsIndex ? tag : idx, tag, r);
+        have = false;
+      }
+      if (busy == 0 && queued == 0) break;
+      if ((!exhausted || cleft > 0) && (uint32_t)__popcll(__ballot(active || pend)) < refill) break;
     }
   }
 }
@@ -634,23 +664,37 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
 // per lane (launched with at most kTraceBlock threads per block).
 template <bool ANY>
 __device__ __forceinline__ bool trace(const DevScene& s, f3 o, f3 d, float tmin, float tmax, Hit& h) {
-  __shared__ uint32_t lds_node1[kLdsStack * kTraceBlock];
-  __shared__ float lds_dist1[kLdsStack * kTraceBlock];
+  __shared__ unsigned long long lds_ring1[kLdsStack * kTraceBlock];
 
   TraceRay r;
   TraceOverflow ov;
   TraceStack st;
-  st.node = (lds_u32*)(lds_node1 + threadIdx.x);
-  st.dist = (lds_f32*)(lds_dist1 + threadIdx.x);
-  st.ov_node = ov.node;
-  st.ov_dist = ov.dist;
+  st.ring = (lds_u64*)(lds_ring1 + threadIdx.x);
+  st.ov = ov.e;
   trace_begin(r, st, o, d, tmin, tmax);
-  // lanes loop independently here, so primitives are tested per lane
-  while (!trace_step<ANY, false>(s, r, st, PrimPool{})) {
+  // lanes loop independently here, so each tests its own primitives
+  for (bool more = true; more;) {
+    LeafGroup leaf;
+    more = trace_node<true>(s, r, st, leaf);
+    if (leaf.hits) {
+      for (uint32_t pm = leaf_prims(leaf); pm; pm &= pm - 1u) {
+        const uint32_t p = leaf.prim_base + uint32_t(__ffs(int(pm)) - 1);
+        float tf = r.tfar;
+        if (!isect_prim(s, p, r.o, r.d, r.tmin, tf)) continue;
+        if (hit_key(tf, p) < r.key()) {
+          r.tfar = tf;
+          r.hitp = p;
+        }
+        if (ANY) {
+          more = false;
+          break;
+        }
+      }
+    }
   }
   if (!ANY) trace_finish(s, r);
   h = r.h;
-  return r.hit;
+  return r.hit();
 }
 
 }  // namespace rad

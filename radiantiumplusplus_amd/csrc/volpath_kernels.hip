@@ -400,7 +400,12 @@ __global__ void __launch_bounds__(kTraceBlock) k_vol_shadow(Wavefront w, DevScen
   const unsigned long long below = (1ull << lane) - 1ull;
   VolShadowRay r;
   bool active = false, exhausted = false;
-  uint32_t cbase = 0, cleft = 0, steps = 0, guard = 0;
+  // the wave's first chunk is its own by position: a launch with little work
+  // costs no atomics (about 11 ns each on one counter)
+  const uint32_t wave = blockIdx.x * (kTraceBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
+                 waves = gridDim.x * (kTraceBlock / 64);
+  uint32_t cbase = wave * kChunk, cleft = cbase < n ? min(kChunk, n - cbase) : 0u, steps = 0, guard = 0;
+  exhausted = static_cast<unsigned long long>(waves) * kChunk >= n;
   for (;;) {
     const unsigned long long need = __ballot(!active);
     if (need && (!exhausted || cleft > 0)) {
@@ -410,7 +415,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_vol_shadow(Wavefront w, DevScen
       if (cleft < want && !exhausted) {
         uint32_t b = 0;
         if (lane == 0) b = atomicAdd(fetch, kChunk);
-        b = __shfl(b, 0);
+        b = __builtin_amdgcn_readfirstlane(b) + waves * kChunk;
         if (b >= n) {
           exhausted = true;
         } else {
