@@ -17,16 +17,36 @@ struct DeviceBvhStats {
   double build_ms = 0;
 };
 
-// bounds: 6 floats per primitive (lo.xyz, hi.xyz); records: 3 float4 per
-// primitive (host memory).  Writes the nodes and the primitive records in
-// leaf order to device buffers.
-void BuildBvh4Device(const float* bounds, const float4* records, uint32_t n, int maxLeaf, hipStream_t st,
-                     DeviceBuffer& nodesOut, DeviceBuffer& primsOut, DeviceBvhStats& stats);
+// Consecutive primitives [begin, next segment's begin) of one shape, in shape
+// order: the triangles of a mesh from tri_offset on, or the one primitive of
+// another shape (other: its index in PrimSource::other_rec; 0xffffffff for a
+// mesh).
+struct PrimSegment {
+  uint32_t begin, geom, tri_offset, other;
+};
 
-// The traversal's nodes from a tree of m BvhNode4 over n primitive records
-// (device buffers): writes them to `out` and returns their number, puts the
-// primitive records in the order of their leaves and renumbers the BvhNode4
-// leaves to match; throws if a child box cannot be bounded.
-uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, DeviceBuffer& prims, uint32_t n, hipStream_t st, DeviceBuffer& out);
+// Where a scene's primitives come from: triangles are in device memory already
+// (DevScene::tris), the few others come from the host (three float4 and six
+// floats of bounds each).
+struct PrimSource {
+  std::vector<PrimSegment> segs;
+  std::vector<float4> other_rec;
+  std::vector<float> other_box;
+  const float4* d_tris = nullptr;
+  uint32_t count = 0;
+};
+
+// Writes the nodes and the primitive records in leaf order to device buffers;
+// work: scratch memory, left allocated for BuildWideNodes.
+void BuildBvh4Device(const PrimSource& src, int maxLeaf, hipStream_t st, DeviceBuffer& nodesOut, DeviceBuffer& primsOut,
+                     DeviceBuffer& work, DeviceBvhStats& stats);
+
+// The traversal's nodes from a tree of m BvhNode4, with leaves of at most
+// maxLeaf, over n primitive records (device buffers): writes them to `out` and
+// returns their number, puts the primitive records in the order of their leaves
+// and renumbers the BvhNode4 leaves to match; throws if a child box cannot be
+// bounded.  work: scratch memory, reused when large enough.
+uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, uint32_t maxLeaf, DeviceBuffer& prims, uint32_t n, hipStream_t st,
+                        DeviceBuffer& work, DeviceBuffer& out);
 
 }  // namespace rad

@@ -51,13 +51,32 @@ __device__ __forceinline__ void atomic_max_f(float* a, float v) {
     atomicMin(reinterpret_cast<unsigned int*>(a), __float_as_uint(v));
 }
 
-__device__ __forceinline__ float wave_min(float v) {
-  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o));
-  return v;
+// Minimum / maximum over the wave, in every lane (all 64 lanes active): data
+// parallel moves within and across rows instead of LDS permutes.
+template <bool MAX>
+__device__ __forceinline__ float wave_extreme(float v) {
+  const auto step = [](float x, float y) { return MAX ? fmaxf(x, y) : fminf(x, y); };
+#define RAD_DPP(ctrl, rows) \
+  v = step(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), ctrl, rows, 0xf, false)))
+  RAD_DPP(0x111, 0xf);  // row_shr:1
+  RAD_DPP(0x112, 0xf);
+  RAD_DPP(0x114, 0xf);
+  RAD_DPP(0x118, 0xf);
+  RAD_DPP(0x142, 0xa);  // row_bcast:15
+  RAD_DPP(0x143, 0xc);  // row_bcast:31
+#undef RAD_DPP
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
-__device__ __forceinline__ float wave_max(float v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  return v;
+__device__ __forceinline__ float wave_min(float v) { return wave_extreme<false>(v); }
+__device__ __forceinline__ float wave_max(float v) { return wave_extreme<true>(v); }
+
+// Unsigned integers in the order of the floats, for LDS minima and maxima.
+__device__ __forceinline__ uint32_t ordered_bits(float v) {
+  const uint32_t u = __float_as_uint(v);
+  return u ^ (uint32_t(int32_t(u) >> 31) | 0x80000000u);
+}
+__device__ __forceinline__ float from_ordered(uint32_t u) {
+  return __uint_as_float(u ^ (uint32_t(int32_t(~u) >> 31) | 0x80000000u));
 }
 
 __device__ __forceinline__ float half_area(const float lo[3], const float hi[3]) {
@@ -67,19 +86,57 @@ __device__ __forceinline__ float half_area(const float lo[3], const float hi[3])
 }
 
 // ---------------------------------------------------------------- ordering
+// A fixed grid, so that the six atomics per wave stay few: with one wave per
+// 64 primitives they took 2.8 ms on 2.6 M primitives (about 11 ns each).
 __global__ void k_centroid_bounds(const float* b, uint32_t n, float* cb) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  float c[3], lo[3], hi[3];
-  for (int a = 0; a < 3; a++) {
-    c[a] = i < n ? 0.5f * (b[6 * size_t(i) + a] + b[6 * size_t(i) + 3 + a]) : 0.f;
-    lo[a] = wave_min(i < n ? c[a] : kInf);
-    hi[a] = wave_max(i < n ? c[a] : -kInf);
-  }
+  float lo[3] = {kInf, kInf, kInf}, hi[3] = {-kInf, -kInf, -kInf};
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    for (int a = 0; a < 3; a++) {
+      const float c = 0.5f * (b[6 * size_t(i) + a] + b[6 * size_t(i) + 3 + a]);
+      lo[a] = fminf(lo[a], c);
+      hi[a] = fmaxf(hi[a], c);
+    }
+  for (int a = 0; a < 3; a++) lo[a] = wave_min(lo[a]), hi[a] = wave_max(hi[a]);
   if (__lane_id() == 0)
     for (int a = 0; a < 3; a++) {
       atomic_min_f(&cb[a], lo[a]);
       atomic_max_f(&cb[3 + a], hi[a]);
     }
+}
+
+// Primitive records and boxes: triangles from the scene's per-triangle
+// records, other shapes (one primitive each) as the host made them.
+__global__ void k_primitives(const PrimSegment* segs, uint32_t nSegs, const float4* tris, const float4* otherRec,
+                             const float* otherBox, uint32_t n, float4* rec, float* box) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  uint32_t l = 0, r = nSegs;  // the last segment that begins at or before i
+  while (r - l > 1) {
+    const uint32_t m = (l + r) / 2;
+    if (segs[m].begin <= i)
+      l = m;
+    else
+      r = m;
+  }
+  const PrimSegment sg = segs[l];
+  float4* o = rec + 3 * size_t(i);
+  float* q = box + 6 * size_t(i);
+  if (sg.other != kNone) {
+    for (int k = 0; k < 3; k++) o[k] = otherRec[3 * size_t(sg.other) + k];
+    for (int k = 0; k < 6; k++) q[k] = otherBox[6 * size_t(sg.other) + k];
+    return;
+  }
+  const uint32_t t = i - sg.begin;
+  const float4* s = tris + 6 * (size_t(sg.tri_offset) + t);
+  const float4 a = s[0], b = s[1], c = s[2];
+  const float v[3][3] = {{a.x, a.y, a.z}, {a.w, b.x, b.y}, {b.z, b.w, c.x}};
+  o[0] = make_float4(v[0][0], v[0][1], v[0][2], __uint_as_float(sg.geom));
+  o[1] = make_float4(v[1][0], v[1][1], v[1][2], __uint_as_float(t));
+  o[2] = make_float4(v[2][0], v[2][1], v[2][2], __uint_as_float(PRIM_TRI));
+  for (int k = 0; k < 3; k++) {
+    q[k] = fminf(fminf(v[0][k], v[1][k]), v[2][k]);
+    q[3 + k] = fmaxf(fmaxf(v[0][k], v[1][k]), v[2][k]);
+  }
 }
 
 __device__ __forceinline__ uint64_t spread21(uint32_t v) {
@@ -133,7 +190,8 @@ struct Task {
 };
 
 struct SmallTask {
-  uint32_t node, begin, end, pad;
+  uint32_t node, begin, end;
+  uint32_t nodes;  // 2 * (end - begin - 1) nodes reserved for the subtree
 };
 
 struct Bin {
@@ -179,133 +237,236 @@ __global__ void k_bins_clear(Bin* bins, uint32_t m) {
   bins[i] = e;
 }
 
-// Adds this lane's box to bins[slot]; lanes of the wave that share a slot
-// are combined first (one set of atomics per distinct slot).
-__device__ __forceinline__ void bin_add(Bin* bins, uint32_t slot, float4 lo, float4 hi) {
-  uint64_t pending = __ballot(slot != kNone);
-  while (pending) {
-    const int leader = __ffsll((unsigned long long)pending) - 1;
-    const uint32_t target = __shfl(slot, leader);
-    const bool mine = slot == target;
-    const uint64_t group = __ballot(mine);
-    pending &= ~group;
-    float l0 = wave_min(mine ? lo.x : kInf), l1 = wave_min(mine ? lo.y : kInf), l2 = wave_min(mine ? lo.z : kInf);
-    float h0 = wave_max(mine ? hi.x : -kInf), h1 = wave_max(mine ? hi.y : -kInf), h2 = wave_max(mine ? hi.z : -kInf);
-    if (__lane_id() == leader) {
-      Bin* e = &bins[target];
-      atomic_min_f(&e->lo[0], l0);
-      atomic_min_f(&e->lo[1], l1);
-      atomic_min_f(&e->lo[2], l2);
-      atomic_max_f(&e->hi[0], h0);
-      atomic_max_f(&e->hi[1], h1);
-      atomic_max_f(&e->hi[2], h2);
-      atomicAdd(&e->count, uint32_t(__popcll(group)));
+// The level passes work on chunks of kLevelChunk consecutive primitives per
+// block.  A large task's primitives are consecutive and more than kSmall, so a
+// chunk meets at most kLevelSlots of them: sums go to LDS by (task of the
+// chunk, bin) and then to memory once per chunk, instead of once per wave and
+// bin (2.6 M primitives, 21 levels: binning 12.7 ms, child centroid bounds 9.4
+// ms, most of it waiting on atomics to a few addresses).
+constexpr int kLevelThreads = 256, kLevelItems = 4;
+constexpr uint32_t kLevelChunk = kLevelThreads * kLevelItems;
+constexpr uint32_t kLevelSlots = kLevelChunk / (kSmall + 1) + 2;
+
+// t[e]: task of item blockIdx.x * kLevelChunk + e * kLevelThreads + threadIdx.x
+// (kNone: none), slot[e]: its number among the chunk's tasks, sTask: the
+// chunk's tasks.  Returns how many there are.
+__device__ __forceinline__ uint32_t chunk_slots(uint32_t n, const uint32_t* owner, uint32_t t[kLevelItems],
+                                                uint32_t slot[kLevelItems], uint32_t* sTask, BuildCtr* ctr) {
+  __shared__ uint32_t sHeads[kLevelItems * kLevelThreads / 64];
+  const uint32_t base = blockIdx.x * kLevelChunk, wave = threadIdx.x >> 6, lane = __lane_id();
+  uint64_t heads[kLevelItems];
+#pragma unroll
+  for (int e = 0; e < kLevelItems; e++) {
+    const uint32_t i = base + e * kLevelThreads + threadIdx.x;
+    t[e] = i < n ? owner[i] : kNone;
+    const bool head = t[e] != kNone && (i == base || owner[i - 1] != t[e]);
+    heads[e] = __ballot(head);
+    if (lane == 0) sHeads[e * (kLevelThreads / 64) + wave] = uint32_t(__popcll(heads[e]));
+  }
+  __syncthreads();
+  uint32_t total = 0;
+#pragma unroll
+  for (int e = 0; e < kLevelItems; e++)
+    for (uint32_t v = 0; v < kLevelThreads / 64; v++) {
+      if (v == wave) slot[e] = total + uint32_t(__popcll(heads[e] & (~0ull >> (63 - lane)))) - 1u;
+      total += sHeads[e * (kLevelThreads / 64) + v];
+    }
+#pragma unroll
+  for (int e = 0; e < kLevelItems; e++) {
+    if (t[e] == kNone) continue;
+    if (slot[e] >= kLevelSlots) {  // not a partition into ranges of more than kSmall: report, leave it out
+      atomicOr(&ctr->error, 16u);
+      t[e] = kNone;
+    } else if (heads[e] >> lane & 1ull) {
+      sTask[slot[e]] = t[e];
     }
   }
+  __syncthreads();
+  return min(total, kLevelSlots);
+}
+
+// LDS sums of one key: box (6 ordered words) and, with COUNT, a count.
+template <bool COUNT>
+__device__ __forceinline__ void lds_add(uint32_t* s, const float lo[3], const float hi[3], uint32_t count) {
+  for (int a = 0; a < 3; a++) {
+    atomicMin(&s[a], ordered_bits(lo[a]));
+    atomicMax(&s[3 + a], ordered_bits(hi[a]));
+  }
+  if (COUNT) atomicAdd(&s[6], count);
+}
+// Adds this lane's box to sums[key] (kNone: nothing).  The two commonest cases,
+// a wave with one or two keys, are combined in registers first; the lanes left
+// over then meet in few places and add theirs one by one.
+template <bool COUNT>
+__device__ __forceinline__ void wave_add(uint32_t* sums, uint32_t key, const float lo[3], const float hi[3]) {
+  constexpr uint32_t W = COUNT ? 7 : 6;
+  uint64_t pending = __ballot(key != kNone);
+  for (int pass = 0; pass < 2 && pending; pass++) {
+    const int leader = __ffsll((unsigned long long)pending) - 1;
+    const uint32_t target = __builtin_amdgcn_readlane(key, leader);
+    const bool mine = key == target;
+    const uint64_t group = __ballot(mine);
+    if (__popcll(group) < 12) break;
+    pending &= ~group;
+    float l[3], h[3];
+    for (int a = 0; a < 3; a++) {
+      l[a] = wave_min(mine ? lo[a] : kInf);
+      h[a] = wave_max(mine ? hi[a] : -kInf);
+    }
+    if (__lane_id() == uint32_t(leader)) lds_add<COUNT>(sums + W * target, l, h, uint32_t(__popcll(group)));
+  }
+  if (pending >> __lane_id() & 1ull) lds_add<COUNT>(sums + W * key, lo, hi, 1u);
 }
 
 // Every primitive of a large node adds its box to one bin per axis.
-__global__ void k_bins_accum(uint32_t n, const uint32_t* owner, const Task* tasks, const float4* blo, const float4* bhi,
-                             Bin* bins) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t t = i < n ? owner[i] : kNone;
-  float4 lo = make_float4(kInf, kInf, kInf, 0.f), hi = make_float4(-kInf, -kInf, -kInf, 0.f);
-  int k[3] = {0, 0, 0};
-  if (t != kNone) {
-    const Task& tk = tasks[t];
-    lo = blo[i];
-    hi = bhi[i];
-    const float4 c = centroid(lo, hi);
-    k[0] = bin_of(c.x, tk.clo[0], tk.chi[0]);
-    k[1] = bin_of(c.y, tk.clo[1], tk.chi[1]);
-    k[2] = bin_of(c.z, tk.clo[2], tk.chi[2]);
-  }
-  for (int a = 0; a < 3; a++) bin_add(bins, t == kNone ? kNone : (t * 3 + a) * kBins + k[a], lo, hi);
-}
-
-// Centroid bounds of the next level's tasks.
-__global__ void k_task_cbounds(uint32_t n, const uint32_t* owner, const float4* blo, const float4* bhi, Task* tasks) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t t = i < n ? owner[i] : kNone;
-  float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (t != kNone) c = centroid(blo[i], bhi[i]);
-  uint64_t pending = __ballot(t != kNone);
-  while (pending) {
-    const int leader = __ffsll((unsigned long long)pending) - 1;
-    const uint32_t target = __shfl(t, leader);
-    const bool mine = t == target;
-    pending &= ~__ballot(mine);
-    float l0 = wave_min(mine ? c.x : kInf), l1 = wave_min(mine ? c.y : kInf), l2 = wave_min(mine ? c.z : kInf);
-    float h0 = wave_max(mine ? c.x : -kInf), h1 = wave_max(mine ? c.y : -kInf), h2 = wave_max(mine ? c.z : -kInf);
-    if (__lane_id() == leader) {
-      Task* e = &tasks[target];
-      atomic_min_f(&e->clo[0], l0);
-      atomic_min_f(&e->clo[1], l1);
-      atomic_min_f(&e->clo[2], l2);
-      atomic_max_f(&e->chi[0], h0);
-      atomic_max_f(&e->chi[1], h1);
-      atomic_max_f(&e->chi[2], h2);
+__global__ void __launch_bounds__(kLevelThreads) k_bins_accum(uint32_t n, const uint32_t* owner, const Task* tasks,
+                                                              const float4* blo, const float4* bhi, Bin* bins,
+                                                              BuildCtr* ctr) {
+  __shared__ uint32_t sSum[kLevelSlots * 3 * kBins * 7], sTask[kLevelSlots];
+  uint32_t t[kLevelItems], slot[kLevelItems];
+  const uint32_t slots = chunk_slots(n, owner, t, slot, sTask, ctr);
+  if (slots == 0) return;
+  for (uint32_t j = threadIdx.x; j < slots * 3 * kBins * 7; j += kLevelThreads)
+    sSum[j] = j % 7 < 3 ? ordered_bits(kInf) : j % 7 < 6 ? ordered_bits(-kInf) : 0u;
+  __syncthreads();
+  for (int e = 0; e < kLevelItems; e++) {
+    float lo[3] = {kInf, kInf, kInf}, hi[3] = {-kInf, -kInf, -kInf};
+    int k[3] = {0, 0, 0};
+    if (t[e] != kNone) {
+      const uint32_t i = blockIdx.x * kLevelChunk + e * kLevelThreads + threadIdx.x;
+      const Task& tk = tasks[t[e]];
+      const float4 l = blo[i], h = bhi[i], c = centroid(l, h);
+      lo[0] = l.x, lo[1] = l.y, lo[2] = l.z;
+      hi[0] = h.x, hi[1] = h.y, hi[2] = h.z;
+      k[0] = bin_of(c.x, tk.clo[0], tk.chi[0]);
+      k[1] = bin_of(c.y, tk.clo[1], tk.chi[1]);
+      k[2] = bin_of(c.z, tk.clo[2], tk.chi[2]);
     }
+    for (int a = 0; a < 3; a++) wave_add<true>(sSum, t[e] == kNone ? kNone : (slot[e] * 3 + a) * kBins + k[a], lo, hi);
+  }
+  __syncthreads();
+  for (uint32_t j = threadIdx.x; j < slots * 3 * kBins; j += kLevelThreads) {
+    const uint32_t* s = sSum + 7 * j;
+    if (s[6] == 0) continue;
+    Bin* e = &bins[size_t(sTask[j / (3 * kBins)]) * 3 * kBins + j % (3 * kBins)];
+    for (int a = 0; a < 3; a++) {
+      atomic_min_f(&e->lo[a], from_ordered(s[a]));
+      atomic_max_f(&e->hi[a], from_ordered(s[3 + a]));
+    }
+    atomicAdd(&e->count, s[6]);
   }
 }
 
-__device__ __forceinline__ void grow(float lo[3], float hi[3], const Bin& b) {
-  for (int a = 0; a < 3; a++) lo[a] = fminf(lo[a], b.lo[a]), hi[a] = fmaxf(hi[a], b.hi[a]);
+// One wave per large task: best binned SAH split over the three axes, children
+// allocated; a child of one primitive becomes a leaf, one of at most kSmall a
+// small task (its subtree's nodes reserved with it), a larger one a task of the
+// next level.  Lane 16 a + k holds bin k of axis a: prefixes and suffixes over
+// an axis are scans within a row of 16 lanes (one thread per task walked the
+// 48 bins from memory in 34 us a level, whatever the number of tasks).
+template <int CTRL, bool MAX>
+__device__ __forceinline__ float row_step(float v) {
+  const float o = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xf, 0xf, false));
+  return MAX ? fmaxf(v, o) : fminf(v, o);
+}
+template <bool SUFFIX, bool MAX>
+__device__ __forceinline__ float row_scan(float v) {  // row_shr for prefixes, row_shl for suffixes
+  constexpr int base = SUFFIX ? 0x100 : 0x110;
+  v = row_step<base + 1, MAX>(v);
+  v = row_step<base + 2, MAX>(v);
+  v = row_step<base + 4, MAX>(v);
+  return row_step<base + 8, MAX>(v);
+}
+template <bool SUFFIX>
+__device__ __forceinline__ uint32_t row_sum(uint32_t c) {
+  constexpr int base = SUFFIX ? 0x100 : 0x110;
+  int v = int(c);
+  v += __builtin_amdgcn_update_dpp(0, v, base + 1, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, base + 2, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, base + 4, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, base + 8, 0xf, 0xf, false);
+  return uint32_t(v);
+}
+__device__ __forceinline__ float prev_lane(float v, float first) {  // the value of the row's lane before, `first` at its start
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x111, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_f(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// One thread per large task: best binned SAH split over the three axes,
-// children allocated; a child of one primitive becomes a leaf, one of at
-// most kSmall a small task, a larger one a task of the next level.
-__global__ void k_split(Task* tasks, uint32_t nTasks, const Bin* bins, N2* n2, Task* next, SmallTask* smalls,
-                        BuildCtr* ctr, uint32_t maxLeaf, Caps caps) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nTasks) return;
-  Task tk = tasks[t];
+// The tasks of a block take their nodes and child tasks with one atomic each.
+constexpr int kSplitWaves = 16;
+__global__ void __launch_bounds__(64 * kSplitWaves) k_split(Task* tasks, uint32_t nTasks, const Bin* bins, N2* n2, Task* next,
+                                                            SmallTask* smalls, BuildCtr* ctr, Caps caps) {
+  __shared__ uint32_t sNeed[3][kSplitWaves], sBase[3];  // nodes, large and small child tasks
+  const int wave = int(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+  const uint32_t t = blockIdx.x * kSplitWaves + uint32_t(wave);
+  const bool valid = t < nTasks;
+  const uint32_t lane = __lane_id();
+  Task tk = tasks[valid ? t : nTasks - 1];
   const uint32_t cnt = tk.end - tk.begin;
-  float lo[3] = {kInf, kInf, kInf}, hi[3] = {-kInf, -kInf, -kInf};
-  for (int k = 0; k < kBins; k++) grow(lo, hi, bins[(t * 3) * kBins + k]);
-  float best = kInf;
-  uint32_t axis = 3, kbin = 0, nl = cnt / 2;
-  float clo[2][3], chi[2][3];  // children boxes
-  for (int c = 0; c < 2; c++)
-    for (int a = 0; a < 3; a++) clo[c][a] = lo[a], chi[c][a] = hi[a];
+  float bl[3] = {kInf, kInf, kInf}, bh[3] = {-kInf, -kInf, -kInf};
+  uint32_t bc = 0;
+  if (lane < 3 * kBins) {
+    const Bin b = bins[size_t(valid ? t : nTasks - 1) * 3 * kBins + lane];
+    for (int a = 0; a < 3; a++) bl[a] = b.lo[a], bh[a] = b.hi[a];
+    bc = b.count;
+  }
+  float pl[3], ph[3], sl[3], sh[3];  // boxes of the bins before this one, of this one and those after it
+  float lo[3], hi[3];
   for (int a = 0; a < 3; a++) {
-    const Bin* ba = bins + (t * 3 + a) * kBins;
-    float sA[kBins];
-    uint32_t sN[kBins];
-    float slo[3] = {kInf, kInf, kInf}, shi[3] = {-kInf, -kInf, -kInf};
-    uint32_t sc = 0;
-    for (int k = kBins - 1; k >= 1; k--) {
-      const Bin b = ba[k];
-      grow(slo, shi, b);
-      sc += b.count;
-      sA[k] = half_area(slo, shi);
-      sN[k] = sc;
-    }
-    float plo[3] = {kInf, kInf, kInf}, phi[3] = {-kInf, -kInf, -kInf};
-    uint32_t pc = 0;
-    for (int k = 1; k < kBins; k++) {
-      const Bin b = ba[k - 1];
-      grow(plo, phi, b);
-      pc += b.count;
-      if (pc == 0 || sN[k] == 0) continue;
-      const float c = half_area(plo, phi) * float(pc) + sA[k] * float(sN[k]);
-      if (c < best) {
-        best = c;
-        axis = uint32_t(a);
-        kbin = uint32_t(k);
-        nl = pc;
-      }
-    }
+    const float il = row_scan<false, false>(bl[a]), ih = row_scan<false, true>(bh[a]);
+    lo[a] = lane_f(il, kBins - 1);
+    hi[a] = lane_f(ih, kBins - 1);
+    pl[a] = prev_lane(il, kInf);
+    ph[a] = prev_lane(ih, -kInf);
+    sl[a] = row_scan<true, false>(bl[a]);
+    sh[a] = row_scan<true, true>(bh[a]);
   }
-  if (axis < 3) {  // exact children boxes from the chosen axis' bins
-    const Bin* ba = bins + (t * 3 + axis) * kBins;
-    for (int c = 0; c < 2; c++)
-      for (int a = 0; a < 3; a++) clo[c][a] = kInf, chi[c][a] = -kInf;
-    for (int k = 0; k < kBins; k++) grow(clo[k < int(kbin) ? 0 : 1], chi[k < int(kbin) ? 0 : 1], ba[k]);
+  const uint32_t pc = row_sum<false>(bc) - bc, sc = row_sum<true>(bc);
+  float cost = kInf;
+  if (lane < 3 * kBins && pc > 0 && sc > 0) cost = half_area(pl, ph) * float(pc) + half_area(sl, sh) * float(sc);
+  const float best = wave_min(cost);
+  const uint64_t at = __ballot(cost == best && best < kInf);
+  const bool found = at != 0;
+  const int win = found ? __ffsll((unsigned long long)at) - 1 : 0;
+  const uint32_t axis = found ? uint32_t(win) / kBins : 3u, kbin = found ? uint32_t(win) % kBins : 0u;
+  const uint32_t nl = found ? __builtin_amdgcn_readlane(pc, win) : cnt / 2;
+  float clo[2][3], chi[2][3];  // children boxes
+  for (int a = 0; a < 3; a++) {
+    clo[0][a] = found ? lane_f(pl[a], win) : lo[a];
+    chi[0][a] = found ? lane_f(ph[a], win) : hi[a];
+    clo[1][a] = found ? lane_f(sl[a], win) : lo[a];
+    chi[1][a] = found ? lane_f(sh[a], win) : hi[a];
   }
-  const uint32_t child = atomicAdd(&ctr->nodes, 2u);
-  if (child + 2 > caps.nodes) {
+  const uint32_t cb[2] = {tk.begin, tk.begin + nl}, ce[2] = {tk.begin + nl, tk.end};
+  uint32_t reserve[2], nLarge = 0, nSmall = 0;
+  for (int s = 0; s < 2; s++) {
+    const uint32_t m = ce[s] - cb[s];
+    reserve[s] = m > 1 && m <= kSmall ? 2 * (m - 1) : 0;
+    nSmall += reserve[s] ? 1u : 0u;
+    nLarge += m > kSmall ? 1u : 0u;
+  }
+  if (lane == 0) {
+    sNeed[0][wave] = valid ? 2u + reserve[0] + reserve[1] : 0u;
+    sNeed[1][wave] = valid ? nLarge : 0u;
+    sNeed[2][wave] = valid ? nSmall : 0u;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    uint32_t sum = 0;
+    for (int v = 0; v < kSplitWaves; v++) {
+      const uint32_t c = sNeed[threadIdx.x][v];
+      sNeed[threadIdx.x][v] = sum;
+      sum += c;
+    }
+    uint32_t* at = threadIdx.x == 0 ? &ctr->nodes : threadIdx.x == 1 ? &ctr->tasks : &ctr->smalls;
+    sBase[threadIdx.x] = sum ? atomicAdd(at, sum) : 0u;
+  }
+  __syncthreads();
+  if (lane != 0 || !valid) return;
+  const uint32_t child = sBase[0] + sNeed[0][wave];
+  uint32_t largeAt = sBase[1] + sNeed[1][wave], smallAt = sBase[2] + sNeed[2][wave];
+  if (child + 2 + reserve[0] + reserve[1] > caps.nodes) {
     atomicOr(&ctr->error, 1u);
     tk.axis = 3;
     tk.nl = cnt / 2;
@@ -318,7 +479,6 @@ __global__ void k_split(Task* tasks, uint32_t nTasks, const Bin* bins, N2* n2, T
   me.left = child;
   me.count = 0;
   n2[tk.node] = me;
-  const uint32_t cb[2] = {tk.begin, tk.begin + nl}, ce[2] = {tk.begin + nl, tk.end};
   for (int s = 0; s < 2; s++) {
     const uint32_t m = ce[s] - cb[s];
     tk.child_task[s] = kNone;
@@ -329,14 +489,14 @@ __global__ void k_split(Task* tasks, uint32_t nTasks, const Bin* bins, N2* n2, T
       leaf.count = m;
       n2[child + s] = leaf;
     } else if (m <= kSmall) {  // the wave builder also decides leaves of at most max_leaf
-      const uint32_t j = atomicAdd(&ctr->smalls, 1u);
+      const uint32_t j = smallAt++;
       if (j >= caps.smalls) {
         atomicOr(&ctr->error, 2u);
         continue;
       }
-      smalls[j] = SmallTask{child + s, cb[s], ce[s], 0};
+      smalls[j] = SmallTask{child + s, cb[s], ce[s], child + 2 + (s ? reserve[0] : 0u)};
     } else {
-      const uint32_t j = atomicAdd(&ctr->tasks, 1u);
+      const uint32_t j = largeAt++;
       if (j >= caps.tasks) {
         atomicOr(&ctr->error, 4u);
         continue;
@@ -376,33 +536,59 @@ __global__ void k_flags(uint32_t n, const uint32_t* owner, const Task* tasks, co
 }
 
 // Stable partition of every large task's range; primitives of finished
-// ranges keep their place.  scan: exclusive prefix sum of the flags.
-__global__ void k_scatter(uint32_t n, const uint32_t* owner, const Task* tasks, const uint32_t* flags,
-                          const uint32_t* scan, const uint32_t* ids, const float4* blo, const float4* bhi, uint32_t* ids2,
-                          float4* blo2, float4* bhi2, uint32_t* owner2, BuildCtr* ctr) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t t = owner[i];
-  uint32_t p = i, o = kNone;
-  if (t != kNone) {
-    const Task& tk = tasks[t];
-    const uint32_t before = scan[i] - scan[tk.begin];  // left-going primitives of the task before i
-    if (flags[i]) {
-      p = tk.begin + before;
-      o = tk.child_task[0];
-    } else {
-      p = tk.begin + tk.nl + (i - tk.begin - before);
-      o = tk.child_task[1];
+// ranges keep their place.  scan: exclusive prefix sum of the flags.  The
+// centroid bounds of the next level's tasks are taken on the way.
+__global__ void __launch_bounds__(kLevelThreads)
+    k_scatter(uint32_t n, const uint32_t* owner, const Task* tasks, const uint32_t* flags, const uint32_t* scan,
+              const uint32_t* ids, const float4* blo, const float4* bhi, uint32_t* ids2, float4* blo2, float4* bhi2,
+              uint32_t* owner2, Task* next, BuildCtr* ctr) {
+  __shared__ uint32_t sSum[kLevelSlots * 2 * 6], sTask[kLevelSlots];
+  uint32_t t[kLevelItems], slot[kLevelItems];
+  const uint32_t slots = chunk_slots(n, owner, t, slot, sTask, ctr);
+  for (uint32_t j = threadIdx.x; j < slots * 2 * 6; j += kLevelThreads)
+    sSum[j] = j % 6 < 3 ? ordered_bits(kInf) : ordered_bits(-kInf);
+  __syncthreads();
+  for (int e = 0; e < kLevelItems; e++) {
+    const uint32_t i = blockIdx.x * kLevelChunk + e * kLevelThreads + threadIdx.x;
+    uint32_t key = kNone;
+    float c3[3] = {0.f, 0.f, 0.f};
+    if (i < n) {
+      uint32_t p = i, o = kNone;
+      const float4 lo = blo[i], hi = bhi[i];
+      if (t[e] != kNone) {
+        const Task& tk = tasks[t[e]];
+        const uint32_t before = scan[i] - scan[tk.begin];  // left-going primitives of the task before i
+        const uint32_t right = flags[i] ? 0u : 1u;
+        p = right ? tk.begin + tk.nl + (i - tk.begin - before) : tk.begin + before;
+        o = tk.child_task[right];
+        if (o != kNone) key = 2 * slot[e] + right;
+        const float4 c = centroid(lo, hi);
+        c3[0] = c.x, c3[1] = c.y, c3[2] = c.z;
+        if (p < tk.begin || p >= tk.end) {  // the bin counts and the flags disagree: report, write nothing
+          atomicOr(&ctr->error, 8u);
+          p = kNone;
+          key = kNone;
+        }
+      }
+      if (p != kNone) {
+        ids2[p] = ids[i];
+        blo2[p] = lo;
+        bhi2[p] = hi;
+        owner2[p] = o;
+      }
     }
-    if (p < tk.begin || p >= tk.end) {  // the bin counts and the flags disagree: report, write nothing
-      atomicOr(&ctr->error, 8u);
-      return;
+    wave_add<false>(sSum, key, c3, c3);
+  }
+  __syncthreads();
+  for (uint32_t j = threadIdx.x; j < 2 * slots; j += kLevelThreads) {
+    const uint32_t* s = sSum + 6 * j;
+    const uint32_t c = tasks[sTask[j / 2]].child_task[j % 2];
+    if (c == kNone || s[0] > s[3]) continue;
+    for (int a = 0; a < 3; a++) {
+      atomic_min_f(&next[c].clo[a], from_ordered(s[a]));
+      atomic_max_f(&next[c].chi[a], from_ordered(s[3 + a]));
     }
   }
-  ids2[p] = ids[i];
-  blo2[p] = blo[i];
-  bhi2[p] = bhi[i];
-  owner2[p] = o;
 }
 
 // One wave per small task (2 to kSmall = 64 primitives, one per lane): the
@@ -412,8 +598,7 @@ __global__ void k_scatter(uint32_t n, const uint32_t* owner, const Task* tasks, 
 // become leaves unless the split is cheaper (the host builder's rule).
 constexpr int kSmallWaves = 4;
 __global__ void __launch_bounds__(64 * kSmallWaves) k_small(const SmallTask* smalls, uint32_t nSmall, uint32_t* ids,
-                                                            float4* blo, float4* bhi, N2* n2, BuildCtr* ctr,
-                                                            uint32_t maxLeaf, Caps caps) {
+                                                            float4* blo, float4* bhi, N2* n2, uint32_t maxLeaf) {
   __shared__ float4 sLo[kSmallWaves][kSmall], sHi[kSmallWaves][kSmall];
   __shared__ uint32_t sId[kSmallWaves][kSmall];
   __shared__ uint32_t sStk[kSmallWaves][kSmall][2];  // (node, begin | end << 8)
@@ -429,6 +614,9 @@ __global__ void __launch_bounds__(64 * kSmallWaves) k_small(const SmallTask* sma
       Hi[lane] = bhi[st.begin + lane];
       Id[lane] = ids[st.begin + lane];
     }
+    // the subtree's nodes were reserved with the task: an atomic per split on
+    // the one node counter bounded this kernel (14.4 ms for 1.3 M splits)
+    uint32_t used = 0;
     int sp = 0;
     if (lane == 0) {
       sStk[wave][0][0] = st.node;
@@ -531,13 +719,8 @@ __global__ void __launch_bounds__(64 * kSmallWaves) k_small(const SmallTask* sma
         Hi[pos] = mhi;
         Id[pos] = myId;
       }
-      uint32_t child = 0;
-      if (lane == 0) child = atomicAdd(&ctr->nodes, 2u);
-      child = __shfl(child, 0);
-      if (child + 2 > caps.nodes) {
-        if (lane == 0) atomicOr(&ctr->error, 1u);
-        break;
-      }
+      const uint32_t child = st.nodes + used;
+      used += 2;
       if (lane == 0) {
         N2 me;
         for (int a = 0; a < 3; a++) me.lo[a] = nlo[a], me.hi[a] = nhi[a];
@@ -688,9 +871,8 @@ __global__ void k_gather_prims(const float4* rec, const uint32_t* ids, uint32_t 
 
 // SAH cost (traversal 1, intersection 1, relative to the root area).
 __global__ void k_sah(const BvhNode4* nodes, uint32_t m, float rootA, double* cost) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  float c = 0.f;
-  if (i < m) {
+  double c = 0.0;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) {
     const BvhNode4& nd = nodes[i];
     for (int s = 0; s < 4; s++) {
       if (nd.child[s] < 0) continue;
@@ -700,7 +882,7 @@ __global__ void k_sah(const BvhNode4* nodes, uint32_t m, float rootA, double* co
     }
   }
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-  if (__lane_id() == 0 && c != 0.f) atomicAdd(cost, double(c));
+  if (__lane_id() == 0 && c != 0.0) atomicAdd(cost, c);
 }
 
 // ---------------------------------------------------------------- traversal nodes
@@ -714,6 +896,9 @@ struct WideJob {
 
 struct WideSlot {  // child `s` of BvhNode4 `n`
   uint32_t n, s;
+};
+struct WideKids {  // the children chosen for a node: BvhNode4 index * 4 + child, kNone: none
+  uint32_t k[8];
 };
 
 __device__ __forceinline__ void slot_box(const BvhNode4* nodes, WideSlot w, float lo[3], float hi[3]) {
@@ -840,8 +1025,8 @@ struct WideLevel {
   uint32_t nodes, next, prims;  // first node of this level, of the next level, first primitive this level places
 };
 template <bool EMIT>
-__global__ void k_wide(const WideJob* jobs, uint32_t nJobs, BvhNode4* nodes, unsigned long long* sums, WideLevel lv,
-                       BvhNode8* out, WideJob* next, uint32_t* perm, uint32_t* error) {
+__global__ void k_wide(const WideJob* jobs, uint32_t nJobs, BvhNode4* nodes, unsigned long long* sums, WideKids* kids,
+                       WideLevel lv, BvhNode8* out, WideJob* next, uint32_t* perm, uint32_t* error) {
   const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= nJobs) {
     if (!EMIT && j == nJobs) sums[j] = 0ull;  // the scan's last entry is the level's total
@@ -860,7 +1045,14 @@ __global__ void k_wide(const WideJob* jobs, uint32_t nJobs, BvhNode4* nodes, uns
     }
     if (n > 1) wrap = (1u << n) - 1u;
   } else {
-    n = wide_children(nodes, jb.n4, w);
+    if (EMIT) {
+      n = 0;
+      for (int i = 0; i < 8; i++)
+        if (kids[j].k[i] != kNone) w[n++] = WideSlot{kids[j].k[i] >> 2, kids[j].k[i] & 3u};
+    } else {
+      n = wide_children(nodes, jb.n4, w);
+      for (int i = 0; i < 8; i++) kids[j].k[i] = i < n ? w[i].n * 4 + w[i].s : kNone;
+    }
     uint32_t acc = 0;
     for (int i = 0; i < n; i++) {
       cnt[i] = nodes[w[i].n].count[w[i].s];
@@ -946,49 +1138,66 @@ unsigned Grid(uint64_t n, unsigned t = 256) { return unsigned((n + t - 1) / t); 
 
 }  // namespace
 
-uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, DeviceBuffer& prims, uint32_t n, hipStream_t st, DeviceBuffer& out) {
-  DeviceBuffer wide, jobs0, jobs1, sums, perm, flag, tmp;
-  flag.alloc(16);
-  HipCheck(hipMemsetAsync(flag.ptr, 0, 4, st), "wide node flag");
-  perm.alloc(size_t(std::max(n, 1u)) * 4);
-  const auto grow = [&](DeviceBuffer& b, size_t bytes, size_t keep) {  // at least `bytes`, the first `keep` kept
-    if (b.bytes >= bytes) return;
-    DeviceBuffer old;
-    std::swap(old.ptr, b.ptr);
-    std::swap(old.bytes, b.bytes);
-    b.alloc(std::max(bytes, 2 * keep));
-    if (keep) HipCheck(hipMemcpyAsync(b.ptr, old.ptr, keep, hipMemcpyDeviceToDevice, st), "wide nodes");
-    HipCheck(hipStreamSynchronize(st), "wide nodes");
+// Consecutive arrays in one allocation; with base == nullptr it only measures.
+struct Carver {
+  char* base;
+  size_t used = 0;
+  template <class T>
+  T* take(size_t n) {
+    T* r = reinterpret_cast<T*>(base ? base + used : nullptr);
+    used += (n * sizeof(T) + 255) & ~size_t(255);
+    return r;
+  }
+};
+
+uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, uint32_t maxLeaf, DeviceBuffer& prims, uint32_t n, hipStream_t st,
+                        DeviceBuffer& work, DeviceBuffer& out) {
+  // One node per BvhNode4 at most, unless leaves need nodes of their own: four
+  // leaves of at most kWideNodePrims / 4 never do.
+  const size_t cap = maxLeaf <= kWideNodePrims / 4 ? size_t(m) : 5 * size_t(m) + n / kWideNodePrims + 8;
+  size_t scanBytes = 0;
+  HipCheck(hipcub::DeviceScan::ExclusiveSum(nullptr, scanBytes, static_cast<unsigned long long*>(nullptr),
+                                            static_cast<unsigned long long*>(nullptr), int(cap + 1), st),
+           "wide scan size");
+  BvhNode8* wide;
+  WideJob *cur, *nxt;
+  unsigned long long* sums;
+  WideKids* kids;
+  uint32_t *perm, *flag;
+  char* tmp;
+  const auto carve = [&](Carver c) {
+    wide = c.take<BvhNode8>(cap);
+    cur = c.take<WideJob>(cap);
+    nxt = c.take<WideJob>(cap);
+    sums = c.take<unsigned long long>(cap + 1);
+    kids = c.take<WideKids>(cap);
+    perm = c.take<uint32_t>(std::max(n, 1u));
+    flag = c.take<uint32_t>(1);
+    tmp = c.take<char>(std::max<size_t>(scanBytes, 16));
+    return c.used;
   };
-  grow(jobs0, 4096 * sizeof(WideJob), 0);
+  const size_t need = carve(Carver{nullptr});
+  if (work.bytes < need) work.alloc(need);
+  carve(Carver{static_cast<char*>(work.ptr)});
+  HipCheck(hipMemsetAsync(flag, 0, 4, st), "wide node flag");
   const WideJob root{0, 0, 0, 0};
-  HipCheck(hipMemcpyAsync(jobs0.ptr, &root, sizeof(root), hipMemcpyHostToDevice, st), "wide root");
-  DeviceBuffer *cur = &jobs0, *nxt = &jobs1;
+  HipCheck(hipMemcpyAsync(cur, &root, sizeof(root), hipMemcpyHostToDevice, st), "wide root");
   uint32_t nJobs = 1;
   WideLevel lv{0, 1, 0};
   while (nJobs > 0) {
-    grow(wide, size_t(lv.nodes + nJobs) * sizeof(BvhNode8), size_t(lv.nodes) * sizeof(BvhNode8));
-    grow(sums, size_t(nJobs + 1) * 8, 0);
-    hipLaunchKernelGGL(k_wide<false>, dim3(Grid(nJobs + 1, 64)), dim3(64), 0, st, cur->as<WideJob>(), nJobs,
-                       nodes.as<BvhNode4>(), sums.as<unsigned long long>(), lv, nullptr, nullptr, nullptr, nullptr);
-    size_t bytes = 0;
-    HipCheck(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, sums.as<unsigned long long>(), sums.as<unsigned long long>(),
-                                              int(nJobs + 1), st),
-             "wide scan size");
-    grow(tmp, std::max<size_t>(bytes, 16), 0);
-    HipCheck(hipcub::DeviceScan::ExclusiveSum(tmp.ptr, bytes, sums.as<unsigned long long>(), sums.as<unsigned long long>(),
-                                              int(nJobs + 1), st),
-             "wide scan");
+    hipLaunchKernelGGL(k_wide<false>, dim3(Grid(nJobs + 1, 64)), dim3(64), 0, st, cur, nJobs, nodes.as<BvhNode4>(), sums, kids,
+                       lv, nullptr, nullptr, nullptr, nullptr);
+    size_t bytes = scanBytes;
+    HipCheck(hipcub::DeviceScan::ExclusiveSum(tmp, bytes, sums, sums, int(nJobs + 1), st), "wide scan");
     unsigned long long total = 0;
-    HipCheck(hipMemcpyAsync(&total, sums.as<unsigned long long>() + nJobs, 8, hipMemcpyDeviceToHost, st), "wide level");
+    HipCheck(hipMemcpyAsync(&total, sums + nJobs, 8, hipMemcpyDeviceToHost, st), "wide level");
     HipCheck(hipStreamSynchronize(st), "wide level");
     const uint32_t inner = uint32_t(total), placed = uint32_t(total >> 32);
-    if (placed > n - lv.prims) throw std::runtime_error("traversal nodes place more primitives than there are");
     lv.next = lv.nodes + nJobs;
-    grow(*nxt, size_t(std::max(inner, 1u)) * sizeof(WideJob), 0);
-    hipLaunchKernelGGL(k_wide<true>, dim3(Grid(nJobs, 64)), dim3(64), 0, st, cur->as<WideJob>(), nJobs, nodes.as<BvhNode4>(),
-                       sums.as<unsigned long long>(), lv, wide.as<BvhNode8>(), nxt->as<WideJob>(), perm.as<uint32_t>(),
-                       flag.as<uint32_t>());
+    if (placed > n - lv.prims || size_t(lv.next) + inner > cap)
+      throw std::runtime_error("traversal nodes exceed their buffers");
+    hipLaunchKernelGGL(k_wide<true>, dim3(Grid(nJobs, 64)), dim3(64), 0, st, cur, nJobs, nodes.as<BvhNode4>(), sums, kids, lv,
+                       wide, nxt, perm, flag);
     lv.nodes = lv.next;
     lv.prims += placed;
     nJobs = inner;
@@ -996,94 +1205,116 @@ uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, DeviceBuffer& prims, ui
   }
   if (lv.prims != n) throw std::runtime_error("traversal nodes do not reference every primitive");
   out.alloc(size_t(lv.nodes) * sizeof(BvhNode8));
-  HipCheck(hipMemcpyAsync(out.ptr, wide.ptr, size_t(lv.nodes) * sizeof(BvhNode8), hipMemcpyDeviceToDevice, st), "wide nodes");
+  HipCheck(hipMemcpyAsync(out.ptr, wide, size_t(lv.nodes) * sizeof(BvhNode8), hipMemcpyDeviceToDevice, st), "wide nodes");
   DeviceBuffer ordered;
   ordered.alloc(size_t(std::max(n, 1u)) * 48);
-  if (n) hipLaunchKernelGGL(k_gather_prims, dim3(Grid(n)), dim3(256), 0, st, prims.as<float4>(), perm.as<uint32_t>(), n,
-                            ordered.as<float4>());
+  if (n) hipLaunchKernelGGL(k_gather_prims, dim3(Grid(n)), dim3(256), 0, st, prims.as<float4>(), perm, n, ordered.as<float4>());
   std::swap(prims.ptr, ordered.ptr);
   std::swap(prims.bytes, ordered.bytes);
   uint32_t e = 0;
-  HipCheck(hipMemcpyAsync(&e, flag.ptr, 4, hipMemcpyDeviceToHost, st), "wide node flag");
+  HipCheck(hipMemcpyAsync(&e, flag, 4, hipMemcpyDeviceToHost, st), "wide node flag");
   HipCheck(hipStreamSynchronize(st), "wide nodes");
   if (e) throw std::runtime_error("BVH node bounds cannot be quantised (non-finite boxes?)");
   return lv.nodes;
 }
 
-void BuildBvh4Device(const float* bounds, const float4* records, uint32_t n, int maxLeaf, hipStream_t st,
-                     DeviceBuffer& nodesOut, DeviceBuffer& primsOut, DeviceBvhStats& stats) {
+void BuildBvh4Device(const PrimSource& src, int maxLeaf, hipStream_t st, DeviceBuffer& nodesOut, DeviceBuffer& primsOut,
+                     DeviceBuffer& work, DeviceBvhStats& stats) {
+  const uint32_t n = src.count;
   if (n == 0) throw std::runtime_error("scene has no primitives");
   if (maxLeaf < 1 || maxLeaf > 16) throw std::runtime_error("max_leaf_size must lie in [1, 16]");
   auto t0 = std::chrono::steady_clock::now();
-  DeviceBuffer dB, dRec, dCb, dKeys, dKeys2, dIds, dIds2, dIds3, dLo, dHi, dLo2, dHi2, dOwn0, dOwn1, dTasks0, dTasks1,
-      dSmall, dBins, dFlags, dScan, dN2, dCtr, dTmp;
-  dB.alloc(size_t(n) * 24);
-  dRec.alloc(size_t(n) * 48);
-  HipCheck(hipMemcpyAsync(dB.ptr, bounds, size_t(n) * 24, hipMemcpyHostToDevice, st), "upload bounds");
-  HipCheck(hipMemcpyAsync(dRec.ptr, records, size_t(n) * 48, hipMemcpyHostToDevice, st), "upload primitives");
-  // ordering
-  dCb.alloc(64);
-  {
-    float init[6] = {kInf, kInf, kInf, -kInf, -kInf, -kInf};
-    HipCheck(hipMemcpyAsync(dCb.ptr, init, 24, hipMemcpyHostToDevice, st), "centroid init");
-  }
-  hipLaunchKernelGGL(k_centroid_bounds, dim3(Grid(n)), dim3(256), 0, st, dB.as<float>(), n, dCb.as<float>());
-  dKeys.alloc(size_t(n) * 8);
-  dKeys2.alloc(size_t(n) * 8);
-  dIds.alloc(size_t(n) * 4);
-  dIds2.alloc(size_t(n) * 4);
-  hipLaunchKernelGGL(k_morton, dim3(Grid(n)), dim3(256), 0, st, dB.as<float>(), n, dCb.as<float>(), dKeys.as<uint64_t>(),
-                     dIds.as<uint32_t>());
-  {
-    size_t tmpBytes = 0;
-    HipCheck(hipcub::DeviceRadixSort::SortPairs(nullptr, tmpBytes, dKeys.as<uint64_t>(), dKeys2.as<uint64_t>(),
-                                                dIds.as<uint32_t>(), dIds2.as<uint32_t>(), int(n), 0, 63, st),
-             "radix sort size");
-    size_t scanBytes = 0;  // the level loop's flag scans reuse this scratch
-    HipCheck(hipcub::DeviceScan::ExclusiveSum(nullptr, scanBytes, static_cast<uint32_t*>(nullptr),
-                                              static_cast<uint32_t*>(nullptr), int(n), st),
-             "scan size");
-    dTmp.alloc(std::max<size_t>(std::max(tmpBytes, scanBytes), 16));
-    HipCheck(hipcub::DeviceRadixSort::SortPairs(dTmp.ptr, tmpBytes, dKeys.as<uint64_t>(), dKeys2.as<uint64_t>(),
-                                                dIds.as<uint32_t>(), dIds2.as<uint32_t>(), int(n), 0, 63, st),
-             "radix sort");
-  }
-  dLo.alloc(size_t(n) * 16);
-  dHi.alloc(size_t(n) * 16);
-  hipLaunchKernelGGL(k_gather_bounds, dim3(Grid(n)), dim3(256), 0, st, dB.as<float>(), dIds2.as<uint32_t>(), n,
-                     dLo.as<float4>(), dHi.as<float4>());
-  // top-down levels
   const uint32_t maxNodes = 2 * n;
-  dN2.alloc(size_t(maxNodes) * sizeof(N2));
   const uint32_t maxTasks = n / (kSmall + 1) + 2;
   const uint32_t maxSmall = n / 2 + 2;  // small tasks hold at least two primitives
-  dTasks0.alloc(size_t(maxTasks) * sizeof(Task));
-  dTasks1.alloc(size_t(maxTasks) * sizeof(Task));
-  dSmall.alloc(size_t(maxSmall) * sizeof(SmallTask));
-  dBins.alloc(size_t(maxTasks) * 3 * kBins * sizeof(Bin));
-  dOwn0.alloc(size_t(n) * 4);
-  dOwn1.alloc(size_t(n) * 4);
-  dFlags.alloc(size_t(n) * 4 + 16);
-  dScan.alloc(size_t(n) * 4 + 16);
-  dLo2.alloc(size_t(n) * 16);
-  dHi2.alloc(size_t(n) * 16);
-  dIds3.alloc(size_t(n) * 4);
-  dCtr.alloc(64);
-  BuildCtr* ctr = dCtr.as<BuildCtr>();
+  const uint32_t others = uint32_t(src.other_rec.size() / 3);
+  size_t sortBytes = 0, scanBytes = 0;
+  HipCheck(hipcub::DeviceRadixSort::SortPairs(nullptr, sortBytes, static_cast<uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr),
+                                              static_cast<uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr), int(n), 0, 63, st),
+           "radix sort size");
+  HipCheck(hipcub::DeviceScan::ExclusiveSum(nullptr, scanBytes, static_cast<uint32_t*>(nullptr),
+                                            static_cast<uint32_t*>(nullptr), int(n), st),
+           "scan size");
+  // One allocation: what lives to the end, then the arrays of the binary build
+  // and, in their place afterwards, those of the collapse (a 4-wide node per
+  // inner binary node at most).
+  float4 *rec, *lo, *hi, *lo2, *hi2, *otherRec;
+  float *box, *cb, *otherBox;
+  uint64_t *keys, *keys2;
+  uint32_t *ids0, *ids, *ids2, *own, *own2, *flags, *scan, *jc, *need;
+  N2* n2;
+  BuildCtr* ctr;
+  Task *cur, *nxt;
+  SmallTask* smalls;
+  Bin* bins;
+  PrimSegment* segs;
+  double* cost;
+  char* tmp;
+  BvhNode4* nodes;
+  Job *jcur, *jnxt;
+  const auto carve = [&](Carver c) {
+    rec = c.take<float4>(3 * size_t(n));
+    n2 = c.take<N2>(maxNodes);
+    ids0 = c.take<uint32_t>(n);
+    ids = c.take<uint32_t>(n);
+    ids2 = c.take<uint32_t>(n);
+    ctr = c.take<BuildCtr>(1);
+    jc = c.take<uint32_t>(2);
+    cost = c.take<double>(1);
+    Carver d = c;
+    box = c.take<float>(6 * size_t(n));
+    cb = c.take<float>(6);
+    keys = c.take<uint64_t>(n);
+    keys2 = c.take<uint64_t>(n);
+    lo = c.take<float4>(n);
+    hi = c.take<float4>(n);
+    lo2 = c.take<float4>(n);
+    hi2 = c.take<float4>(n);
+    own = c.take<uint32_t>(n);
+    own2 = c.take<uint32_t>(n);
+    flags = c.take<uint32_t>(n);
+    scan = c.take<uint32_t>(n);
+    cur = c.take<Task>(maxTasks);
+    nxt = c.take<Task>(maxTasks);
+    smalls = c.take<SmallTask>(maxSmall);
+    bins = c.take<Bin>(size_t(maxTasks) * 3 * kBins);
+    tmp = c.take<char>(std::max<size_t>(std::max(sortBytes, scanBytes), 16));
+    segs = c.take<PrimSegment>(src.segs.size());
+    otherRec = c.take<float4>(std::max(3 * size_t(others), size_t(1)));
+    otherBox = c.take<float>(std::max(6 * size_t(others), size_t(1)));
+    nodes = d.take<BvhNode4>(n);
+    jcur = d.take<Job>(n);
+    jnxt = d.take<Job>(n);
+    need = d.take<uint32_t>(n);
+    return std::max(c.used, d.used);
+  };
+  work.alloc(carve(Carver{nullptr}));
+  carve(Carver{static_cast<char*>(work.ptr)});
+  // primitives
+  HipCheck(hipMemcpyAsync(segs, src.segs.data(), src.segs.size() * sizeof(PrimSegment), hipMemcpyHostToDevice, st), "segments");
+  if (others) {
+    HipCheck(hipMemcpyAsync(otherRec, src.other_rec.data(), size_t(others) * 48, hipMemcpyHostToDevice, st), "primitives");
+    HipCheck(hipMemcpyAsync(otherBox, src.other_box.data(), size_t(others) * 24, hipMemcpyHostToDevice, st), "bounds");
+  }
+  hipLaunchKernelGGL(k_primitives, dim3(Grid(n)), dim3(256), 0, st, segs, uint32_t(src.segs.size()), src.d_tris, otherRec,
+                     otherBox, n, rec, box);
+  // ordering
+  const float init[6] = {kInf, kInf, kInf, -kInf, -kInf, -kInf};
+  HipCheck(hipMemcpyAsync(cb, init, 24, hipMemcpyHostToDevice, st), "centroid init");
+  hipLaunchKernelGGL(k_centroid_bounds, dim3(std::min(Grid(n), 256u)), dim3(256), 0, st, box, n, cb);
+  hipLaunchKernelGGL(k_morton, dim3(Grid(n)), dim3(256), 0, st, box, n, cb, keys, ids0);
+  HipCheck(hipcub::DeviceRadixSort::SortPairs(tmp, sortBytes, keys, keys2, ids0, ids, int(n), 0, 63, st), "radix sort");
+  hipLaunchKernelGGL(k_gather_bounds, dim3(Grid(n)), dim3(256), 0, st, box, ids, n, lo, hi);
+  // top-down levels
   const Caps caps{maxNodes, maxTasks, maxSmall};
-  uint32_t* ids = dIds2.as<uint32_t>();  // Morton order
-  uint32_t* ids2 = dIds3.as<uint32_t>();
-  float4* lo = dLo.as<float4>();
-  float4* hi = dHi.as<float4>();
-  float4* lo2 = dLo2.as<float4>();
-  float4* hi2 = dHi2.as<float4>();
   uint32_t levels = 0, nSmall = 0;
   BuildCtr c0{1, 0, 0, 0};
   if (n == 1) {
-    hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(64), 0, st, lo, hi, n, dN2.as<N2>());
+    hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(64), 0, st, lo, hi, n, n2);
   } else if (n <= kSmall) {
-    SmallTask root{0, 0, n, 0};
-    HipCheck(hipMemcpyAsync(dSmall.ptr, &root, sizeof(root), hipMemcpyHostToDevice, st), "root task");
+    const SmallTask root{0, 0, n, 1};
+    HipCheck(hipMemcpyAsync(smalls, &root, sizeof(root), hipMemcpyHostToDevice, st), "root task");
+    c0.nodes = 1 + 2 * (n - 1);
     c0.smalls = 1;
     nSmall = 1;
   } else {
@@ -1093,33 +1324,26 @@ void BuildBvh4Device(const float* bounds, const float4* records, uint32_t n, int
     root.end = n;
     root.axis = 3;
     root.child_task[0] = root.child_task[1] = kNone;
-    HipCheck(hipMemcpyAsync(&root.clo, dCb.ptr, 12, hipMemcpyDeviceToHost, st), "centroid bounds");
-    HipCheck(hipMemcpyAsync(&root.chi, dCb.as<float>() + 3, 12, hipMemcpyDeviceToHost, st), "centroid bounds");
+    HipCheck(hipMemcpyAsync(&root.clo, cb, 12, hipMemcpyDeviceToHost, st), "centroid bounds");
+    HipCheck(hipMemcpyAsync(&root.chi, cb + 3, 12, hipMemcpyDeviceToHost, st), "centroid bounds");
     HipCheck(hipStreamSynchronize(st), "centroid bounds");
-    HipCheck(hipMemcpyAsync(dTasks0.ptr, &root, sizeof(Task), hipMemcpyHostToDevice, st), "root task");
-    HipCheck(hipMemsetAsync(dOwn0.ptr, 0, size_t(n) * 4, st), "owners");
+    HipCheck(hipMemcpyAsync(cur, &root, sizeof(Task), hipMemcpyHostToDevice, st), "root task");
+    HipCheck(hipMemsetAsync(own, 0, size_t(n) * 4, st), "owners");
   }
   HipCheck(hipMemcpyAsync(ctr, &c0, sizeof(c0), hipMemcpyHostToDevice, st), "counters");
   if (n > kSmall) {
     uint32_t nTasks = 1;
-    Task* cur = dTasks0.as<Task>();
-    Task* nxt = dTasks1.as<Task>();
-    uint32_t* own = dOwn0.as<uint32_t>();
-    uint32_t* own2 = dOwn1.as<uint32_t>();
     while (nTasks > 0) {
       if (++levels > 128) throw std::runtime_error("BVH build did not converge");
-      hipLaunchKernelGGL(k_bins_clear, dim3(Grid(uint64_t(nTasks) * 3 * kBins)), dim3(256), 0, st, dBins.as<Bin>(),
-                         nTasks * 3 * kBins);
-      hipLaunchKernelGGL(k_bins_accum, dim3(Grid(n)), dim3(256), 0, st, n, own, cur, lo, hi, dBins.as<Bin>());
+      hipLaunchKernelGGL(k_bins_clear, dim3(Grid(uint64_t(nTasks) * 3 * kBins)), dim3(256), 0, st, bins, nTasks * 3 * kBins);
+      hipLaunchKernelGGL(k_bins_accum, dim3(Grid(n, kLevelChunk)), dim3(kLevelThreads), 0, st, n, own, cur, lo, hi, bins, ctr);
       HipCheck(hipMemsetAsync(&ctr->tasks, 0, 4, st), "level counter");
-      hipLaunchKernelGGL(k_split, dim3(Grid(nTasks, 64)), dim3(64), 0, st, cur, nTasks, dBins.as<Bin>(), dN2.as<N2>(), nxt,
-                         dSmall.as<SmallTask>(), ctr, uint32_t(maxLeaf), caps);
-      hipLaunchKernelGGL(k_flags, dim3(Grid(n)), dim3(256), 0, st, n, own, cur, lo, hi, dFlags.as<uint32_t>());
-      size_t scanBytes = dTmp.bytes;
-      HipCheck(hipcub::DeviceScan::ExclusiveSum(dTmp.ptr, scanBytes, dFlags.as<uint32_t>(), dScan.as<uint32_t>(), int(n), st),
-               "flag scan");
-      hipLaunchKernelGGL(k_scatter, dim3(Grid(n)), dim3(256), 0, st, n, own, cur, dFlags.as<uint32_t>(),
-                         dScan.as<uint32_t>(), ids, lo, hi, ids2, lo2, hi2, own2, ctr);
+      hipLaunchKernelGGL(k_split, dim3(Grid(nTasks, kSplitWaves)), dim3(64 * kSplitWaves), 0, st, cur, nTasks, bins, n2, nxt, smalls, ctr, caps);
+      hipLaunchKernelGGL(k_flags, dim3(Grid(n)), dim3(256), 0, st, n, own, cur, lo, hi, flags);
+      size_t bytes = scanBytes;
+      HipCheck(hipcub::DeviceScan::ExclusiveSum(tmp, bytes, flags, scan, int(n), st), "flag scan");
+      hipLaunchKernelGGL(k_scatter, dim3(Grid(n, kLevelChunk)), dim3(kLevelThreads), 0, st, n, own, cur, flags, scan, ids, lo, hi,
+                         ids2, lo2, hi2, own2, nxt, ctr);
       std::swap(ids, ids2);
       std::swap(lo, lo2);
       std::swap(hi, hi2);
@@ -1131,68 +1355,45 @@ void BuildBvh4Device(const float* bounds, const float4* records, uint32_t n, int
         throw std::runtime_error("BVH build exceeded its buffers");
       nTasks = h.tasks;
       nSmall = h.smalls;
-      if (nTasks) hipLaunchKernelGGL(k_task_cbounds, dim3(Grid(n)), dim3(256), 0, st, n, own, lo, hi, nxt);
       std::swap(cur, nxt);
     }
   }
   if (nSmall) {
     const uint32_t blocks = std::min<uint32_t>((nSmall + kSmallWaves - 1) / kSmallWaves, 65535u * 4u);
-    hipLaunchKernelGGL(k_small, dim3(blocks), dim3(64 * kSmallWaves), 0, st, dSmall.as<SmallTask>(), nSmall, ids, lo, hi,
-                       dN2.as<N2>(), ctr, uint32_t(maxLeaf), caps);
-    BuildCtr h{};
-    HipCheck(hipMemcpyAsync(&h, ctr, sizeof(h), hipMemcpyDeviceToHost, st), "small readback");
-    HipCheck(hipStreamSynchronize(st), "BVH small subtrees");
-    if (h.error || h.nodes > maxNodes) throw std::runtime_error("BVH build exceeded its buffers");
+    hipLaunchKernelGGL(k_small, dim3(blocks), dim3(64 * kSmallWaves), 0, st, smalls, nSmall, ids, lo, hi, n2, uint32_t(maxLeaf));
   }
-  const uint32_t* sorted = ids;
   // collapse
-  BuildCtr hc{};
-  HipCheck(hipMemcpyAsync(&hc, ctr, sizeof(hc), hipMemcpyDeviceToHost, st), "node count");
-  HipCheck(hipStreamSynchronize(st), "BVH build");
-  const uint32_t n2count = hc.nodes;  // the counter starts at 1 (the root)
-  nodesOut.alloc(size_t(n2count) * sizeof(BvhNode4));
-  DeviceBuffer dJobs0, dJobs1, dJc;
-  dJobs0.alloc(size_t(n2count) * sizeof(Job));
-  dJobs1.alloc(size_t(n2count) * sizeof(Job));
-  dJc.alloc(16);
-  Job rj{0, 0};
-  HipCheck(hipMemcpyAsync(dJobs0.ptr, &rj, sizeof(rj), hipMemcpyHostToDevice, st), "root job");
-  uint32_t jc[2] = {1, 0};
+  const Job rj{0, 0};
+  HipCheck(hipMemcpyAsync(jcur, &rj, sizeof(rj), hipMemcpyHostToDevice, st), "root job");
+  uint32_t hjc[2] = {1, 0};
   uint32_t nJobs = 1, depth = 0;
-  Job* jcur = dJobs0.as<Job>();
-  Job* jnxt = dJobs1.as<Job>();
   std::vector<uint32_t> levelStart{0u};  // the nodes of level k are [levelStart[k], levelStart[k + 1])
   while (nJobs > 0) {
     depth++;
-    levelStart.push_back(jc[0]);
-    jc[1] = 0;
-    HipCheck(hipMemcpyAsync(dJc.ptr, jc, 8, hipMemcpyHostToDevice, st), "collapse counters");
-    hipLaunchKernelGGL(k_collapse, dim3(Grid(nJobs, 64)), dim3(64), 0, st, jcur, nJobs, dN2.as<N2>(),
-                       nodesOut.as<BvhNode4>(), jnxt, dJc.as<uint32_t>());
-    HipCheck(hipMemcpyAsync(jc, dJc.ptr, 8, hipMemcpyDeviceToHost, st), "collapse readback");
+    levelStart.push_back(hjc[0]);
+    hjc[1] = 0;
+    HipCheck(hipMemcpyAsync(jc, hjc, 8, hipMemcpyHostToDevice, st), "collapse counters");
+    hipLaunchKernelGGL(k_collapse, dim3(Grid(nJobs, 64)), dim3(64), 0, st, jcur, nJobs, n2, nodes, jnxt, jc);
+    HipCheck(hipMemcpyAsync(hjc, jc, 8, hipMemcpyDeviceToHost, st), "collapse readback");
     HipCheck(hipStreamSynchronize(st), "collapse level");
-    nJobs = jc[1];
+    nJobs = hjc[1];
     std::swap(jcur, jnxt);
   }
-  const uint32_t n4 = jc[0];
+  const uint32_t n4 = hjc[0];
   levelStart.push_back(n4);
-  uint32_t stackNeed = 0;
-  {
-    DeviceBuffer dNeed;
-    dNeed.alloc(size_t(n4) * sizeof(uint32_t));
-    for (size_t k = levelStart.size() - 1; k-- > 0;) {
-      const uint32_t b = levelStart[k], e = levelStart[k + 1];
-      if (e > b) hipLaunchKernelGGL(k_stack_need, dim3(Grid(e - b)), dim3(256), 0, st, nodesOut.as<BvhNode4>(), b, e,
-                                    dNeed.as<uint32_t>());
-    }
-    HipCheck(hipMemcpyAsync(&stackNeed, dNeed.ptr, sizeof(uint32_t), hipMemcpyDeviceToHost, st), "stack need");
-    HipCheck(hipStreamSynchronize(st), "stack need");
+  for (size_t k = levelStart.size() - 1; k-- > 0;) {
+    const uint32_t b = levelStart[k], e = levelStart[k + 1];
+    if (e > b) hipLaunchKernelGGL(k_stack_need, dim3(Grid(e - b)), dim3(256), 0, st, nodes, b, e, need);
   }
+  uint32_t stackNeed = 0;
+  HipCheck(hipMemcpyAsync(&stackNeed, need, sizeof(uint32_t), hipMemcpyDeviceToHost, st), "stack need");
+  nodesOut.alloc(size_t(n4) * sizeof(BvhNode4));
+  HipCheck(hipMemcpyAsync(nodesOut.ptr, nodes, size_t(n4) * sizeof(BvhNode4), hipMemcpyDeviceToDevice, st), "nodes");
   primsOut.alloc(size_t(n) * 48);
-  hipLaunchKernelGGL(k_gather_prims, dim3(Grid(n)), dim3(256), 0, st, dRec.as<float4>(), sorted, n, primsOut.as<float4>());
+  hipLaunchKernelGGL(k_gather_prims, dim3(Grid(n)), dim3(256), 0, st, rec, ids, n, primsOut.as<float4>());
   // statistics: SAH cost relative to the root box
   BvhNode4 root;
-  HipCheck(hipMemcpyAsync(&root, nodesOut.ptr, sizeof(root), hipMemcpyDeviceToHost, st), "root readback");
+  HipCheck(hipMemcpyAsync(&root, nodes, sizeof(root), hipMemcpyDeviceToHost, st), "root readback");
   HipCheck(hipStreamSynchronize(st), "BVH finish");
   float rlo[3] = {kInf, kInf, kInf}, rhi[3] = {-kInf, -kInf, -kInf};
   for (int s = 0; s < 4; s++) {
@@ -1204,12 +1405,10 @@ void BuildBvh4Device(const float* bounds, const float4* records, uint32_t n, int
   float rootA = 2.f * (dx * dy + dy * dz + dz * dx);
   double sah = 1.0;
   if (rootA > 0.f) {
-    DeviceBuffer dCost;
-    dCost.alloc(16);
-    HipCheck(hipMemsetAsync(dCost.ptr, 0, 8, st), "sah");
-    hipLaunchKernelGGL(k_sah, dim3(Grid(n4)), dim3(256), 0, st, nodesOut.as<BvhNode4>(), n4, rootA, dCost.as<double>());
+    HipCheck(hipMemsetAsync(cost, 0, 8, st), "sah");
+    hipLaunchKernelGGL(k_sah, dim3(std::min(Grid(n4), 256u)), dim3(256), 0, st, nodes, n4, rootA, cost);
     double c = 0;
-    HipCheck(hipMemcpyAsync(&c, dCost.ptr, 8, hipMemcpyDeviceToHost, st), "sah readback");
+    HipCheck(hipMemcpyAsync(&c, cost, 8, hipMemcpyDeviceToHost, st), "sah readback");
     HipCheck(hipStreamSynchronize(st), "sah");
     sah += c;
   }

@@ -237,12 +237,27 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
     HostScene& h = scene->host;
     uint32_t n = uint32_t(h.prim_bounds.size() / 6);
     auto t0 = std::chrono::steady_clock::now();
-    uint32_t nodeCount = 0, depth = 0, stackNeed = 0;
+    uint32_t nodeCount = 0, depth = 0, stackNeed = 0, largestLeaf = uint32_t(maxLeaf);
     float sah = 0.f;
+    DeviceBuffer work;
     if (builder == RAD_BVH_DEVICE) {
       DeviceBvhStats ds;
-      BuildBvh4Device(h.prim_bounds.data(), h.prim_records.data(), n, maxLeaf, scene->ctx->stream, scene->d_nodes,
-                      scene->d_prims, ds);
+      PrimSource src;
+      src.d_tris = scene->d_tris.as<float4>();
+      src.count = n;
+      for (uint32_t k = 0, p = 0; k < h.shapes.size(); k++) {
+        const ShapeRec& s = h.shapes[k];
+        PrimSegment sg{p, k, s.tri_offset, 0xffffffffu};
+        if (s.type != SHAPE_MESH) {
+          sg.other = uint32_t(src.other_rec.size() / 3);
+          src.other_rec.insert(src.other_rec.end(), &h.prim_records[3 * size_t(p)], &h.prim_records[3 * size_t(p)] + 3);
+          src.other_box.insert(src.other_box.end(), &h.prim_bounds[6 * size_t(p)], &h.prim_bounds[6 * size_t(p)] + 6);
+        }
+        const uint32_t prims = s.type == SHAPE_MESH ? s.tri_count : 1u;
+        if (prims) src.segs.push_back(sg);
+        p += prims;
+      }
+      BuildBvh4Device(src, maxLeaf, scene->ctx->stream, scene->d_nodes, scene->d_prims, work, ds);
       nodeCount = ds.node_count;
       depth = ds.depth;
       stackNeed = ds.stack_need;
@@ -256,6 +271,8 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
       scene->d_prims.upload(ordered.data(), ordered.size() * sizeof(float4), scene->ctx->stream);
       scene->d_nodes.upload(r.nodes.data(), r.nodes.size() * sizeof(BvhNode4), scene->ctx->stream);
       HipCheck(hipStreamSynchronize(scene->ctx->stream), "BVH upload");
+      for (const BvhNode4& nd : r.nodes)  // at the builder's depth limit a leaf may be larger than asked for
+        for (uint32_t c : nd.count) largestLeaf = std::max(largestLeaf, c);
       nodeCount = uint32_t(r.nodes.size());
       depth = r.depth;
       stackNeed = r.stack_need;
@@ -270,7 +287,8 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
                                                  " traversal stack entries; the traversal holds " +
                                                  std::to_string(kTraceStackEntries));
     }
-    scene->wide_count = BuildWideNodes(scene->d_nodes, nodeCount, scene->d_prims, n, scene->ctx->stream, scene->d_wnodes);
+    scene->wide_count = BuildWideNodes(scene->d_nodes, nodeCount, largestLeaf, scene->d_prims, n, scene->ctx->stream, work,
+                                       scene->d_wnodes);
     scene->builder = builder;
     scene->bvh_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     scene->dev.nodes = scene->d_nodes.as<BvhNode4>();
