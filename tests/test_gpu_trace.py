@@ -98,3 +98,20 @@ def test_ties_do_not_depend_on_the_batch(hip_ctx):
     assert np.array_equal(whole[order], g.closest(rays[order]))
     assert np.array_equal(whole[100:163], g.closest(rays[100:163]))
     assert np.array_equal(whole[7:8], g.closest(rays[7:8]))
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (7, 5), (8, 8), (9, 17), (23, 3), (65, 31)])
+def test_every_pixel_gets_its_samples(hip_ctx, w, h):
+    """Images whose last tiles are partial: under a constant sky every pixel is
+    the float32 running sum of its spp equal samples times 1/spp."""
+    b = scenes.SceneBuilder()
+    b.sphere(center=(0, 0, -50), radius=1.0, bsdf=b.diffuse(0.5))
+    b.skybox((0.3, 0.7, 1.1))
+    b.set_camera(w, h, 40, origin=(0, 0, 0), target=(0, 0, 1), far=100)
+    b.set_render("path", spp=5, max_depth=4)
+    img, _, st = hip.Scene.from_builder(hip_ctx, b).render(b.render_desc(spp=5, seed=1))
+    acc = np.zeros(3, np.float32)
+    for _ in range(5):
+        acc = (acc + np.array([0.3, 0.7, 1.1], np.float32)).astype(np.float32)
+    assert st.samples == 5 * w * h
+    assert np.array_equal(img, np.broadcast_to((acc * np.float32(1 / np.float32(5))).astype(np.float32), img.shape))
