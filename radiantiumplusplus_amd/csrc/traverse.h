@@ -184,6 +184,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) u32x2 lds_u2;
 typedef __attribute__((address_space(3))) u32x4 lds_u4;
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
 typedef __attribute__((address_space(3))) unsigned long long lds_u64;
 
 // Per-lane private overflow of a traversal stack (entries below the LDS ring).
@@ -435,15 +436,90 @@ __device__ __forceinline__ uint32_t wave_exclusive_sum(uint32_t v) {
   return uint32_t(x) - v;
 }
 
+// Items of a launch for the lanes of a wave, consecutive ones together.  A
+// wave's first share is its own by position and only the rest is dealt out in
+// chunks, one atomic each: a counter takes about 11 ns per atomic (and a load
+// of it waits as long) whoever asks, so with one per wave and 64 items an
+// extension launch of a million rays over a small tree took 263 us, now 150,
+// and an empty launch of 8192 waves 95 us.  A block asks a used-up counter once.
+// All members are wave-uniform.
+struct ItemDealer {
+  uint32_t n, base, left;   // items in all; the wave's own
+  uint32_t dealt, chunk;    // items given out by position; of one later chunk
+  uint32_t* ctr;            // later chunks (nullptr: none)
+  lds_u32* used_up;         // set once the counter has no more for this block
+  bool exhausted;           // nothing left beyond the wave's own
+
+  // wave: this wave's number; those from `waves` on get nothing
+  __device__ __forceinline__ void start(uint32_t items, uint32_t* counter, lds_u32* flag, uint32_t wave, uint32_t waves,
+                                        uint32_t share, uint32_t later) {
+    n = items;
+    ctr = counter;
+    used_up = flag;
+    chunk = later;
+    const unsigned long long b = static_cast<unsigned long long>(wave) * share;
+    base = uint32_t(b);
+    left = wave < waves && b < n ? min(share, uint32_t(n - b)) : 0u;
+    dealt = uint32_t(min(static_cast<unsigned long long>(waves) * share, static_cast<unsigned long long>(n)));
+    exhausted = !ctr || wave >= waves || dealt == n;
+  }
+  __device__ __forceinline__ bool more() const { return !exhausted || left > 0; }
+  // The next item for each lane of `need`; n or more: none.
+  __device__ __forceinline__ uint32_t take(unsigned long long need, uint32_t lane) {
+    const uint32_t want = (uint32_t)__popcll(need);
+    const uint32_t rank = (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
+    uint32_t nbase = 0, nleft = 0;
+    if (left < want && !exhausted) {
+      uint32_t b = n;
+      if (!*(volatile lds_u32*)used_up) {
+        if (lane == 0) b = atomicAdd(ctr, chunk);
+        b = __builtin_amdgcn_readfirstlane(b) + dealt;  // scalar, as are the loops that depend on it
+        if (b >= n) *(volatile lds_u32*)used_up = 1u;
+      }
+      b = __builtin_amdgcn_readfirstlane(b);
+      if (b >= n) {
+        exhausted = true;
+      } else {
+        nbase = b;
+        nleft = min(chunk, n - b);
+        if (n - b <= chunk) exhausted = true;
+      }
+    }
+    uint32_t i = 0xffffffffu;
+    if (rank < left)
+      i = base + rank;
+    else if (rank - left < nleft)
+      i = nbase + (rank - left);
+    const uint32_t fromOld = min(want, left);
+    base += fromOld;
+    left -= fromOld;
+    if (nleft) {
+      const uint32_t fromNew = min(want - fromOld, nleft);
+      base = nbase + fromNew;
+      left = nleft - fromNew;
+    }
+    return i;
+  }
+};
+// Shares of a launch of n items over `waves` resident waves: two fifths by
+// position, the rest in chunks of a third of the mean.  All by position left a
+// frame's first launch waiting for the waves that own its costliest part (1080p
+// large mesh, extension rays 57.9 -> 86 ms), chunks of an eighth and less
+// waited on the counter (volume 15.0 -> 21.0 ms).
+__device__ __forceinline__ void deal_shares(uint32_t n, uint32_t waves, uint32_t& share, uint32_t& chunk) {
+  const uint32_t mean = (n + waves - 1) / waves;
+  share = max(64u, (mean * 2u / 5u + 63u) & ~63u);
+  chunk = min(max(mean / 3u, 64u), 512u);
+}
+
 // Stream traversal for kernels that own a batch of rays.  Rays end at
 // different steps, so a lane that has none takes the next of the batch while
 // the others continue; and about one lane-step in nine reaches leaves, so a
 // wave queues the leaf groups its lanes find and intersects their primitives
 // together, 64 at a time, once enough have gathered (flush_leaves).
 //
-// Rays: with fetch, each wave takes chunks of consecutive items, the first by
-// its position and later ones with one atomic each; with fetch == nullptr,
-// wave w of the grid owns the items [w * per_wave, (w + 1) * per_wave).
+// Rays: dealt out by ItemDealer, from the counter `fetch`; with fetch ==
+// nullptr, wave w of the grid owns the items [w * per_wave, (w + 1) * per_wave).
 // Job: bool load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax, uint32_t& tag)
 //      void finish(uint32_t i, uint32_t tag, const TraceRay& r)
 //      static constexpr bool kTagIsIndex; with it the tag is the item index
@@ -462,8 +538,9 @@ constexpr uint32_t kGroupQueue = kGroupFlush + 64;  // a step adds at most one g
 constexpr uint32_t kPoolSize = kTracePool;
 // Waves that a launch's rays are spread over before a wave fills all its lanes
 // (two per SIMD: 1024 to 4096 measured alike, without it a 64x48 render's
-// traversal took 8 % longer), fewest lanes of a wave, and the largest chunk.
-constexpr uint32_t kSpreadWaves = 2048, kMinLanes = 8, kMaxChunk = 256;
+// traversal took 8 % longer) and fewest lanes of a wave.
+constexpr uint32_t kSpreadWaves = 2048, kMinLanes = 8;
+constexpr uint32_t kResidentWaves = 5 * 4 * 256;  // five per SIMD (the traversal kernels' registers), 256 CUs
 
 template <bool ANY, bool FAR, class Job>
 __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint32_t* fetch, uint32_t per_wave, Job& job) {
@@ -471,6 +548,7 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
   __shared__ u32x4 lds_group[kTraceBlock / 64][kGroupQueue];
   __shared__ u32x2 lds_pool[kTraceBlock / 64][kPoolSize];
   __shared__ unsigned long long lds_key[kTraceBlock];
+  __shared__ uint32_t lds_used_up;  // the counter has no more items for this block
   const uint32_t lane = __lane_id();
   const unsigned long long below = (1ull << lane) - 1ull;
   const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -487,29 +565,24 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
   bool have = false, active = false, pend = false;
   uint32_t idx = 0, tag = 0, visits = 0;
   uint32_t queued = 0;            // leaf groups queued by the wave (wave-uniform)
-  uint32_t cbase = 0, cleft = 0;  // the wave's chunk (wave-uniform)
-  bool exhausted = false;
   // With few rays a wave fills only some of its lanes, so that they spread over
   // the chip: a wave's step takes the longer the more lanes it has (more of
   // them reach leaves), and a launch cannot end before its slowest wave.
-  // With fetch, a wave's first chunk is its own by position and only later
-  // ones cost an atomic: the counter takes about 11 ns per atomic, and one per
-  // wave made an empty launch of 8192 waves last 95 us.
-  const uint32_t wave = blockIdx.x * (kTraceBlock / 64) + wv, waves = gridDim.x * (kTraceBlock / 64);
-  uint32_t lanes, chunk;
+  const uint32_t wave = blockIdx.x * (kTraceBlock / 64) + wv;
+  uint32_t lanes, share, chunk = 0, waves = gridDim.x * (kTraceBlock / 64);
   if (!fetch) {
-    chunk = per_wave;
+    share = per_wave;
     lanes = min(64u, per_wave);
   } else {
+    waves = min(waves, kResidentWaves);
     lanes = min(64u, max(kMinLanes, (n + kSpreadWaves - 1) / kSpreadWaves));
-    chunk = lanes < 64 ? lanes : min(max(n / waves / 4u, 64u), kMaxChunk);
+    deal_shares(n, waves, share, chunk);
+    if (lanes < 64) share = chunk = lanes;
   }
-  {
-    const unsigned long long b = static_cast<unsigned long long>(wave) * chunk;
-    cbase = uint32_t(b);
-    cleft = b < n ? min(chunk, uint32_t(n - b)) : 0u;
-    exhausted = !fetch || static_cast<unsigned long long>(waves) * chunk >= n;
-  }
+  if (threadIdx.x == 0) lds_used_up = 0u;
+  __syncthreads();
+  ItemDealer items;
+  items.start(n, fetch, (lds_u32*)&lds_used_up, wave, waves, share, chunk);
   const unsigned long long usable = ~0ull >> (64 - lanes);
   const uint32_t refill = lanes * 3 / 4;                    // refill once fewer lanes than this have a ray in flight
   const uint32_t flush = min(kGroupFlush, lanes * 3 / 8);  // queued leaf groups at which the wave tests them
@@ -524,37 +597,10 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
       job.finish(Job::kTagIsIndex ? tag : idx, tag, r);
       have = false;
     }
-    if (!exhausted || cleft > 0) {
+    if (items.more()) {
       const unsigned long long need = __ballot(!have) & usable;
       if (need) {
-        const uint32_t want = (uint32_t)__popcll(need);
-        const uint32_t rank = (uint32_t)__popcll(need & below);
-        uint32_t i = 0xffffffffu;
-        uint32_t nbase = 0, nleft = 0;
-        if (cleft < want && !exhausted) {
-          uint32_t b = 0;
-          if (lane == 0) b = atomicAdd(fetch, chunk);
-          b = __builtin_amdgcn_readfirstlane(b) + waves * chunk;  // scalar, as are the loop's exits
-          if (b >= n) {
-            exhausted = true;
-          } else {
-            nbase = b;
-            nleft = min(chunk, n - b);
-            if (n - b <= chunk) exhausted = true;
-          }
-        }
-        if (rank < cleft)
-          i = cbase + rank;
-        else if (rank - cleft < nleft)
-          i = nbase + (rank - cleft);
-        const uint32_t fromOld = min(want, cleft);
-        cbase += fromOld;
-        cleft -= fromOld;
-        if (nleft) {
-          const uint32_t fromNew = min(want - fromOld, nleft);
-          cbase = nbase + fromNew;
-          cleft = nleft - fromNew;
-        }
+        const uint32_t i = items.take(need, lane);
         if ((need >> lane & 1ull) && i < n) {
           f3 o, d;
           float tmin, tmax;
@@ -569,7 +615,7 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
       }
     }
     if (__ballot(have) == 0ull) {
-      if (exhausted && cleft == 0) break;  // every finished ray was written out above
+      if (!items.more()) break;  // every finished ray was written out above
       continue;
     }
     for (;;) {
@@ -655,7 +701,7 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
         have = false;
       }
       if (busy == 0 && queued == 0) break;
-      if ((!exhausted || cleft > 0) && (uint32_t)__popcll(__ballot(active || pend)) < refill) break;
+      if (items.more() && (uint32_t)__popcll(__ballot(active || pend)) < refill) break;
     }
   }
 }
