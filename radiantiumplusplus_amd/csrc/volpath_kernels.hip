@@ -303,6 +303,10 @@ __global__ void __launch_bounds__(256) k_shade_vol(Wavefront w, DevScene scene, 
 // collisions (si.T - mei.T, as vol_path.cpp:300 keeps it), which changes
 // nothing but the cost.  Lanes are refilled from the shadow queue as their
 // rays finish, so one long transmittance walk does not hold its wave.
+// Lanes without a ray at which a wave takes new ones (12 to 40: the same), and
+// the waves that are resident at once (four per SIMD at 126 VGPRs; volume frame,
+// this kernel: 28.1 ms, dealt over three per SIMD 30.7, over eight 37.2).
+constexpr uint32_t kVolShadowRefill = 24, kVolShadowWaves = 4 * 4 * 256;
 struct VolShadowRay {
   f3 o, d, oTrace;  // origin, direction, origin the cached hit distance h.t refers to
   f3 tr;
@@ -334,128 +338,133 @@ __device__ __forceinline__ void vol_shadow_begin(const Wavefront& w, uint32_t i,
   r.siT = kInf;
 }
 
-// One pass of the reference's while loop; returns false once the ray is done.
-__device__ __forceinline__ bool vol_shadow_step(const DevScene& scene, VolShadowRay& r, uint32_t& steps) {
-  const float remaining = r.dist * (1.f - kShadowEps) - r.totalDist;
-  if (!(remaining > 0.f)) return false;
-  bool escaped = false;
-  bool activeMedium = r.medium >= 0;
-  bool activeSurface = !activeMedium;
-  // The reference intersects in the medium branch (vol_path.cpp:258-263) or
-  // the surface branch (:316-320), whichever is active, from the same origin
-  // and only when a new straight segment starts; one call site serves both.
-  if (r.needsIntersection) {
-    r.hitValid = trace<false>(scene, r.o, r.d, 0.f, remaining, r.h);
-    r.siT = r.hitValid ? r.h.t : kInf;
-    r.oTrace = r.o;
-    r.needsIntersection = false;
-  }
-  if (activeMedium) {
-    const MediumRec& M = scene.media[r.medium];
-    MediumSample mei = medium_sample(scene, M, r.o, r.d, remaining, rng_u(r.skey, r.sdim++), r.ch);
-    steps++;
-    if (r.siT < mei.T) mei.T = kInf;
-    float t = fminf(remaining, fminf(mei.T, r.siT)) - mei.minT;
-    if (t >= 0.f) {
-      f3 e = mk(expf(mei.comb.x * -t), expf(mei.comb.y * -t), expf(mei.comb.z * -t));
-      f3 ffp = (r.siT < mei.T || mei.T > remaining) ? e : mul(e, mei.comb);
-      float trPdf = chan(ffp, r.ch);
-      f3 mTr = trPdf > 0.f ? e / trPdf : splat(0.f);
-      r.tr = mul(r.tr, mTr);
-    }
-    if (mei.T > remaining && mei.T != kInf) r.totalDist = r.dist;
-    if (mei.T > remaining) mei.T = kInf;
-    escaped = mei.T == kInf;
-    activeMedium = mei.T != kInf;
-    if (activeMedium) {
-      r.totalDist += mei.T;
-      r.o = mei.p;
-      r.siT = r.siT - mei.T;
-      r.tr = mul(r.tr, mei.sig_n);
-    }
-  }
-  activeSurface = activeSurface || escaped;
-  if (activeSurface) r.totalDist += r.siT;
-  activeSurface = activeSurface && r.hitValid && r.siT != kInf && !activeMedium;
-  int32_t nextMedium = r.medium;
-  if (activeSurface) {
-    const ShapeRec& sr = scene.shapes[r.h.geom];
-    if (sr.bsdf >= 0) r.tr = splat(0.f);
-    // h.t was measured from the origin of the trace that found the hit
-    SurfaceHit si = surface_hit(scene, r.oTrace, r.d, r.h.t, r.h.u, r.h.v, r.h.prim, r.h.geom);
-    r.o = offset_p(si.p, si.n, r.d);
-    if (sr.med_in >= 0 || sr.med_out >= 0) nextMedium = dot(r.d, si.n) > 0.f ? sr.med_out : sr.med_in;
-  }
-  r.needsIntersection = r.needsIntersection || activeSurface;
-  r.medium = nextMedium;
-  return (activeMedium || activeSurface) && !is_zero(r.tr);
+// What a ray does next.  A pass of the reference's while loop is a trace (only
+// when a new straight segment starts), a collision in a medium and the crossing
+// of a surface, each when it applies.
+enum VolShadowState : int { VS_DONE, VS_TRACE, VS_MEDIUM, VS_SURFACE };
+
+__device__ __forceinline__ float vol_shadow_remaining(const VolShadowRay& r) { return r.dist * (1.f - kShadowEps) - r.totalDist; }
+
+__device__ __forceinline__ VolShadowState vol_shadow_pass(const VolShadowRay& r) {
+  if (!(vol_shadow_remaining(r) > 0.f)) return VS_DONE;
+  return r.needsIntersection ? VS_TRACE : VS_MEDIUM;
+}
+// Out of the medium (or never in one): on to the surface the segment ends on.
+__device__ __forceinline__ VolShadowState vol_shadow_leave(VolShadowRay& r) {
+  r.totalDist += r.siT;
+  return r.hitValid && r.siT != kInf ? VS_SURFACE : VS_DONE;
 }
 
+// The reference intersects in the medium branch (vol_path.cpp:258-263) or
+// the surface branch (:316-320), whichever is active, from the same origin
+// and only when a new straight segment starts; one call site serves both.
+__device__ __forceinline__ VolShadowState vol_shadow_trace(const DevScene& scene, VolShadowRay& r) {
+  r.hitValid = trace<false>(scene, r.o, r.d, 0.f, vol_shadow_remaining(r), r.h);
+  r.siT = r.hitValid ? r.h.t : kInf;
+  r.oTrace = r.o;
+  r.needsIntersection = false;
+  return r.medium >= 0 ? VS_MEDIUM : vol_shadow_leave(r);
+}
+
+__device__ __forceinline__ VolShadowState vol_shadow_medium(const DevScene& scene, VolShadowRay& r) {
+  const float remaining = vol_shadow_remaining(r);
+  const MediumRec& M = scene.media[r.medium];
+  MediumSample mei = medium_sample(scene, M, r.o, r.d, remaining, rng_u(r.skey, r.sdim++), r.ch);
+  if (r.siT < mei.T) mei.T = kInf;
+  float t = fminf(remaining, fminf(mei.T, r.siT)) - mei.minT;
+  if (t >= 0.f) {
+    f3 e = mk(expf(mei.comb.x * -t), expf(mei.comb.y * -t), expf(mei.comb.z * -t));
+    f3 ffp = (r.siT < mei.T || mei.T > remaining) ? e : mul(e, mei.comb);
+    float trPdf = chan(ffp, r.ch);
+    f3 mTr = trPdf > 0.f ? e / trPdf : splat(0.f);
+    r.tr = mul(r.tr, mTr);
+  }
+  if (mei.T > remaining && mei.T != kInf) r.totalDist = r.dist;
+  if (mei.T > remaining) mei.T = kInf;
+  if (mei.T == kInf) {
+    const VolShadowState next = vol_shadow_leave(r);
+    return is_zero(r.tr) ? VS_DONE : next;
+  }
+  r.totalDist += mei.T;
+  r.o = mei.p;
+  r.siT = r.siT - mei.T;
+  r.tr = mul(r.tr, mei.sig_n);
+  return is_zero(r.tr) ? VS_DONE : vol_shadow_pass(r);
+}
+
+__device__ __forceinline__ VolShadowState vol_shadow_surface(const DevScene& scene, VolShadowRay& r) {
+  const ShapeRec& sr = scene.shapes[r.h.geom];
+  if (sr.bsdf >= 0) {
+    r.tr = splat(0.f);
+    return VS_DONE;
+  }
+  // h.t was measured from the origin of the trace that found the hit
+  SurfaceHit si = surface_hit(scene, r.oTrace, r.d, r.h.t, r.h.u, r.h.v, r.h.prim, r.h.geom);
+  r.o = offset_p(si.p, si.n, r.d);
+  if (sr.med_in >= 0 || sr.med_out >= 0) r.medium = dot(r.d, si.n) > 0.f ? sr.med_out : sr.med_in;
+  r.needsIntersection = true;
+  return vol_shadow_pass(r);
+}
+
+// A wave runs, step by step, whatever most of its lanes wait for: taking new
+// rays, tracing, a collision or a surface.  With every lane running its whole
+// pass, a quarter of the lanes were active on average (volume frame 44.7 ms in
+// this kernel, now 28.1).
 __global__ void __launch_bounds__(kTraceBlock) k_vol_shadow(Wavefront w, DevScene scene) {
-  __shared__ uint32_t lds[32];
+  __shared__ uint32_t lds[32], used_up;
   const uint32_t n = w.cnt[CNT_SHADOW];
-  uint32_t* fetch = &w.cnt[CNT_FETCH_SH];
-  constexpr uint32_t kChunk = 256;  // queue entries a wave takes with one atomic
   const uint32_t lane = __lane_id();
-  const unsigned long long below = (1ull << lane) - 1ull;
+  const uint32_t wave = blockIdx.x * (kTraceBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t waves = min(gridDim.x * (kTraceBlock / 64), kVolShadowWaves);
+  if (threadIdx.x == 0) used_up = 0u;
+  __syncthreads();
+  uint32_t share, chunk;
+  deal_shares(n, waves, share, chunk);
+  ItemDealer items;
+  items.start(n, &w.cnt[CNT_FETCH_SH], (lds_u32*)&used_up, wave, waves, share, chunk);
   VolShadowRay r;
-  bool active = false, exhausted = false;
-  // the wave's first chunk is its own by position: a launch with little work
-  // costs no atomics (about 11 ns each on one counter)
-  const uint32_t wave = blockIdx.x * (kTraceBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
-                 waves = gridDim.x * (kTraceBlock / 64);
-  uint32_t cbase = wave * kChunk, cleft = cbase < n ? min(kChunk, n - cbase) : 0u, steps = 0, guard = 0;
-  exhausted = static_cast<unsigned long long>(waves) * kChunk >= n;
+  bool have = false;
+  VolShadowState state = VS_DONE;
+  uint32_t steps = 0, guard = 0;
   for (;;) {
-    const unsigned long long need = __ballot(!active);
-    if (need && (!exhausted || cleft > 0)) {
-      const uint32_t want = (uint32_t)__popcll(need);
-      const uint32_t rank = (uint32_t)__popcll(need & below);
-      uint32_t nbase = 0, nleft = 0;
-      if (cleft < want && !exhausted) {
-        uint32_t b = 0;
-        if (lane == 0) b = atomicAdd(fetch, kChunk);
-        b = __builtin_amdgcn_readfirstlane(b) + waves * kChunk;
-        if (b >= n) {
-          exhausted = true;
-        } else {
-          nbase = b;
-          nleft = min(kChunk, n - b);
-          if (b + kChunk >= n) exhausted = true;
-        }
-      }
-      uint32_t i = 0xffffffffu;
-      if (rank < cleft)
-        i = cbase + rank;
-      else if (rank - cleft < nleft)
-        i = nbase + (rank - cleft);
-      const uint32_t fromOld = min(want, cleft);
-      cbase += fromOld;
-      cleft -= fromOld;
-      if (nleft) {
-        const uint32_t fromNew = min(want - fromOld, nleft);
-        cbase = nbase + fromNew;
-        cleft = nleft - fromNew;
-      }
-      if (!active && i < n) {
-        vol_shadow_begin(w, i, r);
-        active = true;
-        guard = 0;
-      }
-    }
-    if (__ballot(active) == 0ull) {
-      if (exhausted && cleft == 0) break;
-      continue;
-    }
-    if (active) {
-      // the guard bounds a walk that no longer moves (finite distances end)
-      if (!vol_shadow_step(scene, r, steps) || ++guard >= 100000) {
+    const uint32_t nTrace = (uint32_t)__popcll(__ballot(have && state == VS_TRACE));
+    const uint32_t nMedium = (uint32_t)__popcll(__ballot(have && state == VS_MEDIUM));
+    const uint32_t nSurface = (uint32_t)__popcll(__ballot(have && state == VS_SURFACE));
+    const uint32_t most = max(nTrace, max(nMedium, nSurface));
+    const uint32_t free = 64u - nTrace - nMedium - nSurface;
+    if (most == 0 || (items.more() && free >= min(most, kVolShadowRefill))) {
+      if (have && state == VS_DONE) {
         if (!is_zero(r.tr)) {
           const float4 l = w.lsum[r.s];
           w.lsum[r.s] = make_float4(l.x + r.c.x * r.tr.x, l.y + r.c.y * r.tr.y, l.z + r.c.z * r.tr.z, l.w);
         }
-        active = false;
+        have = false;
       }
+      if (!items.more()) {
+        if (most == 0) break;
+        continue;
+      }
+      const unsigned long long need = __ballot(!have);
+      const uint32_t i = items.take(need, lane);
+      if (!have && i < n) {
+        vol_shadow_begin(w, i, r);
+        have = true;
+        state = vol_shadow_pass(r);
+        guard = 0;
+      }
+      continue;
+    }
+    if (nTrace == most) {
+      if (have && state == VS_TRACE) state = vol_shadow_trace(scene, r);
+    } else if (nMedium == most) {
+      if (have && state == VS_MEDIUM) {
+        state = vol_shadow_medium(scene, r);
+        steps++;
+        if (++guard >= 100000) state = VS_DONE;  // bounds a walk that no longer moves (finite distances end)
+      }
+    } else if (have && state == VS_SURFACE) {
+      state = vol_shadow_surface(scene, r);
+      if (++guard >= 100000) state = VS_DONE;
     }
   }
   block_count(&w.stats[ST_MEDIUM], steps, lds);
