@@ -668,9 +668,7 @@ rad_status rad_hip_render_start(rad_scene* scene, const rad_render_desc* desc, r
   *out = nullptr;
   return Guard([&] {
     RequireBvh(scene);
-    rad_render_desc d = *desc;
-    ResolveLaunch(scene, d);
-    *out = StartJob(scene, d, TakeSpareArena(scene));
+    *out = StartRender(scene, *desc);
   });
 }
 

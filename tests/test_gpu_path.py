@@ -265,3 +265,25 @@ def test_material_queues_are_a_permutation(hip_ctx, monkeypatch, budget):
     # the unsorted kernel has no material queues: nothing is checked
     _, _, un = s.render(b.render_desc(spp=8, seed=5, flags=F.RAD_RENDER_CHECK_QUEUES | F.RAD_RENDER_UNSORTED))
     assert un.queue_checked == 0
+
+
+@pytest.mark.parametrize("size,spp,guiding,slots", [
+    ((512, 512), 80, 0, 16 << 20),  # 21 M samples: more than the slots
+    ((512, 512), 20, 0, 512 * 512 * 20),
+    ((100, 33), 2, 0, 6600),
+    ((512, 512), 20, 1, 4 << 20),  # online training keeps its records' slots
+])
+def test_slots_chosen_by_the_library(hip_ctx, size, spp, guiding, slots):
+    """The slots of a render that leaves them to the library, on a fresh scene
+    and with its spare arena; the image is the one of any other number."""
+    b = scenes.many_balls(seed=0, width=size[0], height=size[1], spp=spp, n_spheres=8)
+    s = hip.Scene.from_builder(hip_ctx, b)
+    d = b.render_desc(spp=spp, seed=3, guiding=guiding)
+    a, _, st = s.render(d)
+    assert st.slots == slots
+    if guiding:
+        return
+    c, _, st = s.render(d)
+    assert st.slots == slots and np.array_equal(a, c)
+    e, _, st = s.render(b.render_desc(spp=spp, seed=3, path_slots=1 << 20))
+    assert st.slots == min(1 << 20, size[0] * size[1] * spp) and np.array_equal(a, e)
