@@ -53,19 +53,39 @@ __global__ void __launch_bounds__(256) k_guide_infer(GuideNet net, const float* 
 // gradient), so large sample weights stay inside the FP16 range.
 constexpr float kDzScale = 1.f / 32.f;
 
-// Lobe l points from the vertex p to the target c + h * (raw means).
-__device__ inline float record_loss_grad(const float* raw, f3 dir, float wn, f3 p, f3 cen, f3 half, float* d) {
-  float a[kLobes], logv[kLobes], kap[kLobes], c[kLobes], len[kLobes];
-  f3 mu[kLobes];
-  bool kin[kLobes];
+// Reductions over the four lanes of a record (v, v + 16, v + 32, v + 48).
+__device__ __forceinline__ float record_max(float x) {
+  x = fmaxf(x, __shfl_xor(x, 16));
+  return fmaxf(x, __shfl_xor(x, 32));
+}
+__device__ __forceinline__ float record_sum(float x) {
+  x += __shfl_xor(x, 16);
+  return x + __shfl_xor(x, 32);
+}
+
+// Lobe l points from the vertex p to the target c + h * (raw means).  Lane
+// group g of a record's four has the lobes 2 g and 2 g + 1 (raw and d: their
+// outputs); the loss is the same in all four.
+__device__ __forceinline__ float record_loss_grad(const float* raw, f3 dir, float wn, f3 p, f3 cen, f3 half,
+                                                  float d[2 * kRawPerLobe]) {
+  constexpr int N = kLobes / 4;
+  float a[N], logv[N], kap[N], c[N], len[N], lp[N];
+  f3 mu[N];
+  bool kin[N];
   float mx = -kInf;
-  for (int l = 0; l < kLobes; l++) mx = fmaxf(mx, raw[kRawPerLobe * l]);
+#pragma unroll
+  for (int l = 0; l < N; l++) mx = fmaxf(mx, raw[kRawPerLobe * l]);
+  mx = record_max(mx);
   float se = 0.f;
-  for (int l = 0; l < kLobes; l++) {
+#pragma unroll
+  for (int l = 0; l < N; l++) {
     a[l] = expf(raw[kRawPerLobe * l] - mx);
     se += a[l];
   }
-  for (int l = 0; l < kLobes; l++) {
+  se = record_sum(se);
+  float lm = -kInf;
+#pragma unroll
+  for (int l = 0; l < N; l++) {
     a[l] /= se;  // pi_l
     f3 m = lobe_vector(raw + kRawPerLobe * l, p, cen, half);
     len[l] = sqrtf(sqnorm(m));
@@ -75,14 +95,17 @@ __device__ inline float record_loss_grad(const float* raw, f3 dir, float wn, f3 
     kap[l] = expf(fminf(fmaxf(kr, -3.f), 6.f));
     c[l] = dot(mu[l], dir);
     logv[l] = logf(kap[l]) - logf(2.f * kPi) - log1pf(-expf(-2.f * kap[l])) + kap[l] * (c[l] - 1.f);
+    lp[l] = logf(a[l]) + logv[l];
+    lm = fmaxf(lm, lp[l]);
   }
-  float lm = -kInf;
-  for (int l = 0; l < kLobes; l++) lm = fmaxf(lm, logf(a[l]) + logv[l]);
+  lm = record_max(lm);
   float s = 0.f;
-  for (int l = 0; l < kLobes; l++) s += expf(logf(a[l]) + logv[l] - lm);
-  float logq = lm + logf(s);
-  for (int l = 0; l < kLobes; l++) {
-    float r = expf(logf(a[l]) + logv[l] - logq);
+#pragma unroll
+  for (int l = 0; l < N; l++) s += expf(lp[l] - lm);
+  float logq = lm + logf(record_sum(s));
+#pragma unroll
+  for (int l = 0; l < N; l++) {
+    float r = expf(lp[l] - logq);
     float k = kap[l];
     d[kRawPerLobe * l] = -wn * (r - a[l]);
     float e = expf(-2.f * k);
@@ -97,144 +120,210 @@ __device__ inline float record_loss_grad(const float* raw, f3 dir, float wn, f3 
   return -wn * logq;
 }
 
-// One training step over 64 records per block (4 waves x 16).  Gradients
-// (summed over records, not yet divided by the batch size) are added to
-// grad[kParams]; the summed loss to *loss.
-__global__ void __launch_bounds__(256) k_guide_train(GuideNet net, const TrainRecord* recs, const uint32_t* batch,
-                                                     uint32_t B, float wnorm, float wmax, float* grad, float* loss) {
+// Gradients of tiles of 64 records (4 waves x 16), summed over the records but
+// not yet divided by the batch size: row blockIdx.x of `partial` (kTrainRow
+// floats: the parameters, then the loss), which k_guide_train_sum adds up.
+//
+// The matrix products (4 GFLOP at 32768 records) are 5 us of the matrix cores; the
+// kernel is bound by the chain of its phases (LDS operands, the loss, barriers)
+// with one wave per SIMD, as the weights (both operand orders) and the
+// activations of a tile fill the LDS.  So every matrix operand is stored in
+// the order in which the lanes read it, one conflict-free 8-byte read each;
+// the four lanes of a record share its lobes; and the gradient of a block's
+// tiles stays in registers (100 per lane) and is written once: 512 blocks that
+// added their tile's 20.6 K values to one gradient atomically, after operand
+// reads from rows of 128 bytes (8 lanes to a bank), took 115 us at 32768
+// records; now 37 us, and 5 us for the sum of the rows.
+constexpr int kTrainRow = (kParams + 1 + 63) / 64 * 64;
+constexpr uint32_t kTrainBlocks = 256;  // one per CU
+
+// Place of (feature f of the 16 of tile ft, record r of the 16 of wave rt) in
+// an LDS array of operands: 16x16 tiles, 4 records of a lane together.
+__device__ __forceinline__ int train_frag(int ft, int rt, int f, int r) {
+  return (ft * 4 + rt) * 256 + ((r >> 2) * 16 + f) * 4 + (r & 3);
+}
+
+// acc += the product of two operands over the 64 records.
+__device__ __forceinline__ void train_outer(const h4 a[4], const h4 b[4], f4v& acc) {
+#pragma unroll
+  for (int kc = 0; kc < 4; kc++) acc = mfma16(a[kc], b[kc], acc);
+}
+__device__ __forceinline__ void train_operand(const _Float16* tile, int lane, h4 x[4]) {
+#pragma unroll
+  for (int kc = 0; kc < 4; kc++) x[kc] = *reinterpret_cast<const h4*>(tile + kc * 256 + 4 * lane);
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+k_guide_train(GuideNet net, const TrainRecord* recs, const uint32_t* batch, uint32_t B, float wnorm, float wmax,
+              float* partial) {
   __shared__ __align__(16) _Float16 sW[kWeights];
+  __shared__ __align__(16) _Float16 sWt[kBackWeights];
   __shared__ float sB[kBiases];
-  __shared__ __align__(16) _Float16 sAct[kIn * 64 + 4 * kHid * 64];   // layer inputs A_0..A_4, [feature][record]
-  __shared__ __align__(16) _Float16 sDz[4 * kHid * 64 + kOut * 64];   // output gradients dZ_0..dZ_4, [feature][record]
-  __shared__ float sOut[64 * kOut];                     // raw outputs, [record][output]
-  load_weights_lds(sW, sB, net.w, net.b);
-  __syncthreads();
+  __shared__ __align__(16) _Float16 sAct[(kIn + 4 * kHid) * 64];  // layer inputs A_0..A_4 (train_frag)
+  __shared__ __align__(16) _Float16 sDz[(4 * kHid + kOut) * 64];  // output gradients dZ_0..dZ_4 (train_frag)
+  __shared__ float sLoss[4];
+  constexpr int kOutStride = kOut + 1;
+  float* const sOut = reinterpret_cast<float*>(sDz);  // raw outputs [record][output], in the place of dZ_0 and dZ_1
+  static_assert(64 * kOutStride * 4 <= 2 * kHid * 64 * 2, "raw outputs overlap dZ_4");
+  load_weights_lds_train(sW, sWt, sB, net.w, net.b);
   const int lane = __lane_id();
   const int v = lane & 15, g = lane >> 4;
-  const int wave = threadIdx.x >> 6;
-  const int rloc = 16 * wave + v;  // record within the block
-  const uint32_t ridx = blockIdx.x * 64 + rloc;
-  const bool valid = ridx < B;
-  TrainRecord rec{};
-  if (valid) rec = recs[batch ? batch[ridx] : ridx];
-  float f9[kFeat] = {rec.p[0], rec.p[1], rec.p[2], rec.n[0], rec.n[1], rec.n[2], rec.wi[0], rec.wi[1], rec.wi[2]};
-  FeatScalars fs = feat_scalars(f9, net.lo, net.inv_ext);
-  h4 act[4][4];
-  f4v out[3];
-  forward_tile<false>(sW, sB, fs, act, out, nullptr);
-  auto actOff = [](int l) { return l == 0 ? 0 : kIn * 64 + (l - 1) * kHid * 64; };
-  auto dzOff = [](int l) { return l * kHid * 64; };
-  // layer inputs to LDS: X (recomputed one-blob values) and hidden activations
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto act_tile = [&](int l, int ft) { return sAct + ((l == 0 ? 0 : kIn / 16 + (l - 1) * (kHid / 16)) + ft) * 1024; };
+  auto dz_tile = [&](int l, int ft) { return sDz + (l * (kHid / 16) + ft) * 1024; };
+  const h4 ones = h4{1, 1, 1, 1};
+  const f4v zero = f4v{0.f, 0.f, 0.f, 0.f};
+  // wave w's weight gradient tiles: layer 0 (to = w, ti = i), layers 1..4 (to = i, ti = w)
+  f4v g0[5], gh[3][4], g4[3], gb[kLayers];
 #pragma unroll
-  for (int c = 0; c < kIn / 16; c++)
+  for (int i = 0; i < 5; i++) g0[i] = gb[i] = zero;
 #pragma unroll
-    for (int j = 0; j < 4; j++) sAct[actOff(0) + (16 * c + 4 * g + j) * 64 + rloc] = (_Float16)one_blob(fs, c, 4 * g + j);
+  for (int i = 0; i < 12; i++) gh[i / 4][i % 4] = zero;
 #pragma unroll
-  for (int l = 0; l < 4; l++)
+  for (int i = 0; i < 3; i++) g4[i] = zero;
+  float loss = 0.f;
+  const uint32_t tiles = (B + 63) / 64;
+  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const uint32_t ridx = tile * 64 + 16 * wave + v;
+    const bool valid = ridx < B;
+    TrainRecord rec{};
+    if (valid) rec = recs[batch ? batch[ridx] : ridx];
+    __syncthreads();  // weights loaded; the previous tile's operands read
+    float f9[kFeat] = {rec.p[0], rec.p[1], rec.p[2], rec.n[0], rec.n[1], rec.n[2], rec.wi[0], rec.wi[1], rec.wi[2]};
+    FeatScalars fs = feat_scalars(f9, net.lo, net.inv_ext);
+    h4 act[4][4], xs[kIn / 16];
+    {
+      f4v out[3];
+      forward_tile(sW, sB, fs, act, out, xs);
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+      for (int t = 0; t < 3; t++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) sAct[actOff(l + 1) + (16 * t + 4 * g + j) * 64 + rloc] = act[l][t][j];
+        for (int j = 0; j < 4; j++) sOut[(16 * wave + v) * kOutStride + 16 * t + 4 * g + j] = out[t][j];
+    }
 #pragma unroll
-  for (int t = 0; t < 3; t++)
+    for (int c = 0; c < kIn / 16; c++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) sOut[rloc * kOut + 16 * t + 4 * g + j] = out[t][j];
+      for (int j = 0; j < 4; j++) act_tile(0, 0)[train_frag(c, wave, 4 * g + j, v)] = xs[c][j];
+#pragma unroll
+    for (int l = 0; l < 4; l++)
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) act_tile(l + 1, 0)[train_frag(t, wave, 4 * g + j, v)] = act[l][t][j];
+    __syncthreads();
+    {
+      const float* raw = sOut + (16 * wave + v) * kOutStride + 2 * kRawPerLobe * g;
+      const bool used = valid && rec.w > 0.f;
+      const float wn = fminf(rec.w * wnorm, wmax);
+      float d[2 * kRawPerLobe];
+      const float l = record_loss_grad(raw, mk(rec.dir[0], rec.dir[1], rec.dir[2]), wn, mk(rec.p[0], rec.p[1], rec.p[2]),
+                                       mk(net.center[0], net.center[1], net.center[2]),
+                                       mk(net.half[0], net.half[1], net.half[2]), d);
+      if (used && g == 0) loss += l;
+#pragma unroll
+      for (int k = 0; k < 2 * kRawPerLobe; k++) {
+        const int o = 2 * kRawPerLobe * g + k;
+        dz_tile(4, 0)[train_frag(o >> 4, wave, o & 15, v)] = used ? (_Float16)(d[k] * kDzScale) : (_Float16)0.f;
+      }
+#pragma unroll
+      for (int k = 0; k < (kOut - kLobes * kRawPerLobe) / 4; k++)  // padding outputs
+        dz_tile(4, 0)[train_frag(2, wave, 8 + 2 * g + k, v)] = (_Float16)0.f;
+    }
+    __syncthreads();  // raw outputs read; dZ_4 written
+    // backward through the hidden layers of this wave's 16 records
+    h4 dz[4];  // dZ of the layer above, in B-operand form
+#pragma unroll
+    for (int l = 4; l >= 1; l--) {
+      __builtin_amdgcn_sched_barrier(0);  // keep each layer's weight loads inside the layer
+      f4v acc[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) acc[t] = zero;
+#pragma unroll
+      for (int c = 0; c < LayerOut(l) / 16; c++) {
+        h4 b = dz[c];
+        if (l == 4) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) b[j] = dz_tile(4, 0)[train_frag(c, wave, 4 * g + j, v)];
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+          acc[t] = mfma16(*reinterpret_cast<const h4*>(sWt + back_frag_base(l, t, c) + 4 * lane), b, acc[t]);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          _Float16 x = act[l - 1][t][j] > (_Float16)0.f ? (_Float16)acc[t][j] : (_Float16)0.f;
+          dz[t][j] = x;
+          dz_tile(l - 1, 0)[train_frag(t, wave, 4 * g + j, v)] = x;
+        }
+    }
+    __syncthreads();
+    // weight gradients: dW_l[out][in] = sum over the 64 records of dZ_l[out] A_l[in]
+    h4 a[4], b[4];
+    train_operand(dz_tile(0, wave), lane, a);
+#pragma unroll
+    for (int kc = 0; kc < 4; kc++) gb[0] = mfma16(a[kc], ones, gb[0]);
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+      train_operand(act_tile(0, i), lane, b);
+      train_outer(a, b, g0[i]);
+    }
+#pragma unroll
+    for (int l = 1; l < kLayers; l++) {
+      train_operand(act_tile(l, wave), lane, b);
+#pragma unroll
+      for (int i = 0; i < LayerOut(l) / 16; i++) {
+        train_operand(dz_tile(l, i), lane, a);
+        train_outer(a, b, l < 4 ? gh[l - 1][i] : g4[i]);
+        if (i == wave) {
+#pragma unroll
+          for (int kc = 0; kc < 4; kc++) gb[l] = mfma16(a[kc], ones, gb[l]);
+        }
+      }
+    }
+  }
+  float* const row = partial + size_t(blockIdx.x) * kTrainRow;
+  auto put = [&](int l, int to, int ti, f4v x) {
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      row[WeightOffset(l) + (16 * to + 4 * g + j) * LayerIn(l) + 16 * ti + v] = x[j] * (1.f / kDzScale);
+  };
+#pragma unroll
+  for (int i = 0; i < 5; i++) put(0, wave, i, g0[i]);
+#pragma unroll
+  for (int l = 1; l < kLayers; l++)
+#pragma unroll
+    for (int i = 0; i < LayerOut(l) / 16; i++) put(l, i, wave, l < 4 ? gh[l - 1][i] : g4[i]);
+#pragma unroll
+  for (int l = 0; l < kLayers; l++)
+    if (v == 0 && 16 * wave < LayerOut(l)) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) row[BiasOffset(l) + 16 * wave + 4 * g + j] = gb[l][j] * (1.f / kDzScale);
+    }
+#pragma unroll
+  for (int k = 32; k > 0; k >>= 1) loss += __shfl_xor(loss, k);
+  if (lane == 0) sLoss[wave] = loss;
   __syncthreads();
-  // loss and output gradients: one lane per record
-  if (g == 0) {
-    float d[kOut];
-    for (int k = 0; k < kOut; k++) d[k] = 0.f;
-    float l = 0.f;
-    if (valid && rec.w > 0.f) {
-      float wn = fminf(rec.w * wnorm, wmax);
-      l = record_loss_grad(sOut + rloc * kOut, mk(rec.dir[0], rec.dir[1], rec.dir[2]), wn,
-                           mk(rec.p[0], rec.p[1], rec.p[2]), mk(net.center[0], net.center[1], net.center[2]),
-                           mk(net.half[0], net.half[1], net.half[2]), d);
-    }
-    for (int k = 0; k < kOut; k++) sDz[dzOff(4) + k * 64 + rloc] = (_Float16)(d[k] * kDzScale);
-    if (l != 0.f) atomicAdd(loss, l);
-  }
+  if (threadIdx.x == 0) row[kParams] = sLoss[0] + sLoss[1] + sLoss[2] + sLoss[3];
+}
+
+// grad += the sum of the partial rows, *loss += that of their losses.
+__global__ void __launch_bounds__(256) k_guide_train_sum(const float* partial, uint32_t rows, float* grad, float* loss) {
+  __shared__ float part[4][64];
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t i = blockIdx.x * 64 + lane;  // the rows are padded to a multiple of 64
+  float s = 0.f;
+#pragma unroll 8
+  for (uint32_t r = wave; r < rows; r += 4) s += partial[size_t(r) * kTrainRow + i];
+  part[wave][lane] = s;
   __syncthreads();
-  // backward through the hidden layers of this wave's tile
-  h4 dz[4];  // dZ of the layer above, in B-operand form
-  {
-    f4v acc[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++) acc[t] = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      h4 b;
-#pragma unroll
-      for (int j = 0; j < 4; j++) b[j] = sDz[dzOff(4) + (16 * c + 4 * g + j) * 64 + rloc];
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        h4 a;
-#pragma unroll
-        for (int j = 0; j < 4; j++) a[j] = sW[HalfOffset(4) + (16 * c + 4 * g + j) * kHid + 16 * t + v];
-        acc[t] = mfma16(a, b, acc[t]);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        _Float16 x = act[3][t][j] > (_Float16)0.f ? (_Float16)acc[t][j] : (_Float16)0.f;
-        dz[t][j] = x;
-        sDz[dzOff(3) + (16 * t + 4 * g + j) * 64 + rloc] = x;
-      }
-  }
-#pragma unroll
-  for (int l = 3; l >= 1; l--) {
-    f4v acc[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++) acc[t] = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        h4 a;
-#pragma unroll
-        for (int j = 0; j < 4; j++) a[j] = sW[HalfOffset(l) + (16 * c + 4 * g + j) * kHid + 16 * t + v];
-        acc[t] = mfma16(a, dz[c], acc[t]);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        _Float16 x = act[l - 1][t][j] > (_Float16)0.f ? (_Float16)acc[t][j] : (_Float16)0.f;
-        dz[t][j] = x;
-        sDz[dzOff(l - 1) + (16 * t + 4 * g + j) * 64 + rloc] = x;
-      }
-  }
-  __syncthreads();
-  // weight gradients: dW_l[out][in] = sum over the block's 64 records of dZ_l[out] A_l[in]
-  int k = 0;
-  for (int l = 0; l < kLayers; l++) {
-    const int nin = LayerIn(l), nout = LayerOut(l);
-    const int ti_n = nin / 16, to_n = nout / 16;
-    for (int tile = 0; tile < ti_n * to_n; tile++, k++) {
-      if ((k & 3) != wave) continue;
-      const int to = tile / ti_n, ti = tile % ti_n;
-      f4v acc = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kc = 0; kc < 4; kc++) {
-        h4 a = *reinterpret_cast<const h4*>(sDz + dzOff(l) + (16 * to + v) * 64 + 16 * kc + 4 * g);
-        h4 b = *reinterpret_cast<const h4*>(sAct + actOff(l) + (16 * ti + v) * 64 + 16 * kc + 4 * g);
-        acc = mfma16(a, b, acc);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        float x = acc[j];
-        if (x != 0.f) atomicAdd(&grad[WeightOffset(l) + (16 * to + 4 * g + j) * nin + 16 * ti + v], x * (1.f / kDzScale));
-      }
-    }
-    for (int o = threadIdx.x; o < nout; o += blockDim.x) {
-      float sacc = 0.f;
-      for (int r = 0; r < 64; r++) sacc += float(sDz[dzOff(l) + o * 64 + r]);
-      if (sacc != 0.f) atomicAdd(&grad[BiasOffset(l) + o], sacc * (1.f / kDzScale));
-    }
-  }
+  if (wave != 0 || i > uint32_t(kParams)) return;
+  s = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+  if (i < uint32_t(kParams))
+    grad[i] += s;
+  else
+    *loss += s;
 }
 
 // Adam on the FP32 master weights; refreshes the FP16 / bias copies the
@@ -379,10 +468,14 @@ void LaunchInfer(const GuideNet& net, const float* feats, const uint32_t* n_dev,
   hipLaunchKernelGGL(k_guide_infer, dim3(blocks), dim3(256), 0, s, net, feats, n_dev, n_host, slot_of, raw);
 }
 
+size_t TrainWorkBytes(uint32_t B) { return size_t(std::min((B + 63) / 64, kTrainBlocks)) * kTrainRow * 4; }
+
 void LaunchTrain(const GuideNet& net, const TrainRecord* recs, const uint32_t* batch, uint32_t B, float wnorm, float wmax,
-                 float* grad, float* loss, hipStream_t s) {
-  if (B)
-    hipLaunchKernelGGL(k_guide_train, dim3((B + 63) / 64), dim3(256), 0, s, net, recs, batch, B, wnorm, wmax, grad, loss);
+                 float* work, float* grad, float* loss, hipStream_t s) {
+  if (B == 0) return;
+  const uint32_t rows = std::min((B + 63) / 64, kTrainBlocks);
+  hipLaunchKernelGGL(k_guide_train, dim3(rows), dim3(256), 0, s, net, recs, batch, B, wnorm, wmax, work);
+  hipLaunchKernelGGL(k_guide_train_sum, dim3(kTrainRow / 64), dim3(256), 0, s, work, rows, grad, loss);
 }
 
 void GuideState::Step(float lr, float gscale, hipStream_t s) {
@@ -474,11 +567,12 @@ rad_status rad_hip_guide_grad(const float* params, const float* bounds, const ra
     GuideState st;
     st.Upload(std::vector<float>(params, params + kParams));
     GuideNet net = st.Net(bounds, bounds + 3, 0.5f);
-    DeviceBuffer dr;
+    DeviceBuffer dr, work;
     dr.alloc(std::max<size_t>(16, size_t(n) * sizeof(TrainRecord)));
+    work.alloc(TrainWorkBytes(n));
     HipCheck(hipMemcpy(dr.ptr, recs, size_t(n) * sizeof(TrainRecord), hipMemcpyHostToDevice), "copy records");
     HipCheck(hipMemset(st.scal.ptr, 0, 4), "clear loss");
-    LaunchTrain(net, dr.as<TrainRecord>(), nullptr, n, wnorm, 64.f, st.grad.as<float>(), st.scal.as<float>(), nullptr);
+    LaunchTrain(net, dr.as<TrainRecord>(), nullptr, n, wnorm, 64.f, work.as<float>(), st.grad.as<float>(), st.scal.as<float>(), nullptr);
     HipCheck(hipGetLastError(), "guide train launch");
     HipCheck(hipMemcpy(grad, st.grad.ptr, kParams * 4, hipMemcpyDeviceToHost), "copy gradient");
     float l = 0.f;

@@ -13,6 +13,7 @@ namespace guide {
 
 struct GuideState {
   DeviceBuffer params, grad, m1, m2, wh, bias, scal;
+  DeviceBuffer train_work;  // of the training kernel, allocated by the first training pass
   // The FP16 weights and biases as of the last finished training pass (or
   // upload): renders that only read the guide copy these under pub_mu, so a
   // training render on another stream never hands them a half-updated net.
@@ -31,8 +32,10 @@ struct GuideState {
 void InitParams(std::vector<float>& p, uint32_t seed);
 void LaunchInfer(const GuideNet& net, const float* feats, const uint32_t* n_dev, uint32_t n_host, const uint32_t* slot_of,
                  _Float16* raw, int blocks, hipStream_t s);
+// work: TrainWorkBytes(B) bytes.
+size_t TrainWorkBytes(uint32_t B);
 void LaunchTrain(const GuideNet& net, const TrainRecord* recs, const uint32_t* batch, uint32_t B, float wnorm, float wmax,
-                 float* grad, float* loss, hipStream_t s);
+                 float* work, float* grad, float* loss, hipStream_t s);
 void LaunchBatch(uint32_t* batch, uint32_t B, uint32_t n, uint32_t seed, hipStream_t s);
 void LaunchPdf(const float* raw, const float* dirs, uint32_t n, float* pdf, hipStream_t s);
 void LaunchSample(const float* raw, const float* xi, uint32_t n, float* out, hipStream_t s);

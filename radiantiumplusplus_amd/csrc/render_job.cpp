@@ -211,10 +211,11 @@ void Train(rad_job* job, hipStream_t st) {
     const uint32_t steps = TrainSteps();
     const float lr = TrainLr();
     const float wmax = TrainWmax();
+    gs.train_work.alloc(guide::TrainWorkBytes(kTrainBatch));
     for (uint32_t k = 0; k < steps; k++) {
       HipCheck(hipMemsetAsync(gs.scal.ptr, 0, 4, st), "clear loss");
       guide::LaunchBatch(job->batch, kTrainBatch, nrec, gs.steps * 7919u + k + 1u, st);
-      guide::LaunchTrain(net, w.recs, job->batch, kTrainBatch, wnorm, wmax, gs.grad.as<float>(), gs.scal.as<float>(), st);
+      guide::LaunchTrain(net, w.recs, job->batch, kTrainBatch, wnorm, wmax, gs.train_work.as<float>(), gs.grad.as<float>(), gs.scal.as<float>(), st);
       gs.Step(lr, 1.f / float(kTrainBatch), st);
     }
     HipCheck(hipGetLastError(), "guide training launch");

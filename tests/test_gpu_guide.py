@@ -130,6 +130,33 @@ def test_gradient_with_cancelling_records(hip_ctx):
     assert max(errs16) < 3e-2, errs16
 
 
+@pytest.mark.parametrize("n,m", [(1, 64), (63, 65), (64, 1000), (65, 16384), (1000, 16385), (16384, 33000), (16385, 16448)])
+def test_gradient_does_not_depend_on_places(hip_ctx, n, m):
+    """n records, and the same records at random places among m - n of weight
+    zero: other lanes, waves, tiles and blocks.  The records' gradients share a
+    direction, so the two sums differ by their at most 128 roundings of 2^-24."""
+    rng = np.random.default_rng(n)
+    recs = np.zeros(m, np.dtype([("p", "<f4", 3), ("n", "<f4", 3), ("wi", "<f4", 3), ("dir", "<f4", 3),
+                                 ("thr", "<f4", 3), ("lbase", "<f4", 3), ("w", "<f4"), ("prev", "<u4")]))
+    feats = random_feats(rng, m)
+    recs["p"], recs["n"], recs["wi"] = feats[:, 0:3], feats[:, 3:6], feats[:, 6:9]
+    dirs = np.array([0.3, 0.8, -0.5]) + 0.2 * rng.normal(size=(m, 3))
+    recs["dir"] = dirs / np.linalg.norm(dirs, axis=1, keepdims=True)
+    recs["w"][:n] = rng.uniform(0.5, 1.5, n)
+    p, bounds = random_params(3), np.concatenate([LO, HI]).astype(np.float32)
+    out = []
+    for r in (recs[:n].copy(), rng.permutation(recs)):
+        grad, loss = np.zeros(F.RAD_GUIDE_PARAMS, np.float32), C.c_float()
+        hip.check(hip.lib().rad_hip_guide_grad(_fp(p), _fp(bounds), r.ctypes.data_as(C.c_void_p), len(r), C.c_float(1.0),
+                                               _fp(grad), C.byref(loss)))
+        out.append((grad.astype(np.float64) * len(r), loss.value * len(r)))
+    assert out[0][1] != 0 and abs(out[0][1] - out[1][1]) <= 1e-5 * abs(out[0][1])
+    for (wo, bo), (nin, nout) in zip(G.OFFS, G.DIMS):
+        for lo_, hi_ in ((wo, bo), (bo, bo + nout)):
+            a, b = out[0][0][lo_:hi_], out[1][0][lo_:hi_]
+            assert np.linalg.norm(a) > 0 and np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(a)
+
+
 def test_mixture_probes(hip_ctx):
     rng = np.random.default_rng(4)
     raw = rng.normal(size=48).astype(np.float32)
