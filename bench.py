@@ -131,7 +131,7 @@ def summarize(dirs, copy_mib=1024):
         rd = sum(f[k]) / len(f[k]) * f_scale * 1024 / 1e6
         wr = sum(w[k]) / len(w[k]) * w_scale * 1024 / 1e6
         out.append(f"{k[:W]:{W}s} {len(f[k]):10d} {rd:15.1f} {wr:16.1f}")
-    ext = [k for k in f if k.endswith("k_extend")]
+    ext = [k for k in f if k.split("<")[0].endswith("k_extend")]
     if ext and ext[0] in w:
         k = ext[0]
         line = json.loads(open(pmc_json).read().strip().splitlines()[-1])
@@ -604,7 +604,7 @@ def main():
             "valu_busy": _profile_tag(VALU_TAG),
             "valu_note": "fraction of SIMD cycles issuing VALU instructions in k_extend (SQ_ACTIVE_INST_VALU, "
                          "GRBM_GUI_ACTIVE in profiles/k_extend_large_mesh.txt): the kernel is bound by instruction "
-                         "issue, not by HBM bandwidth",
+                         "issue and the latency of its node reads, not by HBM bandwidth",
             "launch": {"path_slots": stats[0].slots, "blocks_per_cu": stats[0].blocks_per_cu,
                        "trace_blocks_per_cu": stats[0].trace_blocks_per_cu},
             "rays_per_s": segs / (ext_ms * 1e-3) if ext_ms > 0 else 0.0,

@@ -4,8 +4,7 @@
 //    the starting order, so neighbouring lanes hold nearby primitives.
 // 2. Top-down, one level of nodes at a time over the whole GPU.  A node
 //    with more than kSmall primitives is split by binned SAH: 16 centroid
-//    bins on each axis, accumulated by every primitive of the node
-//    (wave-aggregated float atomics), the best axis and bin boundary chosen
+//    bins on each axis, summed in LDS per chunk of primitives, the best axis and bin boundary chosen
 //    by the surface-area heuristic, and the node's range partitioned stably
 //    in place through a prefix sum of the go-left flags.  Nodes of at most
 //    kSmall primitives are built to the leaves by one wave each, with an

@@ -408,7 +408,7 @@ __device__ __forceinline__ VolShadowState vol_shadow_surface(const DevScene& sce
 
 // A wave runs, step by step, whatever most of its lanes wait for: taking new
 // rays, tracing, a collision or a surface.  With every lane running its whole
-// pass, a quarter of the lanes were active on average (volume frame 44.7 ms in
+// pass, a quarter of the lanes were active on average (volume frame with 4 M paths in flight 44.7 ms in
 // this kernel, now 28.1).
 __global__ void __launch_bounds__(kTraceBlock) k_vol_shadow(Wavefront w, DevScene scene) {
   __shared__ uint32_t lds[32], used_up;
