@@ -365,4 +365,11 @@ uint32_t BvhStackNeed(const std::vector<BvhNode4>& nodes) {
   return need[0];
 }
 
+uint32_t BvhLargestLeaf(const std::vector<BvhNode4>& nodes) {
+  uint32_t largest = 0;
+  for (const BvhNode4& n : nodes)
+    for (uint32_t c : n.count) largest = std::max(largest, c);
+  return largest;
+}
+
 }  // namespace rad

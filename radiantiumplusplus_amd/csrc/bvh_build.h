@@ -20,7 +20,8 @@ struct BvhBuildResult {
 };
 
 // Host binned-SAH build.  `bounds` holds 6 floats per primitive
-// (lo.xyz, hi.xyz).  Leaves hold at most `max_leaf` primitives.
+// (lo.xyz, hi.xyz).  Leaves hold at most `max_leaf` primitives, but a range
+// that is not split apart after 60 levels is one leaf whatever its size.
 void BuildBvh4Host(const float* bounds, uint32_t count, int max_leaf, BvhBuildResult& out);
 
 // SAH cost of a finished tree (traversal 1, intersection 1, relative to root area).
@@ -28,5 +29,7 @@ float BvhSahCost(const std::vector<BvhNode4>& nodes);
 uint32_t BvhDepth(const std::vector<BvhNode4>& nodes);
 // Worst-case traversal stack entries of the tree (see kTraceStackEntries).
 uint32_t BvhStackNeed(const std::vector<BvhNode4>& nodes);
+// Primitives of the largest leaf.
+uint32_t BvhLargestLeaf(const std::vector<BvhNode4>& nodes);
 
 }  // namespace rad

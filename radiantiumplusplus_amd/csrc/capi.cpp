@@ -265,14 +265,16 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
     } else {
       BvhBuildResult r;
       BuildBvh4Host(h.prim_bounds.data(), n, maxLeaf, r);
+      largestLeaf = BvhLargestLeaf(r.nodes);  // at the builder's depth limit: any size
+      if (largestLeaf > kMaxLeafPrims)  // nothing of the scene has changed yet: it keeps the tree it had
+        throw StatusError(RAD_ERR_INVALID_ARG, "BVH leaf of " + std::to_string(largestLeaf) + " primitives; at most " +
+                                                   std::to_string(kMaxLeafPrims) + " can be traversed");
       std::vector<float4> ordered(3 * size_t(n));
       for (uint32_t i = 0; i < n; i++)
         for (int k = 0; k < 3; k++) ordered[3 * size_t(i) + k] = h.prim_records[3 * size_t(r.order[i]) + k];
       scene->d_prims.upload(ordered.data(), ordered.size() * sizeof(float4), scene->ctx->stream);
       scene->d_nodes.upload(r.nodes.data(), r.nodes.size() * sizeof(BvhNode4), scene->ctx->stream);
       HipCheck(hipStreamSynchronize(scene->ctx->stream), "BVH upload");
-      for (const BvhNode4& nd : r.nodes)  // at the builder's depth limit a leaf may be larger than asked for
-        for (uint32_t c : nd.count) largestLeaf = std::max(largestLeaf, c);
       nodeCount = uint32_t(r.nodes.size());
       depth = r.depth;
       stackNeed = r.stack_need;

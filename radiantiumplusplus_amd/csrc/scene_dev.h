@@ -73,6 +73,12 @@ struct alignas(128) BvhNode8 {
 static_assert(sizeof(BvhNode8) == 128, "traversal node must be one 128-byte line");
 constexpr uint32_t kWidePlaneMax = 2047;  // largest plane value (every integer up to 2048 is exact in binary16)
 constexpr uint32_t kWideNodePrims = 32;   // most primitives in the leaf children of one node
+// Most primitives of a BvhNode4 leaf that the traversal's nodes are made from:
+// a leaf of more than kWideNodePrims takes a node of its own with up to eight
+// children, so larger ones have no place (bvh_gpu.hip).  Trees with larger
+// leaves are refused.
+constexpr uint32_t kMaxLeafPrims = 255;
+static_assert(kMaxLeafPrims <= 8 * kWideNodePrims, "a leaf's node has eight children");
 
 // binary16 bits of an integer 0..2047, and back.
 __host__ __device__ inline uint16_t plane_bits(uint32_t q) {

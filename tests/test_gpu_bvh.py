@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import _oracle as O
+from _trees import mesh_scene, shrinking_sequence
 from radiantiumplusplus_amd import _ffi as F
 from radiantiumplusplus_amd import hip, scenes
 from test_gpu_intersect import check_parity, ray_batch
@@ -153,3 +154,40 @@ def test_deep_trees_are_exact_or_refused(hip_ctx, levels):
         rays["tmax"] = 3e38
         check_parity(o, rays, g.closest(rays), o.closest(rays, brute=True))
         assert np.array_equal(g.occluded(rays).astype(bool), o.occluded(rays, brute=True).astype(bool))
+
+
+def rays_along_z(extent, n, seed):
+    """Rays from z = -1 through points of z = 0 with x and y of up to `extent`, with slopes of its size: exact to
+    float precision however small it is (components below 1e-18 are left out: the traversal raises them to that)."""
+    rng = np.random.default_rng(seed)
+    rays = np.zeros(n, hip.RAY_DTYPE)
+    to, d = rng.uniform(-extent, extent, (n, 2)), rng.uniform(0.01, 1, (n, 2)) * rng.choice([-extent, extent], (n, 2))
+    rays["o"] = np.concatenate([to - d, np.full((n, 1), -1.0)], 1)
+    rays["d"] = np.concatenate([d, np.ones((n, 1))], 1)
+    rays["tmax"] = 3e38
+    return rays
+
+
+@pytest.mark.parametrize("leaf", [33, 255, 256, 603])
+def test_leaf_at_the_host_builders_depth_limit(hip_ctx, leaf):
+    """A leaf of 255 primitives is traversed; a larger one is refused before anything of the scene changes, so the
+    tree it had stays in use."""
+    tris = shrinking_sequence(leaf)
+    b = mesh_scene(tris)
+    o = O.OracleScene(b)
+    rays = rays_along_z(1.2 * float(np.abs(tris[60:]).max()), 4000, leaf)
+    hb = o.closest(rays, brute=True)
+    assert 0.01 < (hb["geom"] != 0xFFFFFFFF).mean() < 0.99
+    g = hip.Scene.from_builder(hip_ctx, b, builder=F.RAD_BVH_DEVICE)
+    before = g.closest(rays)
+    check_parity(o, rays, before, hb)
+    if leaf <= 255:
+        g.build_bvh(F.RAD_BVH_HOST)
+        assert g.bvh_check().max_leaf == leaf
+    else:
+        with pytest.raises(hip.RadError, match=f"leaf of {leaf} ") as e:
+            g.build_bvh(F.RAD_BVH_HOST)
+        assert e.value.status == 1  # RAD_ERR_INVALID_ARG
+        assert np.array_equal(g.closest(rays), before)
+    check_parity(o, rays, g.closest(rays), hb)
+    assert np.array_equal(g.occluded(rays).astype(bool), hb["geom"] != 0xFFFFFFFF)
