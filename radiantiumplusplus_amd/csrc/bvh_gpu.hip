@@ -22,6 +22,7 @@
 #include <stdexcept>
 
 #include "bvh_gpu.h"
+#include "bvh_wide.h"
 
 namespace rad {
 namespace {
@@ -76,12 +77,6 @@ __device__ __forceinline__ uint32_t ordered_bits(float v) {
 }
 __device__ __forceinline__ float from_ordered(uint32_t u) {
   return __uint_as_float(u ^ (uint32_t(int32_t(~u) >> 31) | 0x80000000u));
-}
-
-__device__ __forceinline__ float half_area(const float lo[3], const float hi[3]) {
-  float dx = hi[0] - lo[0], dy = hi[1] - lo[1], dz = hi[2] - lo[2];
-  if (!(dx >= 0.f && dy >= 0.f && dz >= 0.f)) return 0.f;
-  return dx * dy + dy * dz + dz * dx;
 }
 
 // ---------------------------------------------------------------- ordering
@@ -885,146 +880,13 @@ __global__ void k_sah(const BvhNode4* nodes, uint32_t m, float rootA, double* co
 }
 
 // ---------------------------------------------------------------- traversal nodes
-// A node of the 8-wide tree: a BvhNode4 (count 0) whose inner children are
-// opened while they fit, or a leaf that does not fit beside its siblings
-// (count > 0, primitives [begin, begin + count) of the new order, the box of
-// child `src` of BvhNode4 n4).
-struct WideJob {
-  uint32_t n4, src, begin, count;
-};
-
-struct WideSlot {  // child `s` of BvhNode4 `n`
-  uint32_t n, s;
-};
-struct WideKids {  // the children chosen for a node: BvhNode4 index * 4 + child, kNone: none
-  uint32_t k[8];
-};
-
-__device__ __forceinline__ void slot_box(const BvhNode4* nodes, WideSlot w, float lo[3], float hi[3]) {
-  const BvhNode4& nd = nodes[w.n];
-  lo[0] = nd.lox[w.s], lo[1] = nd.loy[w.s], lo[2] = nd.loz[w.s];
-  hi[0] = nd.hix[w.s], hi[1] = nd.hiy[w.s], hi[2] = nd.hiz[w.s];
-}
-
-// The children of the 8-wide node made from BvhNode4 `root`: its own four,
-// then the inner one of largest area replaced by its children while at most
-// eight result and their leaves hold at most kWideNodePrims primitives.
-__device__ int wide_children(const BvhNode4* nodes, uint32_t root, WideSlot out[8]) {
-  int n = 0;
-  uint32_t prims = 0;
-  for (uint32_t s = 0; s < 4; s++)
-    if (nodes[root].child[s] >= 0) {
-      prims += nodes[root].count[s];
-      out[n++] = WideSlot{root, s};
-    }
-  for (;;) {
-    int best = -1;
-    float area = -1.f;
-    uint32_t bestPrims = 0;
-    for (int i = 0; i < n; i++) {
-      const BvhNode4& nd = nodes[out[i].n];
-      if (nd.count[out[i].s] > 0) continue;
-      const BvhNode4& c = nodes[nd.child[out[i].s]];
-      int k = 0;
-      uint32_t p = 0;
-      for (int s = 0; s < 4; s++)
-        if (c.child[s] >= 0) {
-          k++;
-          p += c.count[s];
-        }
-      if (n - 1 + k > 8 || prims + p > kWideNodePrims) continue;
-      float lo[3], hi[3];
-      slot_box(nodes, out[i], lo, hi);
-      const float a = half_area(lo, hi);
-      if (a > area) {
-        area = a;
-        best = i;
-        bestPrims = p;
-      }
-    }
-    if (best < 0) return n;
-    const uint32_t c = uint32_t(nodes[out[best].n].child[out[best].s]);
-    prims += bestPrims;
-    bool first = true;
-    for (uint32_t s = 0; s < 4; s++)
-      if (nodes[c].child[s] >= 0) {
-        out[first ? best : n++] = WideSlot{c, s};
-        first = false;
-      }
-  }
-}
-
-// slot[i]: the slot of child i, chosen greedily so that bit a of a slot says
-// on which side of the node's centre the child's centre lies along axis a.
-__device__ void wide_order(const BvhNode4* nodes, const WideSlot* w, int n, const float lo[3], const float hi[3], int slot[8]) {
-  float d[8][3];
-  for (int i = 0; i < n; i++) {
-    float l[3], h[3];
-    slot_box(nodes, w[i], l, h);
-    for (int a = 0; a < 3; a++) d[i][a] = (l[a] + h[a]) - (lo[a] + hi[a]);
-    slot[i] = -1;
-  }
-  uint32_t used = 0;
-  for (int k = 0; k < n; k++) {
-    float best = -kInf;
-    int bi = -1, bs = 0;
-    for (int i = 0; i < n; i++) {
-      if (slot[i] >= 0) continue;
-      for (int s = 0; s < 8; s++) {
-        if (used >> s & 1u) continue;
-        const float c = (s & 1 ? d[i][0] : -d[i][0]) + (s & 2 ? d[i][1] : -d[i][1]) + (s & 4 ? d[i][2] : -d[i][2]);
-        if (bi < 0 || c > best) best = c, bi = i, bs = s;
-      }
-    }
-    slot[bi] = bs;
-    used |= 1u << bs;
-  }
-}
-
-// Step 2^e per axis, e the smallest with kWidePlaneMax * 2^e >= the node's
-// extent (raised further if rounding keeps a bound out of reach); bounds
-// rounded outward and verified with the traversal's own dequantisation.
-__device__ bool quantize_axis(const float* clo, const float* chi, uint32_t valid, float o, float ext, uint32_t& biased,
-                              uint16_t* qlo, uint16_t* qhi) {
-  constexpr float top = float(kWidePlaneMax);
-  int e = -126;
-  if (ext > 0.f) {
-    frexpf(ext / top, &e);  // ext / top = m 2^e, m in [0.5, 1)
-    e = max(e, -126);
-  }
-  for (; e <= 127; e++) {
-    const uint32_t b = uint32_t(e + 127);
-    const float step = quant_step(b);
-    bool ok = true;
-    for (int i = 0; i < 8 && ok; i++) {
-      qlo[i] = plane_bits(kWidePlaneMax);  // an empty slot: an inverted box
-      qhi[i] = 0;
-      if (!(valid >> i & 1u)) continue;
-      uint32_t a = uint32_t(fminf(fmaxf(floorf((clo[i] - o) / step), 0.f), top));
-      uint32_t c = uint32_t(fminf(fmaxf(ceilf((chi[i] - o) / step), 0.f), top));
-      while (a > 0 && dequant(a, step, o) > clo[i]) a--;
-      while (c < kWidePlaneMax && dequant(c, step, o) < chi[i]) c++;
-      if (!(dequant(a, step, o) <= clo[i] && dequant(c, step, o) >= chi[i])) ok = false;
-      qlo[i] = plane_bits(a);
-      qhi[i] = plane_bits(c);
-    }
-    if (ok) {
-      biased = b;
-      return true;
-    }
-  }
-  return false;
-}
-
-// One thread per node of a level.  EMIT = false: sums[j] = its inner children
-// (low word) and the primitives it places (high word).  EMIT = true, after an
-// exclusive scan of the sums: writes the node, its inner children's jobs, the
-// new place of its primitives, and that place into the BvhNode4 leaves.
+// One thread per node of a level (bvh_wide.h).  EMIT = false: sums[j] =
+// wide_count.  EMIT = true, after an exclusive scan of the sums: wide_emit.
 struct WideLevel {
   uint32_t nodes, next, prims;  // first node of this level, of the next level, first primitive this level places
 };
 template <bool EMIT>
-__global__ void k_wide(const WideJob* jobs, uint32_t nJobs, BvhNode4* nodes, unsigned long long* sums, WideKids* kids,
+__global__ void __launch_bounds__(64) k_wide(const WideJob* jobs, uint32_t nJobs, BvhNode4* nodes, unsigned long long* sums, WideKids* kids,
                        WideLevel lv, BvhNode8* out, WideJob* next, uint32_t* perm, uint32_t* error) {
   const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= nJobs) {
@@ -1032,104 +894,15 @@ __global__ void k_wide(const WideJob* jobs, uint32_t nJobs, BvhNode4* nodes, uns
     return;
   }
   const WideJob jb = jobs[j];
-  WideSlot w[8];
-  uint32_t cnt[8];   // leaf: primitives; 0: inner
-  uint32_t wrap = 0;  // children that are leaves with a node of their own
-  int n;
-  if (jb.count > 0) {  // a leaf on its own: one slot, or the next nodes hold kWideNodePrims each
-    n = int((jb.count + kWideNodePrims - 1) / kWideNodePrims);
-    for (int i = 0; i < n; i++) {
-      w[i] = WideSlot{jb.n4, jb.src};
-      cnt[i] = min(kWideNodePrims, jb.count - uint32_t(i) * kWideNodePrims);
-    }
-    if (n > 1) wrap = (1u << n) - 1u;
-  } else {
-    if (EMIT) {
-      n = 0;
-      for (int i = 0; i < 8; i++)
-        if (kids[j].k[i] != kNone) w[n++] = WideSlot{kids[j].k[i] >> 2, kids[j].k[i] & 3u};
-    } else {
-      n = wide_children(nodes, jb.n4, w);
-      for (int i = 0; i < 8; i++) kids[j].k[i] = i < n ? w[i].n * 4 + w[i].s : kNone;
-    }
-    uint32_t acc = 0;
-    for (int i = 0; i < n; i++) {
-      cnt[i] = nodes[w[i].n].count[w[i].s];
-      if (acc + cnt[i] > kWideNodePrims)
-        wrap |= 1u << i;
-      else
-        acc += cnt[i];
-    }
-  }
-  uint32_t inner = 0, prims = 0;
-  for (int i = 0; i < n; i++) {
-    inner += cnt[i] == 0 || (wrap >> i & 1u) ? 1u : 0u;
-    prims += cnt[i];
-  }
-  if (jb.count > 0) prims = 0;  // placed by its parent
   if (!EMIT) {
-    sums[j] = (static_cast<unsigned long long>(prims) << 32) | inner;
+    sums[j] = wide_count(nodes, jb, kids[j]);
     return;
   }
-  const uint32_t child0 = lv.next + uint32_t(sums[j]), job0 = uint32_t(sums[j]);
-  const uint32_t prim0 = jb.count > 0 ? jb.begin : lv.prims + uint32_t(sums[j] >> 32);
-  float lo[3] = {kInf, kInf, kInf}, hi[3] = {-kInf, -kInf, -kInf};
-  for (int i = 0; i < n; i++) {
-    float l[3], h[3];
-    slot_box(nodes, w[i], l, h);
-    for (int a = 0; a < 3; a++) lo[a] = fminf(lo[a], l[a]), hi[a] = fmaxf(hi[a], h[a]);
-  }
-  int slot[8], at[8];
-  wide_order(nodes, w, n, lo, hi, slot);
-  for (int s = 0; s < 8; s++) at[s] = -1;
-  for (int i = 0; i < n; i++) at[slot[i]] = i;
+  const uint32_t inner = uint32_t(sums[j]), prims = uint32_t(sums[j] >> 32);
   BvhNode8 o;
-  float cl[3][8], ch[3][8];
-  uint32_t valid = 0, imask = 0, placed = 0, k = 0;
-  uint32_t ends[2] = {0, 0};
-  uint32_t later = 0;  // wrapped leaves are placed behind the node's own
-  for (int i = 0; i < n; i++) later += wrap >> i & 1u ? 0u : cnt[i];
-  for (int s = 0; s < 8; s++) {
-    const int i = at[s];
-    if (i >= 0) {
-      float l[3], h[3];
-      slot_box(nodes, w[i], l, h);
-      for (int a = 0; a < 3; a++) cl[a][s] = l[a], ch[a][s] = h[a];
-      valid |= 1u << s;
-      uint32_t begin = prim0;
-      if (cnt[i] > 0 && jb.count == 0) {  // a leaf of the BvhNode4 tree gets its new place
-        const bool wrapped = wrap >> i & 1u;
-        begin += wrapped ? later : placed;
-        (wrapped ? later : placed) += cnt[i];
-        const uint32_t from = uint32_t(nodes[w[i].n].child[w[i].s]);
-        for (uint32_t q = 0; q < cnt[i]; q++) perm[begin + q] = from + q;
-        nodes[w[i].n].child[w[i].s] = int32_t(begin);
-      } else if (cnt[i] > 0) {
-        begin += uint32_t(i) * kWideNodePrims;
-        if (!(wrap >> i & 1u)) placed += cnt[i];
-      }
-      if (cnt[i] == 0 || (wrap >> i & 1u)) {
-        imask |= 1u << s;
-        next[job0 + k] = cnt[i] == 0 ? WideJob{uint32_t(nodes[w[i].n].child[w[i].s]), 0, 0, 0}
-                                     : WideJob{w[i].n, w[i].s, begin, cnt[i]};
-        k++;
-      }
-    }
-    ends[s >> 2] |= placed << (8 * (s & 3));
-  }
-  uint32_t bx = 127, by = 127, bz = 127;
-  const bool ok = quantize_axis(cl[0], ch[0], valid, lo[0], hi[0] - lo[0], bx, o.lox, o.hix) &&
-                  quantize_axis(cl[1], ch[1], valid, lo[1], hi[1] - lo[1], by, o.loy, o.hiy) &&
-                  quantize_axis(cl[2], ch[2], valid, lo[2], hi[2] - lo[2], bz, o.loz, o.hiz);
-  if (!ok) atomicOr(error, 1u);
-  o.ox = lo[0];
-  o.oy = lo[1];
-  o.oz = lo[2];
-  o.exps = bx | by << 8 | bz << 16 | imask << 24;
-  o.child_base = child0;
-  o.prim_base = prim0;
-  o.ends[0] = ends[0];
-  o.ends[1] = ends[1];
+  if (!wide_emit(nodes, jb, kids[j], lv.next + inner, jb.mask & kWideRest ? jb.begin : lv.prims + prims, o, next + inner,
+                        perm))
+    atomicOr(error, 1u);
   out[lv.nodes + j] = o;
 }
 
@@ -1151,8 +924,9 @@ struct Carver {
 
 uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, uint32_t maxLeaf, DeviceBuffer& prims, uint32_t n, hipStream_t st,
                         DeviceBuffer& work, DeviceBuffer& out) {
-  // One node per BvhNode4 at most, unless leaves need nodes of their own: four
-  // leaves of at most kWideNodePrims / 4 never do.
+  // One node per BvhNode4 at most, unless its leaves hold more than
+  // kWideNodePrims (four of at most a quarter of that never do): a chain then has
+  // at most one node per leaf, one more per kWideNodePrims and one for the rest.
   const size_t cap = maxLeaf <= kWideNodePrims / 4 ? size_t(m) : 5 * size_t(m) + n / kWideNodePrims + 8;
   size_t scanBytes = 0;
   HipCheck(hipcub::DeviceScan::ExclusiveSum(nullptr, scanBytes, static_cast<unsigned long long*>(nullptr),
@@ -1179,7 +953,7 @@ uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, uint32_t maxLeaf, Devic
   if (work.bytes < need) work.alloc(need);
   carve(Carver{static_cast<char*>(work.ptr)});
   HipCheck(hipMemsetAsync(flag, 0, 4, st), "wide node flag");
-  const WideJob root{0, 0, 0, 0};
+  const WideJob root{0, kWideAll, 0, 0};
   HipCheck(hipMemcpyAsync(cur, &root, sizeof(root), hipMemcpyHostToDevice, st), "wide root");
   uint32_t nJobs = 1;
   WideLevel lv{0, 1, 0};

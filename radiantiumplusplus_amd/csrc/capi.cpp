@@ -280,7 +280,7 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
       stackNeed = r.stack_need;
       sah = r.sah_cost;
     }
-    // The traversal keeps kTraceStackEntries stack entries per ray; a deeper
+    // The traversal keeps as many groups per ray (kGroupStackEntries); a deeper
     // need would drop subtrees (missed hits, light leaks), so such a tree is
     // refused.  The scene keeps no half-built tree.
     if (stackNeed > kTraceStackEntries) {
@@ -374,11 +374,12 @@ rad_status rad_hip_autotune(rad_scene* scene, const rad_render_desc* probe, rad_
 }
 
 // Errors of the traversal's nodes: primitives not referenced exactly once,
-// node references out of range or repeated, and child boxes that do not
-// contain the triangles and spheres below them.
+// node references out of range or repeated, child boxes that do not contain
+// the triangles and spheres below them, a stack need beyond the traversal's.
 static uint32_t CheckWideNodes(const std::vector<BvhNode8>& wide, const std::vector<float4>& prims, uint32_t n) {
   uint32_t errors = 0;
   std::vector<uint8_t> seen(n, 0), parents(wide.size(), 0);
+  std::vector<uint32_t> need(wide.size(), 0);
   std::vector<std::array<float, 6>> bounds(wide.size());
   for (size_t x = wide.size(); x-- > 0;) {  // children come after their parents
     const BvhNode8& w = wide[x];
@@ -398,6 +399,7 @@ static uint32_t CheckWideNodes(const std::vector<BvhNode8>& wide, const std::vec
         }
         parents[c]++;
         b = bounds[c];
+        need[x] = std::max(need[x], need[c]);
       } else {
         for (uint32_t k = begin; k < end; k++) {
           const uint64_t p = uint64_t(w.prim_base) + k;
@@ -427,7 +429,9 @@ static uint32_t CheckWideNodes(const std::vector<BvhNode8>& wide, const std::vec
         nb[3 + a] = std::max(nb[3 + a], b[3 + a]);
       }
     }
+    need[x] += inner > 1 ? 1u : 0u;
   }
+  errors += !wide.empty() && need[0] > kGroupStackEntries;
   for (uint32_t p = 0; p < n; p++) errors += seen[p] != 1;
   for (size_t x = 0; x < wide.size(); x++) errors += parents[x] != (x ? 1 : 0);
   return errors;

@@ -36,9 +36,9 @@ constexpr uint32_t kTraceStackEntries = 64;
 // Entries of the traversal's own stack.  It holds groups of siblings still to
 // be visited, one per BvhNode8 on the way down that has more than one inner
 // child; such a node holds a BvhNode4 with more than one inner child on the
-// same way, so the need is at most the BvhNode4 tree's, plus two for leaves
-// that get nodes of their own (kWideNodePrims).
-constexpr uint32_t kGroupStackEntries = kTraceStackEntries + 2;
+// same way (the nodes of a chain, bvh_wide.h, have one but for the last), so
+// the need is at most the BvhNode4 tree's.
+constexpr uint32_t kGroupStackEntries = kTraceStackEntries;
 // Entries of a wave's pooled primitive tests per node step (traverse.h); a
 // lane whose entries fall beyond the pool tests them itself.
 constexpr uint32_t kTracePool = 64;
@@ -73,12 +73,9 @@ struct alignas(128) BvhNode8 {
 static_assert(sizeof(BvhNode8) == 128, "traversal node must be one 128-byte line");
 constexpr uint32_t kWidePlaneMax = 2047;  // largest plane value (every integer up to 2048 is exact in binary16)
 constexpr uint32_t kWideNodePrims = 32;   // most primitives in the leaf children of one node
-// Most primitives of a BvhNode4 leaf that the traversal's nodes are made from:
-// a leaf of more than kWideNodePrims takes a node of its own with up to eight
-// children, so larger ones have no place (bvh_gpu.hip).  Trees with larger
-// leaves are refused.
+// Most primitives of a leaf (a leaf of more than kWideNodePrims takes a chain
+// of nodes); trees with larger leaves are refused.
 constexpr uint32_t kMaxLeafPrims = 255;
-static_assert(kMaxLeafPrims <= 8 * kWideNodePrims, "a leaf's node has eight children");
 
 // binary16 bits of an integer 0..2047, and back.
 __host__ __device__ inline uint16_t plane_bits(uint32_t q) {

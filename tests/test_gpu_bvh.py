@@ -183,7 +183,9 @@ def test_leaf_at_the_host_builders_depth_limit(hip_ctx, leaf):
     check_parity(o, rays, before, hb)
     if leaf <= 255:
         g.build_bvh(F.RAD_BVH_HOST)
-        assert g.bvh_check().max_leaf == leaf
+        r = g.bvh_check()
+        assert r.max_leaf == leaf and r.quantized_box_violations == 0 and r.leaf_box_violations == 0
+        assert r.structure_errors == 0 and r.unreferenced_or_repeated == 0
     else:
         with pytest.raises(hip.RadError, match=f"leaf of {leaf} ") as e:
             g.build_bvh(F.RAD_BVH_HOST)
