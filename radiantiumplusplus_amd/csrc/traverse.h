@@ -117,8 +117,8 @@ __device__ __forceinline__ bool isect_rect(const Affine& toObj, f3 ro, f3 rd, fl
 
 __device__ __forceinline__ f3 xyz(float4 a) { return mk(a.x, a.y, a.z); }
 
-// Test one primitive record (its three float4, already loaded); on a hit
-// narrows `tfar` to its distance.
+// Test one primitive record (its three float4, already loaded) against the
+// segment (tnear, tfar]; on a hit `tfar` becomes its distance.
 __device__ __forceinline__ bool isect_rec(const DevScene& s, float4 a, float4 b, float4 c, f3 o, f3 d, float tnear,
                                           float& tfar) {
   const uint32_t kind = __float_as_uint(c.w);
@@ -185,6 +185,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) u32x2 lds_u2;
 typedef __attribute__((address_space(3))) u32x4 lds_u4;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
+typedef __attribute__((address_space(3))) float lds_f32;
 typedef __attribute__((address_space(3))) unsigned long long lds_u64;
 
 // Per-lane private overflow of a traversal stack (entries below the LDS ring).
@@ -227,9 +228,13 @@ struct TraceStack {
   }
 };
 
-// The closest hit is the minimum of (t, primitive) over the accepted
-// primitives, whatever order they are tested in: an unsigned key in that
-// order (t may be negative where tmin is).
+// The closest hit is the minimum of (t, primitive) over the primitives that
+// accept the ray's whole segment, whatever order they are tested in (when a
+// wave tests them depends on its other rays): an unsigned key in that order (t
+// may be negative where tmin is).  Only boxes are tested against the closest
+// hit so far.  A triangle is not: it accepts by T <= |den| * tfar, and at t =
+// T / |den| itself |den| * t may round below T, so one of two coincident
+// triangles would be dropped or kept by the order of the tests.
 __device__ __forceinline__ unsigned long long hit_key(float t, uint32_t prim) {
   const uint32_t u = __float_as_uint(t);
   return (static_cast<unsigned long long>(u ^ (uint32_t(int32_t(u) >> 31) | 0x80000000u)) << 32) | prim;
@@ -548,6 +553,7 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
   __shared__ u32x4 lds_group[kTraceBlock / 64][kGroupQueue];
   __shared__ u32x2 lds_pool[kTraceBlock / 64][kPoolSize];
   __shared__ unsigned long long lds_key[kTraceBlock];
+  __shared__ float lds_tmax[kTraceBlock];  // end of each lane's segment
   __shared__ uint32_t lds_used_up;  // the counter has no more items for this block
   const uint32_t lane = __lane_id();
   const unsigned long long below = (1ull << lane) - 1ull;
@@ -555,6 +561,7 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
   lds_u4* const group = (lds_u4*)lds_group[wv];
   lds_u2* const pool = (lds_u2*)lds_pool[wv];
   lds_u64* const key = (lds_u64*)&lds_key[wv * 64];
+  lds_f32* const seg = (lds_f32*)&lds_tmax[wv * 64];
   TraceOverflow ov;
   TraceStack st;
   st.ring = (lds_u64*)(lds_ring + threadIdx.x);
@@ -607,6 +614,7 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
           if (job.load(i, o, d, tmin, tmax, tag)) {
             if constexpr (!Job::kTagIsIndex) idx = i;
             trace_begin(r, st, o, d, tmin, tmax);
+            seg[lane] = tmax;
             if constexpr (Job::kSuspend) job.resume(tag, r, st);
             visits = 0;
             have = active = true;
@@ -671,12 +679,12 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
             const f3 o = mk(__shfl(r.o.x, e.y), __shfl(r.o.y, e.y), __shfl(r.o.z, e.y));
             const f3 d = mk(__shfl(r.d.x, e.y), __shfl(r.d.y, e.y), __shfl(r.d.z, e.y));
             const float tmin = __shfl(r.tmin, e.y);
-            float tfar = __shfl(r.tfar, e.y);
-            if (valid && isect_prim(s, e.x, o, d, tmin, tfar)) {
+            float th = seg[e.y];
+            if (valid && isect_prim(s, e.x, o, d, tmin, th)) {
               if (ANY)
                 key[e.y] = 0;
               else
-                __hip_atomic_fetch_min(&key[e.y], hit_key(tfar, e.x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                __hip_atomic_fetch_min(&key[e.y], hit_key(th, e.x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
             }
             wave_lds_fence();
           }
@@ -725,10 +733,10 @@ __device__ __forceinline__ bool trace(const DevScene& s, f3 o, f3 d, float tmin,
     if (leaf.hits) {
       for (uint32_t pm = leaf_prims(leaf); pm; pm &= pm - 1u) {
         const uint32_t p = leaf.prim_base + uint32_t(__ffs(int(pm)) - 1);
-        float tf = r.tfar;
-        if (!isect_prim(s, p, r.o, r.d, r.tmin, tf)) continue;
-        if (hit_key(tf, p) < r.key()) {
-          r.tfar = tf;
+        float t = tmax;
+        if (!isect_prim(s, p, r.o, r.d, r.tmin, t)) continue;
+        if (hit_key(t, p) < r.key()) {
+          r.tfar = t;
           r.hitp = p;
         }
         if (ANY) {

@@ -100,6 +100,35 @@ def test_ties_do_not_depend_on_the_batch(hip_ctx):
     assert np.array_equal(whole[7:8], g.closest(rays[7:8]))
 
 
+@pytest.mark.parametrize("builder", [F.RAD_BVH_DEVICE, F.RAD_BVH_HOST])
+@pytest.mark.parametrize("axis", [False, True])
+def test_ties_between_nodes_do_not_depend_on_the_batch(hip_ctx, builder, axis):
+    """A dozen copies of every triangle, one to a leaf, so that they lie in different nodes and are tested at
+    different times; axis: in planes of constant z, where the boxes are flat.  Which copy a ray reports does not depend
+    on what else is traced."""
+    rng = np.random.default_rng(16)
+    p = rng.uniform(-1, 1, (150, 1, 3)) + rng.normal(0, 0.3, (150, 3, 3))
+    if axis:
+        p[:, :, 2] = np.round(4 * p[:, :1, 2]) / 4
+    p = np.concatenate([p] * 12).reshape(-1, 3).astype(np.float32)
+    b = scenes.SceneBuilder()
+    b.mesh(p, np.arange(len(p), dtype=np.uint32), bsdf=b.diffuse(0.5))
+    b.skybox(1.0)
+    b.set_camera(8, 8, 45, origin=(0, 0, -5), target=(0, 0, 0), far=100)
+    g = hip.Scene.from_builder(hip_ctx, b, builder=builder, max_leaf=1)
+    n = 200000
+    rays = ray_batch(np.array([-2.0, -2, -2]), np.array([2.0, 2, 2]), n, 8)
+    whole = g.closest(rays)
+    assert (whole["geom"] != 0xFFFFFFFF).sum() > 10000
+    for seed in range(3):
+        order = np.random.default_rng(seed).permutation(n)
+        got = g.closest(rays[order])
+        assert np.array_equal(whole["t"][order], got["t"])
+        assert (whole[order] != got).sum() == 0
+    few = np.random.default_rng(9).permutation(n)[:3000]
+    assert np.array_equal(whole[few], g.closest(rays[few]))
+
+
 @pytest.mark.parametrize("w,h", [(1, 1), (7, 5), (8, 8), (9, 17), (23, 3), (65, 31)])
 def test_every_pixel_gets_its_samples(hip_ctx, w, h):
     """Images whose last tiles are partial: under a constant sky every pixel is
