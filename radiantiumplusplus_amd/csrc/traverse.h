@@ -255,7 +255,9 @@ struct TraceRay {
   Hit h;           // filled by trace_finish
   static constexpr uint32_t kNoHit = 0xffffffffu;
   __device__ __forceinline__ bool hit() const { return hitp != kNoHit; }
-  __device__ __forceinline__ unsigned long long key() const { return hit_key(tfar, hitp); }
+  // Without a hit any key is closer: t = T / |den| may round above the tmax
+  // that T <= |den| * tmax was accepted with.
+  __device__ __forceinline__ unsigned long long key() const { return hit() ? hit_key(tfar, hitp) : ~0ull; }
 };
 
 // Fills the hit record of a finished closest-hit traversal.

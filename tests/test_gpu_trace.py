@@ -129,6 +129,26 @@ def test_ties_between_nodes_do_not_depend_on_the_batch(hip_ctx, builder, axis):
     assert np.array_equal(whole[few], g.closest(rays[few]))
 
 
+def test_hits_at_the_end_of_the_segment(hip_ctx):
+    """A triangle accepts T <= |den| * tmax, whose right side may round up: a hit at t = T / |den| one ulp above tmax is
+    a hit of both queries.  The rays are those that the brute force keeps with tmax one ulp below their t."""
+    b = soup(300, 0.3, 11)
+    o = O.OracleScene(b)
+    g = hip.Scene.from_builder(hip_ctx, b)
+    lo, hi = o.bounds()
+    rays = ray_batch(lo, hi, 60000, 12)
+    rays["tmax"] = 3e38
+    h = o.closest(rays, brute=True)
+    hit = h["geom"] != 0xFFFFFFFF
+    rays, h = rays[hit], h[hit]
+    rays["tmax"] = np.nextafter(h["t"], np.float32(0))
+    kept = o.closest(rays, brute=True)
+    end = (kept["geom"] != 0xFFFFFFFF) & (kept["t"] > rays["tmax"])
+    assert end.sum() > 100
+    check_parity(o, rays, g.closest(rays), kept)
+    assert np.array_equal(g.occluded(rays).astype(bool), kept["geom"] != 0xFFFFFFFF)
+
+
 @pytest.mark.parametrize("w,h", [(1, 1), (7, 5), (8, 8), (9, 17), (23, 3), (65, 31)])
 def test_every_pixel_gets_its_samples(hip_ctx, w, h):
     """Images whose last tiles are partial: under a constant sky every pixel is
