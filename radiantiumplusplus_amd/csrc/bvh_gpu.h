@@ -36,10 +36,11 @@ struct PrimSource {
   uint32_t count = 0;
 };
 
-// Writes the nodes and the primitive records in leaf order to device buffers;
-// work: scratch memory, left allocated for BuildWideNodes.
+// Writes the nodes and the primitive records in leaf order to device buffers,
+// whose old contents hold until outputsValid is cleared, just before the first
+// write; work: scratch memory, left allocated for BuildWideNodes.
 void BuildBvh4Device(const PrimSource& src, int maxLeaf, hipStream_t st, DeviceBuffer& nodesOut, DeviceBuffer& primsOut,
-                     DeviceBuffer& work, DeviceBvhStats& stats);
+                     bool& outputsValid, DeviceBuffer& work, DeviceBvhStats& stats);
 
 // The traversal's nodes from a tree of m BvhNode4, with leaves of at most
 // maxLeaf, over n primitive records (device buffers): writes them to `out` and

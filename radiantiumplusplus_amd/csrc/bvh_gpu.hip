@@ -992,7 +992,7 @@ uint32_t BuildWideNodes(DeviceBuffer& nodes, uint32_t m, uint32_t maxLeaf, Devic
 }
 
 void BuildBvh4Device(const PrimSource& src, int maxLeaf, hipStream_t st, DeviceBuffer& nodesOut, DeviceBuffer& primsOut,
-                     DeviceBuffer& work, DeviceBvhStats& stats) {
+                     bool& outputsValid, DeviceBuffer& work, DeviceBvhStats& stats) {
   const uint32_t n = src.count;
   if (n == 0) throw std::runtime_error("scene has no primitives");
   if (maxLeaf < 1 || maxLeaf > 16) throw std::runtime_error("max_leaf_size must lie in [1, 16]");
@@ -1160,6 +1160,7 @@ void BuildBvh4Device(const PrimSource& src, int maxLeaf, hipStream_t st, DeviceB
   }
   uint32_t stackNeed = 0;
   HipCheck(hipMemcpyAsync(&stackNeed, need, sizeof(uint32_t), hipMemcpyDeviceToHost, st), "stack need");
+  outputsValid = false;
   nodesOut.alloc(size_t(n4) * sizeof(BvhNode4));
   HipCheck(hipMemcpyAsync(nodesOut.ptr, nodes, size_t(n4) * sizeof(BvhNode4), hipMemcpyDeviceToDevice, st), "nodes");
   primsOut.alloc(size_t(n) * 48);

@@ -237,6 +237,9 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
     HostScene& h = scene->host;
     uint32_t n = uint32_t(h.prim_bounds.size() / 6);
     auto t0 = std::chrono::steady_clock::now();
+    // The scene has no tree from the first write to the buffers of the old one
+    // until the new one is complete, whatever fails in between; a failure before
+    // that write leaves the old tree in use.
     uint32_t nodeCount = 0, depth = 0, stackNeed = 0, largestLeaf = uint32_t(maxLeaf);
     float sah = 0.f;
     DeviceBuffer work;
@@ -257,7 +260,7 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
         if (prims) src.segs.push_back(sg);
         p += prims;
       }
-      BuildBvh4Device(src, maxLeaf, scene->ctx->stream, scene->d_nodes, scene->d_prims, work, ds);
+      BuildBvh4Device(src, maxLeaf, scene->ctx->stream, scene->d_nodes, scene->d_prims, scene->bvh_ready, work, ds);
       nodeCount = ds.node_count;
       depth = ds.depth;
       stackNeed = ds.stack_need;
@@ -272,6 +275,7 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
       std::vector<float4> ordered(3 * size_t(n));
       for (uint32_t i = 0; i < n; i++)
         for (int k = 0; k < 3; k++) ordered[3 * size_t(i) + k] = h.prim_records[3 * size_t(r.order[i]) + k];
+      scene->bvh_ready = false;
       scene->d_prims.upload(ordered.data(), ordered.size() * sizeof(float4), scene->ctx->stream);
       scene->d_nodes.upload(r.nodes.data(), r.nodes.size() * sizeof(BvhNode4), scene->ctx->stream);
       HipCheck(hipStreamSynchronize(scene->ctx->stream), "BVH upload");
@@ -282,13 +286,11 @@ rad_status rad_hip_bvh_build(rad_scene* scene, const rad_bvh_opts* opts) {
     }
     // The traversal keeps as many groups per ray (kGroupStackEntries); a deeper
     // need would drop subtrees (missed hits, light leaks), so such a tree is
-    // refused.  The scene keeps no half-built tree.
-    if (stackNeed > kTraceStackEntries) {
-      scene->bvh_ready = false;
+    // refused.
+    if (stackNeed > kTraceStackEntries)
       throw StatusError(RAD_ERR_UNSUPPORTED, "BVH needs " + std::to_string(stackNeed) +
                                                  " traversal stack entries; the traversal holds " +
                                                  std::to_string(kTraceStackEntries));
-    }
     scene->wide_count = BuildWideNodes(scene->d_nodes, nodeCount, largestLeaf, scene->d_prims, n, scene->ctx->stream, work,
                                        scene->d_wnodes);
     scene->builder = builder;

@@ -193,3 +193,33 @@ def test_leaf_at_the_host_builders_depth_limit(hip_ctx, leaf):
         assert np.array_equal(g.closest(rays), before)
     check_parity(o, rays, g.closest(rays), hb)
     assert np.array_equal(g.occluded(rays).astype(bool), hb["geom"] != 0xFFFFFFFF)
+
+
+def test_failed_rebuild(hip_ctx):
+    """A rebuild refused for its arguments leaves the tree in use; one that fails after it has written to the tree's
+    buffers (here: a stack need above 64) leaves the scene without one until a build succeeds."""
+    b, centres = nested_clumps(43)
+    g = hip.Scene.from_builder(hip_ctx, b, builder=F.RAD_BVH_DEVICE)
+    assert g.info().bvh_stack_need == 64  # the deepest that is traversed
+    rng = np.random.default_rng(1)
+    rays = np.zeros(6000, hip.RAY_DTYPE)
+    org = rng.normal(size=(6000, 3))
+    org = 3.0 * org / np.linalg.norm(org, axis=1, keepdims=True)
+    d = centres[rng.integers(len(centres), size=6000)] + rng.normal(0, 1e-3, (6000, 3)) - org
+    rays["o"], rays["d"], rays["tmax"] = org, d / np.linalg.norm(d, axis=1, keepdims=True), 3e38
+    hb = O.OracleScene(b).closest(rays, brute=True)
+    check_parity(O.OracleScene(b), rays, g.closest(rays), hb)
+    for kw in ({"max_leaf": 17}, {"builder": 7}):
+        with pytest.raises(hip.RadError) as e:
+            g.build_bvh(**kw)
+        assert e.value.status == 1
+        check_parity(O.OracleScene(b), rays, g.closest(rays), hb)
+    with pytest.raises(hip.RadError, match="stack") as e:
+        g.build_bvh(F.RAD_BVH_HOST)
+    assert e.value.status == 4
+    for query in (g.closest, g.occluded, lambda r: g.render(b.render_desc(spp=1, seed=1)), lambda r: g.bvh_check()):
+        with pytest.raises(hip.RadError) as e:
+            query(rays)
+        assert e.value.status == 7  # RAD_ERR_STATE
+    g.build_bvh(F.RAD_BVH_DEVICE)
+    check_parity(O.OracleScene(b), rays, g.closest(rays), hb)
