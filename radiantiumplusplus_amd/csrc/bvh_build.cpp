@@ -4,6 +4,7 @@
 // ulps so the device slab test never rejects a primitive the exact
 // primitive test would accept.
 #include "bvh_build.h"
+#include "bvh_wide.h"
 
 #include <algorithm>
 #include <atomic>
@@ -12,6 +13,7 @@
 #include <cstring>
 #include <future>
 #include <limits>
+#include <stdexcept>
 #include <thread>
 
 namespace rad {
@@ -363,6 +365,33 @@ uint32_t BvhStackNeed(const std::vector<BvhNode4>& nodes) {
     need[n] = inner ? inner - 1 + deepest : 0;
   }
   return need[0];
+}
+
+void BuildWideNodesHost(std::vector<BvhNode4>& nodes, uint32_t n, std::vector<BvhNode8>& wide, std::vector<uint32_t>& perm) {
+  wide.clear();
+  perm.assign(n, 0);
+  std::vector<WideJob> jobs{{0, kWideAll, 0, 0}};
+  uint32_t prims = 0;
+  bool bounded = true;
+  while (!jobs.empty()) {
+    const uint32_t next = uint32_t(wide.size() + jobs.size());
+    std::vector<WideJob> nextJobs;
+    uint32_t placed = 0;
+    for (const WideJob& jb : jobs) {
+      WideKids kids;
+      const unsigned long long sum = wide_count(nodes.data(), jb, kids);
+      const uint32_t inner = uint32_t(nextJobs.size()), prim0 = jb.mask & kWideRest ? jb.begin : prims + placed;
+      placed += uint32_t(sum >> 32);
+      if (placed > n - prims) throw std::runtime_error("traversal nodes exceed their buffers");
+      nextJobs.resize(inner + uint32_t(sum));
+      wide.emplace_back();
+      bounded &= wide_emit(nodes.data(), jb, kids, next + inner, prim0, wide.back(), nextJobs.data() + inner, perm.data());
+    }
+    prims += placed;
+    jobs = std::move(nextJobs);
+  }
+  if (prims != n) throw std::runtime_error("traversal nodes do not reference every primitive");
+  if (!bounded) throw std::runtime_error("BVH node bounds cannot be quantised (non-finite boxes?)");
 }
 
 uint32_t BvhLargestLeaf(const std::vector<BvhNode4>& nodes) {

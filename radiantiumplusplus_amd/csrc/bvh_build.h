@@ -24,6 +24,11 @@ struct BvhBuildResult {
 // that is not split apart after 60 levels is one leaf whatever its size.
 void BuildBvh4Host(const float* bounds, uint32_t count, int max_leaf, BvhBuildResult& out);
 
+// The traversal's nodes (bvh_wide.h) from a tree over n primitives: their leaf
+// order is given as perm (new place -> old place), and the leaves of `nodes` are
+// renumbered to match.  Throws if a child box cannot be bounded.
+void BuildWideNodesHost(std::vector<BvhNode4>& nodes, uint32_t n, std::vector<BvhNode8>& wide, std::vector<uint32_t>& perm);
+
 // SAH cost of a finished tree (traversal 1, intersection 1, relative to root area).
 float BvhSahCost(const std::vector<BvhNode4>& nodes);
 uint32_t BvhDepth(const std::vector<BvhNode4>& nodes);

@@ -144,23 +144,36 @@ __host__ __device__ inline void wide_order(const float l[3][8], const float h[3]
     for (int a = 0; a < 3; a++) d[a][i] = (l[a][i] + h[a][i]) - (lo[a] + hi[a]);
     slot[i] = 0;
   }
-  uint32_t used = 0, todo = valid;
+  // each child's best free slot; after a choice only children that wanted the
+  // same slot look again
+  float c[8];
+  uint32_t want[8], used = 0, todo = valid, again = valid;
   while (todo) {
+    uint32_t bi = 8;
     float best = -kInf;
-    uint32_t bi = 8, bs = 0;
 #pragma unroll
     for (uint32_t i = 0; i < 8; i++) {
-      if (!(todo >> i & 1u)) continue;
+      if (again >> i & 1u) {
+        want[i] = 8;
 #pragma unroll
-      for (uint32_t s = 0; s < 8; s++) {
-        const float c = (s & 1 ? d[0][i] : -d[0][i]) + (s & 2 ? d[1][i] : -d[1][i]) + (s & 4 ? d[2][i] : -d[2][i]);
-        if (!(used >> s & 1u) && (bi == 8 || c > best)) best = c, bi = i, bs = s;
+        for (uint32_t s = 0; s < 8; s++) {
+          const float v = (s & 1 ? d[0][i] : -d[0][i]) + (s & 2 ? d[1][i] : -d[1][i]) + (s & 4 ? d[2][i] : -d[2][i]);
+          if (!(used >> s & 1u) && (want[i] == 8 || v > c[i])) c[i] = v, want[i] = s;
+        }
       }
+      if ((todo >> i & 1u) && (bi == 8 || c[i] > best)) best = c[i], bi = i;
     }
+    uint32_t bs = 0;
 #pragma unroll
-    for (uint32_t i = 0; i < 8; i++) slot[i] = i == bi ? bs : slot[i];
+    for (uint32_t i = 0; i < 8; i++) {
+      bs = i == bi ? want[i] : bs;
+      slot[i] = i == bi ? want[i] : slot[i];
+    }
     todo &= ~(1u << bi);
     used |= 1u << bs;
+    again = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; i++) again |= (todo >> i & 1u) && want[i] == bs ? 1u << i : 0u;
   }
 }
 
@@ -178,13 +191,14 @@ __host__ __device__ inline bool quantize_axis(const float clo[8], const float ch
   }
   for (; e <= 127; e++) {
     biased = uint32_t(e + 127);
-    const float step = quant_step(biased);
+    const float step = quant_step(biased), inv = biased < 254 ? quant_step(254 - biased) : 0x1p-127f;  // 1 / step
     bool ok = true;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       if (!(valid >> i & 1u)) continue;
-      uint32_t a = uint32_t(fminf(fmaxf(floorf((clo[i] - o) / step), 0.f), top));
-      uint32_t c = uint32_t(fminf(fmaxf(ceilf((chi[i] - o) / step), 0.f), top));
+      const float y = fminf(fmaxf((chi[i] - o) * inv, 0.f), top);
+      uint32_t a = uint32_t(fminf(fmaxf((clo[i] - o) * inv, 0.f), top)), c = uint32_t(y);
+      if (float(c) < y) c++;
       while (a > 0 && dequant(a, step, o) > clo[i]) a--;
       while (c < kWidePlaneMax && dequant(c, step, o) < chi[i]) c++;
       if (!(dequant(a, step, o) <= clo[i] && dequant(c, step, o) >= chi[i])) ok = false;
@@ -243,7 +257,7 @@ __host__ __device__ inline unsigned long long wide_count(const BvhNode4* nodes, 
 // Bound by the latency of one thread's steps: the levels of a tree follow each
 // other and most are small.  Every array is indexed by constants, so that none
 // is in scratch memory or read through a loop over lanes (2.6 M primitives, 12
-// levels: 980 us with arrays indexed by slot, now 606).
+// levels: 980 us with arrays indexed by slot, now 504).
 __host__ __device__ inline bool wide_emit(BvhNode4* nodes, WideJob jb, const WideKids& kids, uint32_t child0, uint32_t prim0,
                                           BvhNode8& o, WideJob* next, uint32_t* perm) {
   const WideKids kd = kids;

@@ -13,42 +13,18 @@ extern "C" uint32_t probe_host_leaf(const float* bounds, uint32_t n, int max_lea
 }
 extern "C" uint32_t probe_max_leaf_prims() { return kMaxLeafPrims; }
 
-// The 8-wide nodes of a BvhNode4 tree over n primitives, level by level as the
-// device makes them.  Returns the errors found: primitives not placed exactly
+// The 8-wide nodes of a BvhNode4 tree over n primitives.  Returns the errors found: primitives not placed exactly
 // once, BvhNode4 leaves that do not name their primitives' new places, wide
 // leaves and children that do not lead to every primitive inside the boxes of
 // all nodes on the way.  out: nodes, the traversal's stack need, the BvhNode4
-// tree's, levels.
-static uint32_t Wide(std::vector<BvhNode4>& nodes, const float* bounds, const std::vector<uint32_t>& order, uint32_t out[4]) {
+// tree's.
+static uint32_t Wide(std::vector<BvhNode4>& nodes, const float* bounds, const std::vector<uint32_t>& order, uint32_t out[3]) {
   const uint32_t n = uint32_t(order.size());
   const std::vector<BvhNode4> before = nodes;
   std::vector<BvhNode8> wide;
-  std::vector<uint32_t> perm(n, kWideNone);
-  std::vector<WideJob> jobs{{0, kWideAll, 0, 0}};
-  uint32_t prims = 0, levels = 0, errors = 0;
-  while (!jobs.empty()) {
-    std::vector<WideKids> kids(jobs.size());
-    std::vector<unsigned long long> sums(jobs.size());
-    unsigned long long total = 0;
-    for (size_t j = 0; j < jobs.size(); j++) {
-      sums[j] = total;
-      total += wide_count(nodes.data(), jobs[j], kids[j]);
-    }
-    const uint32_t next = uint32_t(wide.size() + jobs.size());
-    std::vector<WideJob> nj(total & 0xffffffffu);
-    for (size_t j = 0; j < jobs.size(); j++) {
-      const uint32_t inner = uint32_t(sums[j]);
-      BvhNode8 o;
-      if (!wide_emit(nodes.data(), jobs[j], kids[j], next + inner,
-                     jobs[j].mask & kWideRest ? jobs[j].begin : prims + uint32_t(sums[j] >> 32), o, nj.data() + inner, perm.data()))
-        errors++;
-      wide.push_back(o);
-    }
-    prims += uint32_t(total >> 32);
-    jobs = nj;
-    levels++;
-  }
-  errors += prims != n;
+  std::vector<uint32_t> perm;
+  uint32_t errors = 0;
+  BuildWideNodesHost(nodes, n, wide, perm);
   std::vector<uint32_t> seen(n, 0), need(wide.size(), 0), reached(n, 0);
   for (uint32_t p : perm)
     if (p >= n || seen[p]++) errors++;
@@ -98,11 +74,10 @@ static uint32_t Wide(std::vector<BvhNode4>& nodes, const float* bounds, const st
   out[0] = uint32_t(wide.size());
   out[1] = need[0];
   out[2] = BvhStackNeed(nodes);
-  out[3] = levels;
   return errors;
 }
 
-extern "C" uint32_t probe_wide_host(const float* bounds, uint32_t n, int max_leaf, uint32_t out[4]) {
+extern "C" uint32_t probe_wide_host(const float* bounds, uint32_t n, int max_leaf, uint32_t out[3]) {
   BvhBuildResult r;
   BuildBvh4Host(bounds, n, max_leaf, r);
   return Wide(r.nodes, bounds, r.order, out);
@@ -110,7 +85,7 @@ extern "C" uint32_t probe_wide_host(const float* bounds, uint32_t n, int max_lea
 
 // A chain of `length` BvhNode4 with `inner` inner children (the others end in
 // one leaf) and leaves of the given sizes, primitive i at x = i.
-extern "C" uint32_t probe_wide_chain(uint32_t length, uint32_t inner, const uint32_t* leaves, uint32_t nLeaves, uint32_t out[4]) {
+extern "C" uint32_t probe_wide_chain(uint32_t length, uint32_t inner, const uint32_t* leaves, uint32_t nLeaves, uint32_t out[3]) {
   std::vector<BvhNode4> nodes;
   std::vector<float> bounds;
   std::vector<uint32_t> order;

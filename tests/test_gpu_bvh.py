@@ -223,3 +223,27 @@ def test_failed_rebuild(hip_ctx):
         assert e.value.status == 7  # RAD_ERR_STATE
     g.build_bvh(F.RAD_BVH_DEVICE)
     check_parity(O.OracleScene(b), rays, g.closest(rays), hb)
+
+
+@pytest.mark.parametrize("copies", [1, 6])
+@pytest.mark.parametrize("n", [60, 1500, 1700, 9000, 14000])
+def test_small_and_large_tree_paths(hip_ctx, n, copies):
+    """Triangle counts on both sides of the sizes at which the traversal's nodes are made on the host (host builder),
+    by one block and level by level: hits, ties between copies and the tree's structure."""
+    rng = np.random.default_rng(n)
+    t = rng.uniform(-1, 1, (n // copies, 1, 3)) + rng.normal(0, 0.1, (n // copies, 3, 3))
+    b = mesh_scene(np.concatenate([t] * copies))
+    o = O.OracleScene(b)
+    lo, hi = o.bounds()
+    rays = ray_batch(lo, hi, 2000, n)
+    hb = o.closest(rays, brute=True)
+    for builder in (F.RAD_BVH_DEVICE, F.RAD_BVH_HOST):
+        for max_leaf in (1, 4, 16):
+            g = hip.Scene.from_builder(hip_ctx, b, builder=builder, max_leaf=max_leaf)
+            r = g.bvh_check()
+            assert r.structure_errors == 0 and r.unreferenced_or_repeated == 0 and r.leaf_box_violations == 0
+            assert r.child_box_violations == 0 and r.quantized_box_violations == 0
+            h = g.closest(rays)
+            check_parity(o, rays, h, hb)
+            g.build_bvh(builder, max_leaf)  # again, into the buffers that are there
+            assert np.array_equal(h, g.closest(rays))
