@@ -210,6 +210,7 @@ void rad_hip_shutdown(rad_ctx* ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+  ctx->wide->release();
   delete ctx;
 }
 
@@ -220,6 +221,7 @@ rad_status rad_hip_scene_create(rad_ctx* ctx, const rad_scene_desc* desc, rad_sc
     HipCheck(hipSetDevice(ctx->device), "hipSetDevice");
     auto s = std::make_unique<rad_scene>();
     s->ctx = ctx;
+    s->wide = ctx->wide;
     AssembleScene(*desc, s->host);
     UploadScene(s.get());
     *out = s.release();
@@ -339,6 +341,8 @@ rad_status rad_hip_autotune(rad_scene* scene, const rad_render_desc* probe, rad_
   if (!scene || !probe || !rep) return Fail(RAD_ERR_INVALID_ARG, "NULL argument");
   return Guard([&] {
     RequireBvh(scene);
+    HipCheck(hipSetDevice(scene->ctx->device), "hipSetDevice");
+    scene->wide->release();  // the trials reach 64 M slots
     std::memset(rep, 0, sizeof(*rep));
     const uint64_t samples = uint64_t(probe->width > 0 ? probe->width : scene->host.cam.width) *
                              uint64_t(probe->height > 0 ? probe->height : scene->host.cam.height) * probe->spp;
@@ -559,6 +563,7 @@ rad_status rad_hip_scene_info(const rad_scene* scene, rad_scene_info* info) {
 void rad_hip_scene_destroy(rad_scene* scene) {
   if (!scene) return;
   (void)hipSetDevice(scene->ctx->device);
+  scene->wide->release(scene);
   delete scene;
 }
 

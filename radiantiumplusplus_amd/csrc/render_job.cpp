@@ -48,6 +48,7 @@ struct rad_job {
   uint32_t* tally = nullptr;  // RAD_RENDER_CHECK_QUEUES: tally words per extend-queue position (inside the arena)
   bool tally_selftest = false;
   bool joined = false;
+  bool wide = false;          // `arena` is the context's
 };
 
 namespace rad {
@@ -418,34 +419,67 @@ void ResolveLaunch(const rad_scene* scene, rad_render_desc& d) {
   }
 }
 
+// The context's wide arena of at least `need` bytes for a job of the scene;
+// null: another job has it, or it would take more than a quarter of the free
+// memory.
+static std::unique_ptr<DeviceBuffer> TakeWideArena(rad_scene* scene, uint64_t need) {
+  WideArena& w = *scene->wide;
+  HipCheck(hipSetDevice(scene->ctx->device), "hipSetDevice");
+  std::lock_guard<std::mutex> lk(w.mu);
+  if (w.busy) return nullptr;
+  std::unique_ptr<DeviceBuffer> a = std::move(w.buffer);
+  if (!a || a->bytes < need) {
+    a.reset();
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess || need > free / 4) return nullptr;
+    a = std::make_unique<DeviceBuffer>();
+    try {
+      a->alloc(need);
+    } catch (const std::exception&) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+  }
+  w.busy = true;
+  w.user = scene;
+  return a;
+}
+
 // Every iteration ends with a few long paths and starts with launches that fill
 // up: with four times the slots there are a quarter of the iterations.  64 spp
 // frames, 4 M / 8 M / 16 M / 32 M slots: cloud of dense grids 82.3 / 75.7 / 72.2
 // / 69.0 ms, 512^2 materials 8.65 / 7.89 / 7.89 ms, guided room 41.1 / - / 38.95
 // ms (64 M: 37.8).  16 M, as the arena grows with them: 1.5 GB at 4 M, 5.9 GB at
-// 16 M.  Not for
+// 16 M.  One arena of that size serves all scenes of a context, so a process
+// holds one more than with 4 M, however many scenes it has rendered.  Not for
+//  - a render while another has it: together they fill the device;
 //  - an arena above a quarter of the free memory: what else the process
-//    allocates has to fit beside the spare arenas of its scenes;
+//    allocates has to fit beside it;
 //  - served requests (they come by StartJob): they share a memory budget and
 //    fill the device together;
 //  - online guide training: the slots decide which vertices become records.
 rad_job* StartRender(rad_scene* scene, const rad_render_desc& desc) {
   rad_render_desc d = desc;
   ResolveLaunch(scene, d);
-  std::unique_ptr<DeviceBuffer> arena = TakeSpareArena(scene);
   if (desc.path_slots == 0 && scene->tuned_slots.load() == 0 && desc.guiding != 1) {
     rad_render_desc wide = d;
     wide.path_slots = kAloneSlots;
     const uint64_t need = Shape(scene, wide).bytes;
-    bool fits = arena && arena->bytes >= need;
-    if (!fits && need > Shape(scene, d).bytes) {
-      HipCheck(hipSetDevice(scene->ctx->device), "hipSetDevice");
-      size_t free = 0, total = 0;
-      fits = hipMemGetInfo(&free, &total) == hipSuccess && need <= free / 4;
+    if (need > Shape(scene, d).bytes) {
+      if (std::unique_ptr<DeviceBuffer> arena = TakeWideArena(scene, need)) {
+        try {
+          rad_job* job = StartJob(scene, wide, std::move(arena));
+          job->wide = true;
+          return job;
+        } catch (...) {
+          std::lock_guard<std::mutex> lk(scene->wide->mu);
+          scene->wide->busy = false;
+          throw;
+        }
+      }
     }
-    if (fits) d = wide;
   }
-  return StartJob(scene, d, std::move(arena));
+  return StartJob(scene, d, TakeSpareArena(scene));
 }
 
 uint64_t JobFootprint(const rad_scene* scene, const rad_render_desc& desc, uint32_t* slots) {
@@ -494,7 +528,13 @@ rad_job* StartJob(rad_scene* scene, const rad_render_desc& desc, std::unique_ptr
     job->arena = std::move(reuse);
   } else {
     job->arena = std::make_unique<DeviceBuffer>();
-    job->arena->alloc(js.bytes);
+    try {
+      job->arena->alloc(js.bytes);
+    } catch (const std::exception&) {
+      (void)hipGetLastError();
+      if (!scene->wide->release()) throw;
+      job->arena->alloc(js.bytes);
+    }
   }
   char* p = static_cast<char*>(job->arena->ptr);
   char* const end = p + job->arena->bytes;
@@ -657,8 +697,12 @@ void DestroyJob(rad_job* job) {
     (void)hipStreamDestroy(job->stream);
   }
   if (job->h_cnt) (void)hipHostFree(job->h_cnt);
-  if (job->arena) {  // keep the larger arena on the scene for its next job
-    rad_scene* sc = job->scene;
+  rad_scene* const sc = job->scene;
+  if (job->wide) {
+    std::lock_guard<std::mutex> lk(sc->wide->mu);
+    sc->wide->busy = false;
+    sc->wide->buffer = std::move(job->arena);
+  } else if (job->arena) {  // keep the larger arena on the scene for its next job
     std::lock_guard<std::mutex> lk(sc->arena_mu);
     if (!sc->spare_arena || sc->spare_arena->bytes < job->arena->bytes) sc->spare_arena = std::move(job->arena);
   }

@@ -23,7 +23,8 @@ struct StatusError : std::runtime_error {
 // its job see one launch configuration even if the autotuner runs between.
 void ResolveLaunch(const rad_scene* scene, rad_render_desc& desc);
 rad_job* StartJob(rad_scene* scene, const rad_render_desc& desc, std::unique_ptr<DeviceBuffer> reuse = nullptr);
-// A render on its own, its arena the scene's spare one if that is large enough.
+// A render that is not of a server: more paths in flight while it is the only
+// one of its context, its arena the context's or the scene's spare one.
 rad_job* StartRender(rad_scene* scene, const rad_render_desc& desc);
 bool JobComplete(const rad_job* job);
 // Detach the job's arena (joins its thread first) so a later job can reuse it.

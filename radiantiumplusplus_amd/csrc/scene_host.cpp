@@ -27,6 +27,13 @@ void DeviceBuffer::alloc(size_t n) {
   bytes = n;
 }
 
+bool WideArena::release(const rad_scene* of) {
+  std::lock_guard<std::mutex> lk(mu);
+  if (!buffer || (of && user != of)) return false;
+  buffer.reset();
+  return true;
+}
+
 void DeviceBuffer::upload(const void* src, size_t n, hipStream_t s) {
   alloc(std::max<size_t>(n, 16));
   if (n) HipCheck(hipMemcpyAsync(ptr, src, n, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
@@ -751,7 +758,12 @@ CameraRec MakeCameraRec(const rad_camera_desc& c) {
 }  // namespace rad
 
 uint64_t rad_scene::device_bytes() const {
-  return d_nodes.bytes + d_wnodes.bytes + d_prims.bytes + d_shapes.bytes + d_pos.bytes + d_nrm.bytes + d_uv.bytes + d_idx.bytes +
+  uint64_t arena = 0;
+  {
+    std::lock_guard<std::mutex> lk(wide->mu);
+    if (wide->buffer && wide->user == this) arena = wide->buffer->bytes;
+  }
+  return arena + d_nodes.bytes + d_wnodes.bytes + d_prims.bytes + d_shapes.bytes + d_pos.bytes + d_nrm.bytes + d_uv.bytes + d_idx.bytes +
          d_tris.bytes +
          d_bsdfs.bytes + d_lights.bytes + d_cdf.bytes + d_media.bytes + d_grid.bytes + d_tex.bytes + d_texels.bytes +
          d_ldist.bytes + (spare_arena ? spare_arena->bytes : 0);

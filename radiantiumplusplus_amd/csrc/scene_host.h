@@ -14,13 +14,7 @@
 #include "bvh_build.h"
 #include "scene_dev.h"
 
-struct rad_ctx {
-  int device = 0;
-  hipStream_t stream = nullptr;
-  void* scratch = nullptr;  // device address of this device's static staging array (capi.cpp)
-  std::string arch;
-  int cu_count = 0;
-};
+struct rad_scene;
 
 namespace rad {
 
@@ -72,10 +66,33 @@ struct DeviceBuffer {
   T* as() const { return reinterpret_cast<T*>(ptr); }
 };
 
+// The arena of a render with the device to itself (StartRender), one for all
+// scenes of a context: a job has it (busy), or it is kept for the next such
+// render until the scene that had it last is destroyed or the memory is needed.
+// Held by the context and its scenes, which may be destroyed in any order.
+struct WideArena {
+  std::mutex mu;
+  bool busy = false;
+  std::unique_ptr<DeviceBuffer> buffer;
+  const rad_scene* user = nullptr;  // scene of the last job that had it
+  // Frees the memory if no job has it (and, with `of`, if that scene had it
+  // last); true if there was any.
+  bool release(const rad_scene* of = nullptr);
+};
+
 std::string HipErr(hipError_t e);
 void HipCheck(hipError_t e, const char* what);
 
 }  // namespace rad
+
+struct rad_ctx {
+  int device = 0;
+  hipStream_t stream = nullptr;
+  void* scratch = nullptr;  // device address of this device's static staging array (capi.cpp)
+  std::string arch;
+  int cu_count = 0;
+  std::shared_ptr<rad::WideArena> wide = std::make_shared<rad::WideArena>();
+};
 
 namespace rad {
 namespace guide {
@@ -108,5 +125,6 @@ struct rad_scene {
   // competed with the first renders after each allocation.
   std::unique_ptr<rad::DeviceBuffer> spare_arena;
   std::mutex arena_mu;
+  std::shared_ptr<rad::WideArena> wide;  // the context's
   uint64_t device_bytes() const;
 };

@@ -205,6 +205,8 @@ extern "C" {
 
 rad_status rad_hip_server_create(rad_ctx* ctx, const rad_server_opts* opts, rad_server** out) {
   if (!ctx || !out) return Fail(RAD_ERR_INVALID_ARG, "NULL argument");
+  (void)hipSetDevice(ctx->device);
+  ctx->wide->release();  // the budget is for what the device holds beside the scenes
   auto s = std::make_unique<rad_server>();
   s->ctx = ctx;
   s->budget = opts && opts->hbm_budget ? opts->hbm_budget : (uint64_t(32) << 30);

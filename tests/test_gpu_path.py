@@ -9,7 +9,7 @@ import pytest
 import _oracle as O
 import stats
 from radiantiumplusplus_amd import _ffi as F
-from radiantiumplusplus_amd import hip, scenes
+from radiantiumplusplus_amd import hip, scenes, serve
 
 pytestmark = pytest.mark.gpu
 
@@ -287,3 +287,41 @@ def test_slots_chosen_by_the_library(hip_ctx, size, spp, guiding, slots):
     assert st.slots == slots and np.array_equal(a, c)
     e, _, st = s.render(b.render_desc(spp=spp, seed=3, path_slots=1 << 20))
     assert st.slots == min(1 << 20, size[0] * size[1] * spp) and np.array_equal(a, e)
+
+
+def test_one_wide_arena_for_all_scenes(hip_ctx):
+    """The 16 M slots of a render that leaves them to the library: a context holds one arena of that size, for one
+    render at a time.  A second render beside it has the default 4 M and the same image; the arena goes with the scene
+    that had it last, and to a server's creation."""
+    bs = [scenes.many_balls(seed=i, width=512, height=512, spp=80, n_spheres=8) for i in range(3)]
+    ss = [hip.Scene.from_builder(hip_ctx, b) for b in bs]
+    d = [b.render_desc(spp=80, seed=3) for b in bs]
+    base = [s.info().device_bytes for s in ss]
+    imgs, held = [], []
+    for s, r in zip(ss, d):
+        img, _, st = s.render(r)
+        assert st.slots == 16 << 20
+        imgs.append(img)
+        held.append([x.info().device_bytes - b0 for x, b0 in zip(ss, base)])
+    wide = held[0][0]
+    assert wide > 4 << 30
+    assert held == [[wide, 0, 0], [0, wide, 0], [0, 0, wide]]
+    jobs = [s.start(r) for s, r in zip(ss, d)]  # all in flight
+    for k, j in enumerate(jobs):
+        img, _, st = j.wait()
+        assert st.slots == (16 << 20 if k == 0 else 4 << 20) and np.array_equal(img, imgs[k])
+    for j in reversed(jobs):
+        j.close()
+    held = [x.info().device_bytes - b0 for x, b0 in zip(ss, base)]
+    assert held[0] == wide and 0 < held[1] < wide / 2 and 0 < held[2] < wide / 2  # their spare arenas
+    serve.Server(hip_ctx, hbm_budget=1 << 30).close()
+    assert ss[0].info().device_bytes == base[0]
+    _, _, st = ss[1].render(d[1])
+    assert st.slots == 16 << 20
+    bad = bs[0].render_desc(spp=80, seed=3)
+    bad.integrator = 7
+    with pytest.raises(hip.RadError):  # refused after the arena was taken: it is free again
+        ss[0].render(bad)
+    ss[1].close()
+    img, _, st = ss[2].render(d[2])
+    assert st.slots == 16 << 20 and np.array_equal(img, imgs[2])
