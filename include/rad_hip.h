@@ -358,12 +358,12 @@ typedef struct rad_bvh_report {
   uint32_t structure_errors;         /* out-of-range or repeated node references, unreachable nodes */
   uint32_t unreferenced_or_repeated; /* primitives not referenced exactly once by the leaves */
   uint32_t child_box_violations;     /* child boxes not inside the parent's slot box */
-  uint32_t leaf_box_violations;      /* triangles / spheres not inside their leaf box */
+  uint32_t leaf_box_violations;      /* primitives not inside their leaf box */
   float sah_cost;                    /* traversal 1, intersection 1, relative to the root box area */
   int32_t builder;
   uint32_t quantized_box_violations; /* errors of the traversal's quantised 8-wide nodes: dequantised child boxes
-                                        that do not contain the triangles and spheres below them, primitives or
-                                        nodes not referenced exactly once */
+                                        that do not contain the primitives below them, primitives or nodes not
+                                        referenced exactly once, a stack need above the traversal's 64 */
 } rad_bvh_report;
 typedef struct rad_scene_info {
   uint64_t primitive_count;

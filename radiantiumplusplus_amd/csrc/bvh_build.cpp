@@ -394,6 +394,62 @@ void BuildWideNodesHost(std::vector<BvhNode4>& nodes, uint32_t n, std::vector<Bv
   if (!bounded) throw std::runtime_error("BVH node bounds cannot be quantised (non-finite boxes?)");
 }
 
+uint32_t CheckWideNodes(const std::vector<BvhNode8>& wide, const float* boxes, uint32_t n, uint32_t* stackNeed) {
+  uint32_t errors = 0;
+  std::vector<uint8_t> seen(n, 0), parents(wide.size(), 0);
+  std::vector<uint32_t> need(wide.size(), 0);
+  std::vector<Box> below(wide.size());  // of the primitives below each node
+  const auto margin = [](float v) { return std::fabs(v) * 2.0f * 1.1920929e-7f + 5e-31f; };
+  for (size_t x = wide.size(); x-- > 0;) {  // children come after their parents
+    const BvhNode8& w = wide[x];
+    const uint16_t *lo[3] = {w.lox, w.loy, w.loz}, *hi[3] = {w.hix, w.hiy, w.hiz};
+    const float origin[3] = {w.ox, w.oy, w.oz};
+    uint32_t inner = 0, begin = 0;
+    for (int s = 0; s < 8; s++) {
+      const uint32_t end = (w.ends[s >> 2] >> (8 * (s & 3))) & 0xffu;
+      Box b;
+      if (w.exps >> 24 >> s & 1u) {
+        const uint32_t c = w.child_base + inner++;
+        if (c <= x || c >= wide.size()) {
+          errors++;
+          continue;
+        }
+        parents[c]++;
+        b = below[c];
+        need[x] = std::max(need[x], need[c]);
+      } else {
+        for (uint32_t k = begin; k < end; k++) {
+          const uint64_t p = uint64_t(w.prim_base) + k;
+          if (p >= n || k >= kWideNodePrims) {
+            errors++;
+            continue;
+          }
+          if (seen[p]++) errors++;
+          Box q;
+          std::memcpy(q.lo, boxes + 6 * p, 12);
+          std::memcpy(q.hi, boxes + 6 * p + 3, 12);
+          b.grow(q);
+        }
+      }
+      begin = end;
+      below[x].grow(b);
+      for (int a = 0; a < 3; a++) {
+        const float step = quant_step(w.exps >> (8 * a));
+        if (b.lo[a] <= b.hi[a] && !(dequant(plane_value(lo[a][s]), step, origin[a]) <= b.lo[a] - margin(b.lo[a]) &&
+                                    dequant(plane_value(hi[a][s]), step, origin[a]) >= b.hi[a] + margin(b.hi[a])))
+          errors++;
+      }
+    }
+    need[x] += inner > 1 ? 1u : 0u;
+  }
+  const uint32_t rootNeed = wide.empty() ? 0 : need[0];
+  if (stackNeed) *stackNeed = rootNeed;
+  errors += rootNeed > kGroupStackEntries;
+  for (uint32_t p = 0; p < n; p++) errors += seen[p] != 1;
+  for (size_t x = 0; x < wide.size(); x++) errors += parents[x] != (x ? 1 : 0);
+  return errors;
+}
+
 uint32_t BvhLargestLeaf(const std::vector<BvhNode4>& nodes) {
   uint32_t largest = 0;
   for (const BvhNode4& n : nodes)

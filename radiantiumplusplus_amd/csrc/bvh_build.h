@@ -29,6 +29,13 @@ void BuildBvh4Host(const float* bounds, uint32_t count, int max_leaf, BvhBuildRe
 // renumbered to match.  Throws if a child box cannot be bounded.
 void BuildWideNodesHost(std::vector<BvhNode4>& nodes, uint32_t n, std::vector<BvhNode8>& wide, std::vector<uint32_t>& perm);
 
+// Errors of the traversal's nodes over n primitives (boxes: six floats each, in
+// the order of the leaves): primitives not referenced exactly once, node
+// references out of range or repeated, child boxes that do not contain the
+// primitives below them with half the margin that the builders widen boxes by,
+// a stack need (to `need` if given) beyond the traversal's.
+uint32_t CheckWideNodes(const std::vector<BvhNode8>& wide, const float* boxes, uint32_t n, uint32_t* need = nullptr);
+
 // SAH cost of a finished tree (traversal 1, intersection 1, relative to root area).
 float BvhSahCost(const std::vector<BvhNode4>& nodes);
 uint32_t BvhDepth(const std::vector<BvhNode4>& nodes);

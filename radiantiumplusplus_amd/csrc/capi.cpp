@@ -2,7 +2,6 @@
 // BVH build, ray-batch intersection, asynchronous render jobs and the
 // per-function probes.  No exception crosses this boundary.
 #include <algorithm>
-#include <array>
 #include <atomic>
 #include <chrono>
 #include <cstdlib>
@@ -392,68 +391,25 @@ rad_status rad_hip_autotune(rad_scene* scene, const rad_render_desc* probe, rad_
   });
 }
 
-// Errors of the traversal's nodes: primitives not referenced exactly once,
-// node references out of range or repeated, child boxes that do not contain
-// the triangles and spheres below them, a stack need beyond the traversal's.
-static uint32_t CheckWideNodes(const std::vector<BvhNode8>& wide, const std::vector<float4>& prims, uint32_t n) {
-  uint32_t errors = 0;
-  std::vector<uint8_t> seen(n, 0), parents(wide.size(), 0);
-  std::vector<uint32_t> need(wide.size(), 0);
-  std::vector<std::array<float, 6>> bounds(wide.size());
-  for (size_t x = wide.size(); x-- > 0;) {  // children come after their parents
-    const BvhNode8& w = wide[x];
-    std::array<float, 6>& nb = bounds[x];
-    nb = {kInf, kInf, kInf, -kInf, -kInf, -kInf};
-    const float step[3] = {quant_step(w.exps), quant_step(w.exps >> 8), quant_step(w.exps >> 16)};
-    const float org[3] = {w.ox, w.oy, w.oz};
-    uint32_t inner = 0, begin = 0;
-    for (int s = 0; s < 8; s++) {
-      const uint32_t end = (w.ends[s >> 2] >> (8 * (s & 3))) & 0xffu;
-      std::array<float, 6> b = {kInf, kInf, kInf, -kInf, -kInf, -kInf};
-      if (w.exps >> 24 >> s & 1u) {
-        const uint32_t c = w.child_base + inner++;
-        if (c <= x || c >= wide.size()) {
-          errors++;
-          continue;
-        }
-        parents[c]++;
-        b = bounds[c];
-        need[x] = std::max(need[x], need[c]);
-      } else {
-        for (uint32_t k = begin; k < end; k++) {
-          const uint64_t p = uint64_t(w.prim_base) + k;
-          if (p >= n || k >= kWideNodePrims) {
-            errors++;
-            continue;
-          }
-          if (seen[p]++) errors++;
-          const float4 r[3] = {prims[3 * p], prims[3 * p + 1], prims[3 * p + 2]};
-          uint32_t kind;
-          std::memcpy(&kind, &r[2].w, 4);
-          if (kind == PRIM_RECT) continue;  // bounded through their shape transform
-          for (int v = 0; v < (kind == PRIM_TRI ? 3 : 1); v++) {
-            const float q[3] = {r[v].x, r[v].y, r[v].z}, rad = kind == PRIM_TRI ? 0.f : r[0].w;
-            for (int a = 0; a < 3; a++) b[a] = std::min(b[a], q[a] - rad), b[3 + a] = std::max(b[3 + a], q[a] + rad);
-          }
-        }
-      }
-      begin = end;
-      const uint16_t* lo[3] = {w.lox, w.loy, w.loz};
-      const uint16_t* hi[3] = {w.hix, w.hiy, w.hiz};
-      for (int a = 0; a < 3; a++) {
-        if (b[a] <= b[3 + a] && !(dequant(plane_value(lo[a][s]), step[a], org[a]) <= b[a] &&
-                                  dequant(plane_value(hi[a][s]), step[a], org[a]) >= b[3 + a]))
-          errors++;
-        nb[a] = std::min(nb[a], b[a]);
-        nb[3 + a] = std::max(nb[3 + a], b[3 + a]);
-      }
-    }
-    need[x] += inner > 1 ? 1u : 0u;
+// The scene's boxes (six floats) of n primitive records.
+static std::vector<float> PrimBoxes(const HostScene& h, const std::vector<float4>& prims, uint32_t n) {
+  std::vector<uint32_t> first;  // primitive of each shape
+  uint32_t total = 0;
+  for (const ShapeRec& s : h.shapes) {
+    first.push_back(total);
+    total += s.type == SHAPE_MESH ? s.tri_count : 1u;
   }
-  errors += !wide.empty() && need[0] > kGroupStackEntries;
-  for (uint32_t p = 0; p < n; p++) errors += seen[p] != 1;
-  for (size_t x = 0; x < wide.size(); x++) errors += parents[x] != (x ? 1 : 0);
-  return errors;
+  std::vector<float> box(6 * size_t(n));
+  for (size_t p = 0; p < n; p++) {
+    uint32_t kind, geom, id = 0;
+    std::memcpy(&kind, &prims[3 * p + 2].w, 4);
+    std::memcpy(&geom, kind == PRIM_TRI ? &prims[3 * p].w : &prims[3 * p + 1].w, 4);
+    if (kind == PRIM_TRI) std::memcpy(&id, &prims[3 * p + 1].w, 4);
+    const bool known = geom < first.size() && uint64_t(first[geom]) + id < total;
+    for (int k = 0; k < 6; k++)  // an unknown primitive is in no box
+      box[6 * p + k] = known ? h.prim_bounds[6 * (size_t(first[geom]) + id) + k] : k < 3 ? -kInf : kInf;
+  }
+  return box;
 }
 
 rad_status rad_hip_bvh_check(rad_scene* scene, rad_bvh_report* rep) {
@@ -471,6 +427,7 @@ rad_status rad_hip_bvh_check(rad_scene* scene, rad_bvh_report* rep) {
              "traversal nodes");
     HipCheck(hipMemcpy(prims.data(), scene->d_prims.ptr, prims.size() * sizeof(float4), hipMemcpyDeviceToHost), "prims");
     std::memset(rep, 0, sizeof(*rep));
+    const std::vector<float> box = PrimBoxes(scene->host, prims, n);
     std::vector<uint8_t> seen(n, 0), visited(m, 0);
     std::vector<uint32_t> stack{0}, depthOf{1};
     auto inside = [](float a0, float a1, float b0, float b1) { return b0 <= a0 && a1 <= b1; };
@@ -496,19 +453,7 @@ rad_status rad_hip_bvh_check(rad_scene* scene, rad_bvh_report* rep) {
               continue;
             }
             if (seen[p]++) rep->structure_errors++;
-            const float4 a = prims[3 * size_t(p)], b = prims[3 * size_t(p) + 1], c = prims[3 * size_t(p) + 2];
-            uint32_t kind;
-            std::memcpy(&kind, &c.w, 4);
-            float lo[3], hi[3];
-            if (kind == PRIM_TRI) {
-              lo[0] = std::min({a.x, b.x, c.x}), hi[0] = std::max({a.x, b.x, c.x});
-              lo[1] = std::min({a.y, b.y, c.y}), hi[1] = std::max({a.y, b.y, c.y});
-              lo[2] = std::min({a.z, b.z, c.z}), hi[2] = std::max({a.z, b.z, c.z});
-            } else if (kind == PRIM_SPHERE) {
-              lo[0] = a.x - a.w, hi[0] = a.x + a.w, lo[1] = a.y - a.w, hi[1] = a.y + a.w, lo[2] = a.z - a.w, hi[2] = a.z + a.w;
-            } else {
-              continue;  // rectangles: bounded through their shape transform
-            }
+            const float *lo = &box[6 * size_t(p)], *hi = lo + 3;
             if (!(inside(lo[0], hi[0], nd.lox[s], nd.hix[s]) && inside(lo[1], hi[1], nd.loy[s], nd.hiy[s]) &&
                   inside(lo[2], hi[2], nd.loz[s], nd.hiz[s])))
               rep->leaf_box_violations++;
@@ -535,7 +480,7 @@ rad_status rad_hip_bvh_check(rad_scene* scene, rad_bvh_report* rep) {
       if (seen[p] != 1) rep->unreferenced_or_repeated++;
     for (uint32_t x = 0; x < m; x++)
       if (!visited[x]) rep->structure_errors++;
-    rep->quantized_box_violations = CheckWideNodes(wide, prims, n);
+    rep->quantized_box_violations = CheckWideNodes(wide, box.data(), n);
     rep->node_count = m;
     rep->primitive_count = n;
     rep->sah_cost = BvhSahCost(nodes);

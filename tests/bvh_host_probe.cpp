@@ -13,74 +13,64 @@ extern "C" uint32_t probe_host_leaf(const float* bounds, uint32_t n, int max_lea
 }
 extern "C" uint32_t probe_max_leaf_prims() { return kMaxLeafPrims; }
 
-// The 8-wide nodes of a BvhNode4 tree over n primitives.  Returns the errors found: primitives not placed exactly
-// once, BvhNode4 leaves that do not name their primitives' new places, wide
-// leaves and children that do not lead to every primitive inside the boxes of
-// all nodes on the way.  out: nodes, the traversal's stack need, the BvhNode4
-// tree's.
-static uint32_t Wide(std::vector<BvhNode4>& nodes, const float* bounds, const std::vector<uint32_t>& order, uint32_t out[3]) {
+// The 8-wide nodes of a BvhNode4 tree over the primitives `order`.  Returns
+// the errors found: CheckWideNodes, primitives not placed exactly once,
+// BvhNode4 leaves that do not name their primitives' new places.  out: nodes,
+// the traversal's stack need, the BvhNode4 tree's.
+static uint32_t Wide(std::vector<BvhNode4>& nodes, const float* bounds, const std::vector<uint32_t>& order, uint32_t out[3],
+                     std::vector<BvhNode8>& wide, std::vector<float>& boxes) {
   const uint32_t n = uint32_t(order.size());
   const std::vector<BvhNode4> before = nodes;
-  std::vector<BvhNode8> wide;
-  std::vector<uint32_t> perm;
+  std::vector<uint32_t> perm, seen(n, 0);
   uint32_t errors = 0;
   BuildWideNodesHost(nodes, n, wide, perm);
-  std::vector<uint32_t> seen(n, 0), need(wide.size(), 0), reached(n, 0);
-  for (uint32_t p : perm)
-    if (p >= n || seen[p]++) errors++;
+  boxes.clear();
+  for (uint32_t p : perm) {
+    if (p >= n || seen[p]++) return 1;
+    boxes.insert(boxes.end(), bounds + 6 * size_t(order[p]), bounds + 6 * size_t(order[p]) + 6);
+  }
   for (size_t x = 0; x < nodes.size(); x++)
     for (int s = 0; s < 4; s++)
       for (uint32_t q = 0; q < nodes[x].count[s]; q++) errors += perm[nodes[x].child[s] + q] != before[x].child[s] + q;
-  struct Box {
-    float lo[3], hi[3];
-  };
-  std::vector<Box> box(wide.size());  // of the primitives below
-  for (size_t x = wide.size(); x-- > 0;) {
-    const BvhNode8& w = wide[x];
-    Box nb{{kInf, kInf, kInf}, {-kInf, -kInf, -kInf}};
-    uint32_t inner = 0, begin = 0;
-    for (int s = 0; s < 8; s++) {
-      const uint32_t end = (w.ends[s >> 2] >> (8 * (s & 3))) & 0xffu;
-      Box b{{kInf, kInf, kInf}, {-kInf, -kInf, -kInf}};
-      if (w.exps >> 24 >> s & 1u) {
-        const uint32_t c = w.child_base + inner++;
-        if (c <= x || c >= wide.size()) return errors + 1;
-        b = box[c];
-        need[x] = std::max(need[x], need[c]);
-      } else {
-        for (uint32_t k = begin; k < end; k++) {
-          if (k >= kWideNodePrims || w.prim_base + k >= n) return errors + 1;
-          reached[w.prim_base + k]++;
-          const float* p = bounds + 6 * size_t(order[perm[w.prim_base + k]]);
-          for (int a = 0; a < 3; a++) b.lo[a] = std::min(b.lo[a], p[a]), b.hi[a] = std::max(b.hi[a], p[3 + a]);
-        }
-      }
-      begin = end;
-      const uint16_t* lo[3] = {w.lox, w.loy, w.loz};
-      const uint16_t* hi[3] = {w.hix, w.hiy, w.hiz};
-      const float org[3] = {w.ox, w.oy, w.oz};
-      for (int a = 0; a < 3; a++) {
-        const float step = quant_step(w.exps >> (8 * a));
-        if (b.lo[a] <= b.hi[a])
-          errors += !(dequant(plane_value(lo[a][s]), step, org[a]) <= b.lo[a] && dequant(plane_value(hi[a][s]), step, org[a]) >= b.hi[a]);
-        nb.lo[a] = std::min(nb.lo[a], b.lo[a]);
-        nb.hi[a] = std::max(nb.hi[a], b.hi[a]);
-      }
-    }
-    need[x] += inner > 1 ? 1 : 0;
-    box[x] = nb;
-  }
-  for (uint32_t r : reached) errors += r != 1;
   out[0] = uint32_t(wide.size());
-  out[1] = need[0];
   out[2] = BvhStackNeed(nodes);
-  return errors;
+  return errors + CheckWideNodes(wide, boxes.data(), n, &out[1]);
 }
 
 extern "C" uint32_t probe_wide_host(const float* bounds, uint32_t n, int max_leaf, uint32_t out[3]) {
   BvhBuildResult r;
   BuildBvh4Host(bounds, n, max_leaf, r);
-  return Wide(r.nodes, bounds, r.order, out);
+  std::vector<BvhNode8> wide;
+  std::vector<float> boxes;
+  return Wide(r.nodes, bounds, r.order, out, wide, boxes);
+}
+
+// CheckWideNodes of a host-built tree in which one thing of node x is wrong:
+// what 0-5 a plane (lo / hi of x, y, z) of child slot s is moved inside its
+// box, 6 its primitives and 7 its inner children are the next ones.  -1: the
+// node has no such thing.
+extern "C" int32_t probe_wide_broken(const float* bounds, uint32_t n, uint32_t x, int s, int what) {
+  BvhBuildResult r;
+  BuildBvh4Host(bounds, n, 4, r);
+  std::vector<BvhNode8> wide;
+  std::vector<float> boxes;
+  uint32_t out[3];
+  if (Wide(r.nodes, bounds, r.order, out, wide, boxes)) return -2;
+  x %= uint32_t(wide.size());
+  BvhNode8& w = wide[x];
+  uint16_t* plane[6] = {w.lox, w.hix, w.loy, w.hiy, w.loz, w.hiz};
+  if (what < 6) {
+    const uint32_t lo = plane_value(plane[what & ~1][s]), hi = plane_value(plane[what | 1][s]);
+    if (lo >= hi) return -1;  // an empty slot
+    plane[what][s] = plane_bits(what & 1 ? lo : hi);
+  } else if (what == 6) {
+    if ((w.ends[1] >> 24) == 0) return -1;
+    w.prim_base++;
+  } else {
+    if (!(w.exps >> 24)) return -1;
+    w.child_base++;
+  }
+  return int32_t(CheckWideNodes(wide, boxes.data(), n));
 }
 
 // A chain of `length` BvhNode4 with `inner` inner children (the others end in
@@ -127,5 +117,13 @@ extern "C" uint32_t probe_wide_chain(uint32_t length, uint32_t inner, const uint
     nodes[x].lox[s] = nodes[x].loy[s] = nodes[x].loz[s] = 0.f;
     nodes[x].hix[s] = float(order.size()), nodes[x].hiy[s] = nodes[x].hiz[s] = 1.f;
   }
-  return Wide(nodes, bounds.data(), order, out);
+  for (BvhNode4& nd : nodes)
+    for (int s = 0; s < 4; s++) {
+      if (nd.child[s] < 0) continue;
+      nd.lox[s] = Widen(nd.lox[s], false), nd.loy[s] = Widen(nd.loy[s], false), nd.loz[s] = Widen(nd.loz[s], false);
+      nd.hix[s] = Widen(nd.hix[s], true), nd.hiy[s] = Widen(nd.hiy[s], true), nd.hiz[s] = Widen(nd.hiz[s], true);
+    }
+  std::vector<BvhNode8> wide;
+  std::vector<float> boxes;
+  return Wide(nodes, bounds.data(), order, out, wide, boxes);
 }
