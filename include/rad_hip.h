@@ -302,7 +302,8 @@ typedef struct rad_render_desc {
   uint32_t request_id;     /* RNG stream key for serving (0 for single renders) */
   int32_t width, height;   /* image size override (0 = the scene camera's); fov and pose are the scene's */
   uint32_t blocks_per_cu;        /* persistent grid of the per-path kernels (0 = tuned / default) */
-  uint32_t trace_blocks_per_cu;  /* persistent grid of the traversal kernels (0 = tuned / default) */
+  uint32_t trace_blocks_per_cu;  /* persistent grid of the traversal kernels (0 = tuned / default); rays are dealt to
+                                    the waves of at most 5 blocks per CU */
 } rad_render_desc;
 
 typedef struct rad_job_stats {

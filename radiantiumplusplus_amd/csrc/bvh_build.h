@@ -1,6 +1,6 @@
 // Acceleration-structure builders.  Both produce the same 4-wide node layout
-// (BvhNode4) over a primitive permutation; the device traversal is agnostic
-// of which builder ran.  Replaces the Embree BVH build (embree.cpp:18-43).
+// (BvhNode4) over a primitive permutation; the traversal's 8-wide nodes are made
+// from it whichever builder ran.  Replaces the Embree BVH build (embree.cpp:18-43).
 #pragma once
 
 #include <cstdint>

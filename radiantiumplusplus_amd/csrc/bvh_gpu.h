@@ -1,5 +1,6 @@
-// Device BVH builder: Morton-ordered primitives, level-synchronous binned
-// SAH splits, collapse to the 4-wide node layout of the traversal.
+// Device BVH builder: Morton-ordered primitives, level-synchronous binned SAH
+// splits, collapse to 4-wide nodes; and the traversal's 8-wide nodes from the
+// 4-wide tree of either builder.
 #pragma once
 
 #include <cstdint>

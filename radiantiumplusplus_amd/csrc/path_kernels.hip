@@ -69,8 +69,9 @@ __device__ __forceinline__ void finish_records(const Wavefront& w, uint32_t s, f
 // sample row after the other.  The rays that a launch has in flight, and the
 // bounces that follow, then come from a small part of the image, so the part of
 // the tree and of the triangle records that they touch stays in L2 longer
-// than with one sample of the whole image after the other (1080p large mesh
-// 126.0 -> 123.5 ms, 637x397 materials 10.2 -> 9.8, volume 113.4 -> 109.7).
+// than with one sample of the whole image after the other (whole renders, best
+// of five of one seed: 1080p large mesh 126.0 -> 123.5 ms, 637x397 materials 10.2
+// -> 9.8, volume 113.4 -> 109.7).
 __device__ __forceinline__ void pass_sample(uint32_t id, uint32_t W, uint32_t H, uint32_t rows, uint32_t& px, uint32_t& py,
                                             uint32_t& row) {
   constexpr uint32_t T = 8;

@@ -27,8 +27,8 @@ struct alignas(128) BvhNode4 {
 };
 static_assert(sizeof(BvhNode4) == 128, "BVH node must be one 128-byte line");
 
-// Entries of a traversal stack (node, entry distance).  A node visit pushes
-// all but the nearest of its hit inner children, so a tree needs at most
+// Most entries of a stack of nodes that a 4-wide traversal of the BvhNode4 tree
+// may need.  A visit pushes all but one of the hit inner children, so it needs
 // need(n) = (inner children of n - 1) + max over inner children c of need(c)
 // entries (0 for a node whose children are all leaves); the builders compute
 // need(root) and a tree that needs more than this is refused.
@@ -39,8 +39,8 @@ constexpr uint32_t kTraceStackEntries = 64;
 // same way (the nodes of a chain, bvh_wide.h, have one but for the last), so
 // the need is at most the BvhNode4 tree's.
 constexpr uint32_t kGroupStackEntries = kTraceStackEntries;
-// Entries of a wave's pooled primitive tests per node step (traverse.h); a
-// lane whose entries fall beyond the pool tests them itself.
+// Entries of a wave's pooled primitive tests (traverse.h); what falls beyond
+// the pool waits for the next round of tests.
 constexpr uint32_t kTracePool = 64;
 
 // The traversal's node: up to eight children, one 128-byte L2 line, built from

@@ -51,9 +51,9 @@ struct ExtendJob {
   }
 };
 
-// The traversal kernels are capped at 96 VGPRs (five waves per SIMD, nothing
-// spills): they wait on node loads more than half of a wave's time, and
-// resident waves hide that.  1080p 64-spp large-mesh frame, extension rays
+// The traversal kernels are capped at 96 VGPRs (five waves per SIMD; nothing
+// spills, two to five registers with 64-bit node addresses): they wait on node
+// loads more than half of a wave's time, and resident waves hide that.  1080p 64-spp large-mesh frame, extension rays
 // 62.8 ms at four waves, 62.5 at five, 74.3 at six (42 registers spill).  Over
 // the 4-wide tree with primitives tested every step they took 68 ms
 // (0.88 of the SIMD cycles issuing, 0.46 of the lanes active; now 0.62 and

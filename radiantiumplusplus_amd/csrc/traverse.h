@@ -547,7 +547,11 @@ constexpr uint32_t kPoolSize = kTracePool;
 // (two per SIMD: 1024 to 4096 measured alike, without it a 64x48 render's
 // traversal took 8 % longer) and fewest lanes of a wave.
 constexpr uint32_t kSpreadWaves = 2048, kMinLanes = 8;
-constexpr uint32_t kResidentWaves = 5 * 4 * 256;  // five per SIMD (the traversal kernels' registers), 256 CUs
+// Waves that rays are dealt to: those resident at once where the kernel has the
+// device to itself, five per SIMD (the traversal kernels' registers) on 256 CUs.
+// A grid of more (trace_blocks_per_cu above 5) only adds waves that start
+// and leave.
+constexpr uint32_t kResidentWaves = 5 * 4 * 256;
 
 template <bool ANY, bool FAR, class Job>
 __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint32_t* fetch, uint32_t per_wave, Job& job) {
@@ -599,7 +603,8 @@ __device__ __forceinline__ void trace_stream(const DevScene& s, uint32_t n, uint
     // Finished closest-hit rays are written out here, together: a wave's 64
     // rays end a few at a time, and recomputing and storing the hit in the
     // step in which its ray ended ran that code with about four lanes active
-    // in nearly every step (1080p large-mesh frame 145.6 -> 138.0 ms).  An
+    // in nearly every step (1080p large-mesh frame, on
+    // 4-wide nodes, 145.6 -> 138.0 ms).  An
     // any-hit ray has one byte or nothing to write and does so when it ends.
     if (!ANY && have && !active && !pend) {
       trace_finish(s, r);

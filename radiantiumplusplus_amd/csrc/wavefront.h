@@ -8,10 +8,10 @@
 // per queue, by position).  Whoever appends a path to the next queue moves
 // its state there, so every kernel reads and writes path state in queue
 // order, never scattered by a slot number.  Camera samples are
-// handed out from a global counter in sample-major order (id -> pixel
-// id % pixels, sample row0 + id / pixels), so the queue stays full until
-// the pass runs out of samples and the primary rays of a wave are adjacent
-// pixels.  A finished sample's radiance goes to its own 16-byte result
+// handed out from a global counter, 8 x 8 pixel tile by tile and within a tile
+// one sample row after the other (pass_sample, path_kernels.hip), so the queue
+// stays full until the pass runs out of samples and the primary rays of a wave
+// are one tile.  A finished sample's radiance goes to its own 16-byte result
 // entry; after the pass, k_accum adds the entries of each pixel in sample
 // order (the order of sample_renderer.cpp:97-105), so the image does not
 // depend on which path ran which sample.  Each iteration runs

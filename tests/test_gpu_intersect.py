@@ -103,11 +103,11 @@ def test_empty_batch_and_bvh_info(hip_ctx):
 
 @pytest.mark.parametrize("pool", [1, 5])
 def test_primitives_beyond_the_wave_pool(hip_ctx, monkeypatch, pool):
-    """A wave tests up to 64 leaf primitives per node step as one pool; a
-    lane whose entries fall beyond it tests them itself.  RAD_TRACE_POOL
-    shrinks the pool so that this path carries most primitives: hits must
-    still match the brute force, and images must equal the full pool's bit
-    for bit (the closest hit is the minimum of (t, primitive) either way)."""
+    """A wave tests up to 64 leaf primitives at a time as one pool; what falls
+    beyond it waits for the next round.  RAD_TRACE_POOL shrinks the pool so
+    that most primitives wait: hits must still match the brute force, and
+    images must equal the full pool's bit for bit (the closest hit is the
+    minimum of (t, primitive) either way)."""
     b = scenes.many_balls(seed=6, n_spheres=64, slices=32, width=24, height=24)
     o = O.OracleScene(b)
     full = hip.Scene.from_builder(hip_ctx, b)
