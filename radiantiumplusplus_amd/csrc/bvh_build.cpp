@@ -385,7 +385,7 @@ void BuildWideNodesHost(std::vector<BvhNode4>& nodes, uint32_t n, std::vector<Bv
       if (placed > n - prims) throw std::runtime_error("traversal nodes exceed their buffers");
       nextJobs.resize(inner + uint32_t(sum));
       wide.emplace_back();
-      bounded &= wide_emit(nodes.data(), jb, kids, next + inner, prim0, wide.back(), nextJobs.data() + inner, perm.data());
+      bounded &= wide_emit(nodes.data(), jb, kids, next + inner, prim0, &wide.back(), nextJobs.data() + inner, perm.data());
     }
     prims += placed;
     jobs = std::move(nextJobs);

@@ -899,11 +899,9 @@ __global__ void __launch_bounds__(64) k_wide(const WideJob* jobs, uint32_t nJobs
     return;
   }
   const uint32_t inner = uint32_t(sums[j]), prims = uint32_t(sums[j] >> 32);
-  BvhNode8 o;
-  if (!wide_emit(nodes, jb, kids[j], lv.next + inner, jb.mask & kWideRest ? jb.begin : lv.prims + prims, o, next + inner,
-                        perm))
+  if (!wide_emit(nodes, jb, kids[j], lv.next + inner, jb.mask & kWideRest ? jb.begin : lv.prims + prims, out + lv.nodes + j,
+                 next + inner, perm))
     atomicOr(error, 1u);
-  out[lv.nodes + j] = o;
 }
 
 // All levels of a small tree in one block: a level of k_wide costs two launches,
@@ -911,8 +909,8 @@ __global__ void __launch_bounds__(64) k_wide(const WideJob* jobs, uint32_t nJobs
 // of a level are taken in groups of kWideThreads with running sums, so the
 // nodes are those of the level passes.  Bound, as k_wide, by the latency of one
 // thread's steps, here on one compute unit.  Whole builds, level passes / one
-// block: 82 nodes of the 4-wide tree 1414 / 1269 us, 1611 2538 / 2364, 3651
-// 3025 / 2925, 8720 3281 / 3602.
+// block: 82 nodes of the 4-wide tree 1321 / 1251 us, 1611 2408 / 2302, 3651
+// 2897 / 2862, 8720 3123 / 3501.
 constexpr int kWideThreads = 512;
 constexpr uint32_t kWideTreeNodes = 4096;  // largest 4-wide tree made so
 struct WideTotals {
@@ -962,11 +960,9 @@ __global__ void __launch_bounds__(kWideThreads) k_wide_tree(WideJob* cur, WideJo
       }
       if (mine) {
         const uint32_t inner = uint32_t(before);
-        BvhNode8 o;
-        if (!wide_emit(nodes, jb, kids[j], next + inner, jb.mask & kWideRest ? jb.begin : prims + uint32_t(before >> 32), o,
-                       nxt + inner, perm))
+        if (!wide_emit(nodes, jb, kids[j], next + inner, jb.mask & kWideRest ? jb.begin : prims + uint32_t(before >> 32),
+                       out + first + j, nxt + inner, perm))
           sBad = 1;
-        out[first + j] = o;
       }
       __syncthreads();  // sWave is read; the next level's jobs are written
     }

@@ -4,6 +4,7 @@
 #pragma once
 
 #include <cmath>
+#include <cstddef>
 #include <cstdint>
 
 #include "scene_dev.h"
@@ -107,7 +108,8 @@ __host__ __device__ inline int wide_children(const BvhNode4* nodes, uint32_t roo
 // part is placed has its parts in nodes of their own, one after the other, so
 // that its primitives stay consecutive.  Every node places primitives or the
 // last inner children, so a chain ends.
-__host__ __device__ inline void chain_children(const BvhNode4& nd, const WideJob& jb, uint32_t kid[8], uint32_t cnt[8], WideJob& rest) {
+__host__ __device__ inline void chain_children(const BvhNode4& nd, const WideJob& jb, uint32_t kid[8], uint32_t cnt[8],
+                                               WideJob& rest) {
   for (int i = 0; i < 8; i++) kid[i] = kWideNone, cnt[i] = 0;
   uint32_t left = 0, acc = 0;  // children still to be placed, primitives taken
   for (uint32_t s = 0; s < 4; s++) left |= nd.child[s] >= 0 ? jb.mask & 1u << s : 0u;
@@ -136,8 +138,8 @@ __host__ __device__ inline void chain_children(const BvhNode4& nd, const WideJob
 // slot[i]: the slot of child i (of those in `valid`), chosen greedily so that
 // bit a of a slot says on which side of the node's centre the child's centre
 // lies along axis a.
-__host__ __device__ inline void wide_order(const float l[3][8], const float h[3][8], uint32_t valid, const float lo[3],
-                                           const float hi[3], uint32_t slot[8]) {
+RAD_HD void wide_order(const float l[3][8], const float h[3][8], uint32_t valid, const float lo[3], const float hi[3],
+                       uint32_t slot[8]) {
   float d[3][8];
 #pragma unroll
   for (int i = 0; i < 8; i++) {
@@ -181,8 +183,8 @@ __host__ __device__ inline void wide_order(const float l[3][8], const float h[3]
 // extent (raised further if rounding keeps a bound out of reach), and the
 // children's planes qlo, qhi in it, rounded outward and verified with the
 // traversal's own dequantisation.
-__host__ __device__ inline bool quantize_axis(const float clo[8], const float chi[8], uint32_t valid, float o, float ext,
-                                              uint32_t& biased, uint32_t qlo[8], uint32_t qhi[8]) {
+RAD_HD bool quantize_axis(const float clo[8], const float chi[8], uint32_t valid, float o, float ext, uint32_t& biased,
+                          uint32_t qlo[8], uint32_t qhi[8]) {
   constexpr float top = float(kWidePlaneMax);
   int e = -126;
   if (ext > 0.f) {
@@ -210,8 +212,9 @@ __host__ __device__ inline bool quantize_axis(const float clo[8], const float ch
   return false;
 }
 
-// The planes of eight slots from those of the children.
-__host__ __device__ inline void place_planes(const uint32_t q[8], const uint32_t slot[8], uint32_t valid, uint32_t empty, uint16_t out[8]) {
+// The planes of eight slots from those of the children, to the 16-byte chunk
+// `out`.
+RAD_HD void place_planes(const uint32_t q[8], const uint32_t slot[8], uint32_t valid, uint32_t empty, char* out) {
   uint32_t w[4] = {0, 0, 0, 0}, used = 0;
 #pragma unroll
   for (int i = 0; i < 8; i++) {
@@ -222,7 +225,8 @@ __host__ __device__ inline void place_planes(const uint32_t q[8], const uint32_t
     for (uint32_t v = 0; v < 4; v++) w[v] |= slot[i] >> 1 == v ? b : 0u;
   }
 #pragma unroll
-  for (uint32_t s = 0; s < 8; s++) out[s] = used >> s & 1u ? uint16_t(w[s >> 1] >> (16 * (s & 1u))) : uint16_t(empty);
+  for (uint32_t s = 0; s < 8; s++) w[s >> 1] |= used >> s & 1u ? 0u : empty << (16 * (s & 1u));
+  __builtin_memcpy(__builtin_assume_aligned(out, 16), w, 16);
 }
 
 // First pass over a job: its children go to `kids`; returns how many of them
@@ -256,10 +260,11 @@ __host__ __device__ inline unsigned long long wide_count(const BvhNode4* nodes, 
 //
 // Bound by the latency of one thread's steps: the levels of a tree follow each
 // other and most are small.  Every array is indexed by constants, so that none
-// is in scratch memory or read through a loop over lanes (2.6 M primitives, 12
-// levels: 980 us with arrays indexed by slot, now 504).
-__host__ __device__ inline bool wide_emit(BvhNode4* nodes, WideJob jb, const WideKids& kids, uint32_t child0, uint32_t prim0,
-                                          BvhNode8& o, WideJob* next, uint32_t* perm) {
+// is in scratch memory or read through a loop over lanes, and the axes share
+// their code, which a launch reads anew (60 KB with three copies, now 31; 2.6 M
+// primitives, 12 levels: 980 us with arrays indexed by slot, now 501).
+RAD_HD bool wide_emit(BvhNode4* nodes, WideJob jb, const WideKids& kids, uint32_t child0, uint32_t prim0, BvhNode8* out,
+                      WideJob* next, uint32_t* perm) {
   const WideKids kd = kids;
   const bool chain = is_chain(nodes[jb.n4], jb);
   uint32_t cnt[8], valid = 0;  // cnt: primitives of a leaf, 0: inner
@@ -325,28 +330,37 @@ __host__ __device__ inline bool wide_emit(BvhNode4* nodes, WideJob jb, const Wid
     for (uint32_t q = 0; q < cnt[i]; q++) perm[begin + q] = from + q;
     if (!chain || skip + cnt[i] == leaf.count[s]) leaf.child[s] = int32_t(begin - skip);
   }
-  uint32_t bx = 127, by = 127, bz = 127, qx[2][8], qy[2][8], qz[2][8];
+  // one axis after the other through the same code
+  static_assert(offsetof(BvhNode8, lox) == 0 && offsetof(BvhNode8, hix) == 16 && offsetof(BvhNode8, loz) == 48 &&
+                    offsetof(BvhNode8, loy) == 64 && offsetof(BvhNode8, hiy) == 96 && offsetof(BvhNode8, hiz) == 112,
+                "plane chunks");
+  char* const chunk = reinterpret_cast<char*>(out);
+  uint32_t exps = imask << 24;
+  out->ox = lo[0];
+  out->oy = lo[1];
+  out->oz = lo[2];
+  bool ok = true;
+#pragma nounroll
+  for (int a = 0; a < 3; a++) {
+    uint32_t biased = 127, q[2][8] = {};
+    ok = quantize_axis(l[0], h[0], valid, lo[0], hi[0] - lo[0], biased, q[0], q[1]) && ok;
+    exps |= (biased & 0xffu) << (8 * a);
+    // an empty slot: an inverted box
+    place_planes(q[0], slot, valid, plane_bits(kWidePlaneMax), chunk + (a == 0 ? 0 : a == 1 ? 64 : 48));
+    place_planes(q[1], slot, valid, 0, chunk + (a == 0 ? 16 : a == 1 ? 96 : 112));
 #pragma unroll
-  for (int i = 0; i < 8; i++)
-    for (int k = 0; k < 2; k++) qx[k][i] = qy[k][i] = qz[k][i] = 0;
-  const bool ok = quantize_axis(l[0], h[0], valid, lo[0], hi[0] - lo[0], bx, qx[0], qx[1]) &&
-                  quantize_axis(l[1], h[1], valid, lo[1], hi[1] - lo[1], by, qy[0], qy[1]) &&
-                  quantize_axis(l[2], h[2], valid, lo[2], hi[2] - lo[2], bz, qz[0], qz[1]);
-  const uint32_t none = plane_bits(kWidePlaneMax);  // an empty slot: an inverted box
-  place_planes(qx[0], slot, valid, none, o.lox);
-  place_planes(qx[1], slot, valid, 0, o.hix);
-  place_planes(qy[0], slot, valid, none, o.loy);
-  place_planes(qy[1], slot, valid, 0, o.hiy);
-  place_planes(qz[0], slot, valid, none, o.loz);
-  place_planes(qz[1], slot, valid, 0, o.hiz);
-  o.ox = lo[0];
-  o.oy = lo[1];
-  o.oz = lo[2];
-  o.exps = bx | by << 8 | bz << 16 | imask << 24;
-  o.child_base = child0;
-  o.prim_base = prim0;
-  o.ends[0] = ends[0];
-  o.ends[1] = ends[1];
+    for (int i = 0; i < 8; i++) {
+      l[0][i] = l[1][i], l[1][i] = l[2][i];
+      h[0][i] = h[1][i], h[1][i] = h[2][i];
+    }
+    lo[0] = lo[1], lo[1] = lo[2];
+    hi[0] = hi[1], hi[1] = hi[2];
+  }
+  out->exps = exps;
+  out->child_base = child0;
+  out->prim_base = prim0;
+  out->ends[0] = ends[0];
+  out->ends[1] = ends[1];
   return ok;
 }
 

@@ -80,8 +80,7 @@ constexpr uint32_t kMaxLeafPrims = 255;
 // binary16 bits of an integer 0..2047, and back.
 __host__ __device__ inline uint16_t plane_bits(uint32_t q) {
   if (q == 0) return 0;
-  int e = 0;
-  while (q >> (e + 1)) e++;
+  const int e = 31 - __builtin_clz(q);
   return uint16_t(((e + 15) << 10) | ((q << (10 - e)) & 0x3ffu));
 }
 __host__ __device__ inline uint32_t plane_value(uint16_t h) {
