@@ -419,6 +419,13 @@ void ResolveLaunch(const rad_scene* scene, rad_render_desc& d) {
   }
 }
 
+// Keeps the larger arena on the scene for its next job.
+static void KeepSpareArena(rad_scene* scene, std::unique_ptr<DeviceBuffer> arena) {
+  if (!arena) return;
+  std::lock_guard<std::mutex> lk(scene->arena_mu);
+  if (!scene->spare_arena || scene->spare_arena->bytes < arena->bytes) scene->spare_arena = std::move(arena);
+}
+
 // The context's wide arena of at least `need` bytes for a job of the scene;
 // null: another job has it, or it would take more than a quarter of the free
 // memory.
@@ -466,6 +473,9 @@ rad_job* StartRender(rad_scene* scene, const rad_render_desc& desc) {
     wide.path_slots = kAloneSlots;
     const uint64_t need = Shape(scene, wide).bytes;
     if (need > Shape(scene, d).bytes) {
+      std::unique_ptr<DeviceBuffer> spare = TakeSpareArena(scene);  // large after a render with more slots asked for
+      if (spare && spare->bytes >= need) return StartJob(scene, wide, std::move(spare));
+      KeepSpareArena(scene, std::move(spare));
       if (std::unique_ptr<DeviceBuffer> arena = TakeWideArena(scene, need)) {
         try {
           rad_job* job = StartJob(scene, wide, std::move(arena));
@@ -702,9 +712,8 @@ void DestroyJob(rad_job* job) {
     std::lock_guard<std::mutex> lk(sc->wide->mu);
     sc->wide->busy = false;
     sc->wide->buffer = std::move(job->arena);
-  } else if (job->arena) {  // keep the larger arena on the scene for its next job
-    std::lock_guard<std::mutex> lk(sc->arena_mu);
-    if (!sc->spare_arena || sc->spare_arena->bytes < job->arena->bytes) sc->spare_arena = std::move(job->arena);
+  } else {
+    KeepSpareArena(sc, std::move(job->arena));
   }
   delete job;
 }

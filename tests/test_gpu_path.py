@@ -325,3 +325,20 @@ def test_one_wide_arena_for_all_scenes(hip_ctx):
     ss[1].close()
     img, _, st = ss[2].render(d[2])
     assert st.slots == 16 << 20 and np.array_equal(img, imgs[2])
+
+
+def test_large_spare_arena_serves_the_default_render(hip_ctx):
+    """A scene whose last render asked for many slots has an arena that a default render fits: it takes that, and the
+    context's wide arena stays free for another scene."""
+    bs = [scenes.many_balls(seed=i, width=512, height=512, spp=80, n_spheres=8) for i in range(2)]
+    ss = [hip.Scene.from_builder(hip_ctx, b) for b in bs]
+    base = [s.info().device_bytes for s in ss]
+    img = ss[0].render(bs[0].render_desc(spp=80, seed=3, path_slots=20 << 20))[0]
+    held = ss[0].info().device_bytes
+    jobs = [s.start(b.render_desc(spp=80, seed=3)) for s, b in zip(ss, bs)]
+    got = [j.wait() for j in jobs]
+    assert [g[2].slots for g in got] == [16 << 20, 16 << 20] and np.array_equal(got[0][0], img)
+    for j in jobs:
+        j.close()
+    assert ss[0].info().device_bytes == held
+    assert ss[1].info().device_bytes - base[1] > 4 << 30
